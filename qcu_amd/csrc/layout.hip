@@ -10,48 +10,65 @@
 
 namespace qcu {
 
-// one thread per (p, mu, site): rows 0 and 1 of the 3x3 link
-template <int P>
-__global__ void __launch_bounds__(256) k_gauge_in(const double2 *ext, Geom g, void *a, void *b) {
+// Links in every precision the lattice keeps, from one read of the field.
+// 256 consecutive links (36 KiB) are staged through LDS with whole-line loads,
+// then each thread takes rows 0 and 1 of its own link (a stride of 36 banks
+// between lanes: no conflicts for 16-byte reads) and writes them
+// component-planar.  HBM bound: 144 bytes read and 168 written per link with
+// all three precisions.
+template <int M>  // bit k: precision k
+__global__ void __launch_bounds__(256) k_gauge_in(const double2 *ext, Geom g, GaugeOut o) {
+  __shared__ double2 sh[256 * 9];
   const int vh = g.vh;
-  const long n = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (n >= 8L * vh) return;
+  const long total = 8L * vh;
+  const long n0 = (long)blockIdx.x * 256;
+  const int m = (int)(total - n0 < 256 ? total - n0 : 256) * 9;  // entries of this block
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    const int k = q * 256 + threadIdx.x;
+    if (k < m) sh[k] = ext[n0 * 9 + k];
+  }
+  __syncthreads();
+  const long n = n0 + threadIdx.x;
+  if (n >= total) return;
   const int pm = (int)(n / vh), i = (int)(n - (long)pm * vh);
   const int mu = pm >> 1, p = pm & 1;  // external order [mu][p]
-  const double2 *src = ext + n * 9;
+  const int slab = p * 4 + mu;         // internal order [p][mu]
   double2 u[6];
 #pragma unroll
-  for (int k = 0; k < 6; ++k) u[k] = src[k];
-  const int slab = p * 4 + mu;  // internal order [p][mu]
-  if (P == P64) {
-    double2 *dst = (double2 *)a + (size_t)slab * 6 * vh + i;
+  for (int k = 0; k < 6; ++k) u[k] = sh[threadIdx.x * 9 + k];
+  if (M & 1) {
+    double2 *dst = (double2 *)o.u64 + (size_t)slab * 6 * vh + i;
 #pragma unroll
     for (int k = 0; k < 6; ++k) dst[(size_t)k * vh] = u[k];
-  } else if (P == P32) {
-    float4 *dst = (float4 *)a + (size_t)slab * 3 * vh + i;
+  }
+  if (M & 2) {
+    float4 *dst = (float4 *)o.u32 + (size_t)slab * 3 * vh + i;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
       dst[(size_t)k * vh] = make_float4((float)u[2 * k].x, (float)u[2 * k].y, (float)u[2 * k + 1].x,
                                         (float)u[2 * k + 1].y);
-  } else {
+  }
+  if (M & 4) {
     unsigned w[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k)
       w[k] = (unsigned)f2h((float)u[k].x) | ((unsigned)f2h((float)u[k].y) << 16);
-    ((uint4 *)a)[(size_t)slab * vh + i] = make_uint4(w[0], w[1], w[2], w[3]);
-    ((uint2 *)b)[(size_t)slab * vh + i] = make_uint2(w[4], w[5]);
+    ((uint4 *)o.u16a)[(size_t)slab * vh + i] = make_uint4(w[0], w[1], w[2], w[3]);
+    ((uint2 *)o.u16b)[(size_t)slab * vh + i] = make_uint2(w[4], w[5]);
   }
 }
 
-int gauge_ext_to_internal(const void *ext, const Geom &g, int prec, void *a, void *b, hipStream_t s) {
+int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeOut &o, hipStream_t s) {
   const long n = 8L * g.vh;
-  const int bs = 256;
-  const int nb = (int)((n + bs - 1) / bs);
-  switch (prec) {
-    case P64: hipLaunchKernelGGL(k_gauge_in<P64>, dim3(nb), dim3(bs), 0, s, (const double2 *)ext, g, a, b); break;
-    case P32: hipLaunchKernelGGL(k_gauge_in<P32>, dim3(nb), dim3(bs), 0, s, (const double2 *)ext, g, a, b); break;
-    case P16: hipLaunchKernelGGL(k_gauge_in<P16>, dim3(nb), dim3(bs), 0, s, (const double2 *)ext, g, a, b); break;
-    default: set_error(QCU_ERR_ARG, "bad precision"); return QCU_ERR_ARG;
+  const dim3 nb((unsigned)((n + 255) / 256)), bs(256);
+  const double2 *e = (const double2 *)ext;
+  switch (mask) {
+    case 1: hipLaunchKernelGGL(k_gauge_in<1>, nb, bs, 0, s, e, g, o); break;
+    case 3: hipLaunchKernelGGL(k_gauge_in<3>, nb, bs, 0, s, e, g, o); break;
+    case 5: hipLaunchKernelGGL(k_gauge_in<5>, nb, bs, 0, s, e, g, o); break;
+    case 7: hipLaunchKernelGGL(k_gauge_in<7>, nb, bs, 0, s, e, g, o); break;
+    default: set_error(QCU_ERR_ARG, "bad precision mask"); return QCU_ERR_ARG;
   }
   QCU_HIP(hipGetLastError());
   return 0;

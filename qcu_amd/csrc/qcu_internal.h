@@ -119,7 +119,11 @@ struct BatchOp {
 // kernel launchers (implemented in the .hip files)
 // --------------------------------------------------------------------------
 // layout.hip
-int gauge_ext_to_internal(const void *ext, const Geom &g, int prec, void *a, void *b, hipStream_t s);
+struct GaugeOut {
+  void *u64, *u32, *u16a, *u16b;
+};
+// mask bit k: links of precision k are written (bit 0, FP64, always set)
+int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeOut &out, hipStream_t s);
 // 64-bit content hash of an external gauge field (scratch: gauge_hash_scratch_bytes() of device memory)
 int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, hipStream_t s);
 size_t gauge_hash_scratch_bytes();
@@ -138,10 +142,17 @@ int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, in
         SpinorPtr y, SysState *st, double *partials, const LaunchCfg &cfg, hipStream_t s, bool use_clover = true);
 
 // clover.hip
-// packed A (clov, optional) and A^-1 (cinv) of one parity from FP64 internal links
-int clover_build(const LinkPtr &U64, const Geom &g, double coeff, int parity, void *clov, void *cinv,
-                 int *bad_dev, hipStream_t s);
-int clover_convert(const void *c64, const Geom &g, int prec, void *dst, float *norm, hipStream_t s);
+// packed A and A^-1 of one parity; FP32 and FP16 copies of A^-1 where asked for
+// (both parities alike; the FP16 one needs its per-site scales)
+struct CloverOut {
+  void *clov, *cinv64;
+  void *cinv32;    // or null
+  void *cinv16;    // or null
+  float *cinv16n;
+};
+// both parities from FP64 internal links; *bad_dev counts singular blocks
+int clover_build(const LinkPtr &U64, const Geom &g, double coeff, const CloverOut (&out)[2], int *bad_dev,
+                 hipStream_t s);
 
 // blas.hip (every reduction is per system and finishes with finish())
 int batch_blocks(const BatchOp &op, int bsz);

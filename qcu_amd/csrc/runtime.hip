@@ -140,33 +140,32 @@ int Lattice::load_gauge(const void *ext, int mask) {
   prec_mask = 0;
   solver.reset();  // its batch table and graphs point at the previous state
   QCU_TRY(U64.alloc(8 * vh * 6 * 16));
-  QCU_TRY(gauge_ext_to_internal(ext, g, P64, U64.p, nullptr, stream));
-  if (mask & 2) {
-    QCU_TRY(U32.alloc(8 * vh * 6 * 8));
-    QCU_TRY(gauge_ext_to_internal(ext, g, P32, U32.p, nullptr, stream));
-  }
+  if (mask & 2) QCU_TRY(U32.alloc(8 * vh * 6 * 8));
   if (mask & 4) {
     QCU_TRY(U16a.alloc(8 * vh * 16));
     QCU_TRY(U16b.alloc(8 * vh * 8));
-    QCU_TRY(gauge_ext_to_internal(ext, g, P16, U16a.p, U16b.p, stream));
   }
+  QCU_TRY(gauge_ext_to_internal(ext, g, mask, GaugeOut{U64.p, U32.p, U16a.p, U16b.p}, stream));
   if (has_clover()) {
     int *bad = (int *)flag.p;
     QCU_HIP(hipMemsetAsync(bad, 0, sizeof(int), stream));
+    CloverOut out[2];
     for (int p = 0; p < 2; ++p) {
       QCU_TRY(clov64[p].alloc(vh * 72 * 8));
       QCU_TRY(cinv64[p].alloc(vh * 72 * 8));
-      QCU_TRY(clover_build(links(P64), g, kappa * csw, p, clov64[p].p, cinv64[p].p, bad, stream));
+      out[p] = CloverOut{clov64[p].p, cinv64[p].p, nullptr, nullptr, nullptr};
       if (mask & 2) {
         QCU_TRY(cinv32[p].alloc(vh * 72 * 4));
-        QCU_TRY(clover_convert(cinv64[p].p, g, P32, cinv32[p].p, nullptr, stream));
+        out[p].cinv32 = cinv32[p].p;
       }
       if (mask & 4) {
         QCU_TRY(cinv16[p].alloc(vh * 72 * 2));
         QCU_TRY(cinv16n[p].alloc(vh * 4));
-        QCU_TRY(clover_convert(cinv64[p].p, g, P16, cinv16[p].p, (float *)cinv16n[p].p, stream));
+        out[p].cinv16 = cinv16[p].p;
+        out[p].cinv16n = (float *)cinv16n[p].p;
       }
     }
+    QCU_TRY(clover_build(links(P64), g, kappa * csw, out, bad, stream));
     int hbad = 0;
     QCU_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, stream));
     QCU_HIP(hipStreamSynchronize(stream));
