@@ -81,11 +81,46 @@ int check_grid(const QcuParam *grid) {
   return 0;
 }
 
+// The FP64 operators read the caller's input and write its output directly; an
+// input that overlaps the output is copied first.
+bool overlap(const void *out, const void *in, size_t bytes) {
+  return (const char *)out < (const char *)in + bytes && (const char *)in < (const char *)out + bytes;
+}
+
+// out = [A_p^-1] D in (mat: out = M in) in FP64 on the caller's fields of `bytes` bytes
+int direct_op(Lattice &lat, void *out, const void *in, size_t bytes, int parity, int mat, bool clover, void *copy) {
+  const void *src = in;
+  if (overlap(out, in, bytes)) {
+    if (!copy) {
+      QCU_TRY(lat.stage_in.alloc(bytes));
+      copy = lat.stage_in.p;
+    }
+    QCU_HIP(hipMemcpyAsync(copy, in, bytes, hipMemcpyDeviceToDevice, lat.stream));
+    src = copy;
+  }
+  QCU_TRY(hop_ext(lat.self, out, src, parity, mat, clover, lat.stream));
+  QCU_HIP(hipStreamSynchronize(lat.stream));
+  return 0;
+}
+
+// the same hop in a lower precision, through half spinors a and b of that precision
+int staged_op(Lattice &lat, void *out, const void *in, int parity, int prec, bool clover, const SpinorPtr &a,
+              const SpinorPtr &b) {
+  QCU_TRY(spinor_ext_to_batch(in, lat.self, 0, 0, a, prec, lat.stream));
+  SpinorPtr none{};
+  QCU_TRY(hop(lat.self, prec, b, a, parity, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr,
+              tuned_cfg(lat.self, prec), lat.stream, clover));
+  QCU_TRY(spinor_batch_to_ext(b, lat.self, 0, 0, out, prec, lat.stream));
+  QCU_HIP(hipStreamSynchronize(lat.stream));
+  return 0;
+}
+
+size_t half_bytes(const Lattice &lat) { return (size_t)lat.g.vh * 12 * 16; }
+
 // resident lattices of the legacy entry points, one per (device, kind):
 // kind 0 Wilson with kappa 0.125, kind 1 clover with kappa*csw = 1
 struct Legacy {
   Lattice lat;
-  Spinor a, b;
   DevBuf hash_buf;               // scratch of the gauge hash
   const void *gauge = nullptr;   // caller's gauge of the resident links (null: none)
   unsigned long long hash = 0;   // its content hash
@@ -119,8 +154,6 @@ Legacy *legacy_ctx(const QcuParam *param, int kind, int *rc) {
   }
   std::unique_ptr<Legacy> l(new Legacy());
   *rc = kind == 0 ? l->lat.init(param->lattice_size, 0.125, 0.0, 1) : l->lat.init(param->lattice_size, 1.0, 1.0, 1);
-  if (!*rc) *rc = l->a.create(P64, l->lat.g.vh);
-  if (!*rc) *rc = l->b.create(P64, l->lat.g.vh);
   if (*rc) return nullptr;
   Legacy *raw = l.get();
   g_legacy[key] = std::move(l);
@@ -139,13 +172,7 @@ int legacy_dslash(void *out, void *in, void *gauge, QcuParam *param, int parity,
   if (!L) return rc;
   Lattice &lat = L->lat;
   QCU_TRY(legacy_load_gauge(*L, gauge));
-  QCU_TRY(spinor_ext_to_batch(in, lat.self, 0, 0, L->a.ptr(), P64, lat.stream));
-  SpinorPtr none{};
-  QCU_TRY(hop(lat.self, P64, L->b.ptr(), L->a.ptr(), parity, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr,
-              tuned_cfg(lat.self, P64), lat.stream, clover != 0));
-  QCU_TRY(spinor_batch_to_ext(L->b.ptr(), lat.self, 0, 0, out, P64, lat.stream));
-  QCU_HIP(hipStreamSynchronize(lat.stream));
-  return 0;
+  return direct_op(lat, out, in, half_bytes(lat), parity, 0, clover != 0, nullptr);
 }
 
 int lattice_solver(Lattice &lat, Solver **S) {
@@ -287,16 +314,9 @@ int qcuDslash(QcuLatticeHandle h, void *out, const void *in, int parity, int clo
   QCU_CHECK(!clover || lat.has_clover(), QCU_ERR_STATE, "lattice has no clover term (csw = 0)");
   QCU_TRY(check_dev_ptr(out, "out"));
   QCU_TRY(check_dev_ptr(in, "in"));
-  Spinor a, b;
-  QCU_TRY(a.create(prec, lat.g.vh));
-  QCU_TRY(b.create(prec, lat.g.vh));
-  QCU_TRY(spinor_ext_to_batch(in, lat.self, 0, 0, a.ptr(), prec, lat.stream));
-  SpinorPtr none{};
-  QCU_TRY(hop(lat.self, prec, b.ptr(), a.ptr(), parity, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr,
-              tuned_cfg(lat.self, prec), lat.stream, clover != 0));
-  QCU_TRY(spinor_batch_to_ext(b.ptr(), lat.self, 0, 0, out, prec, lat.stream));
-  QCU_HIP(hipStreamSynchronize(lat.stream));
-  return 0;
+  if (prec == P64) return direct_op(lat, out, in, half_bytes(lat), parity, 0, clover != 0, nullptr);
+  for (Spinor &v : lat.stage) QCU_TRY(v.create(prec, lat.g.vh));
+  return staged_op(lat, out, in, parity, prec, clover != 0, lat.stage[0].ptr(), lat.stage[1].ptr());
 }
 
 // ---- the hop without allocation ----------------------------------------------
@@ -355,6 +375,7 @@ int qcuDslashNoAlloc(QcuLatticeHandle h, void *out, const void *in, int parity, 
   QCU_CHECK(dev == lat.device, QCU_ERR_STATE, "the current device is not the lattice's");
   void *base = nullptr;
   QCU_TRY(noalloc_scratch(dev, &base));
+  if (prec == P64) return direct_op(lat, out, in, half_bytes(lat), parity, 0, clover != 0, base);
   SpinorPtr a, b;
   const size_t data = round256(spinor_bytes(prec, lat.g.vh));
   a.p = base;
@@ -363,13 +384,7 @@ int qcuDslashNoAlloc(QcuLatticeHandle h, void *out, const void *in, int parity, 
   b.p = (char *)base + half;
   b.norm = prec == P16 ? (float *)((char *)base + half + data) : nullptr;
   b.stride = lat.g.vh;
-  QCU_TRY(spinor_ext_to_batch(in, lat.self, 0, 0, a, prec, lat.stream));
-  SpinorPtr none{};
-  QCU_TRY(hop(lat.self, prec, b, a, parity, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr,
-              tuned_cfg(lat.self, prec), lat.stream, clover != 0));
-  QCU_TRY(spinor_batch_to_ext(b, lat.self, 0, 0, out, prec, lat.stream));
-  QCU_HIP(hipStreamSynchronize(lat.stream));
-  return 0;
+  return staged_op(lat, out, in, parity, prec, clover != 0, a, b);
 }
 
 int qcuMatFull(QcuLatticeHandle h, void *out, const void *in) {
@@ -379,25 +394,7 @@ int qcuMatFull(QcuLatticeHandle h, void *out, const void *in) {
   QCU_CHECK(lat.gauge_loaded, QCU_ERR_STATE, "gauge field not loaded");
   QCU_TRY(check_dev_ptr(out, "out"));
   QCU_TRY(check_dev_ptr(in, "in"));
-  const BatchOp &op = lat.self;
-  const int vh = lat.g.vh;
-  const size_t half = (size_t)vh * 12 * 16;
-  Spinor x[2], t, o;
-  for (int p = 0; p < 2; ++p) QCU_TRY(x[p].create(P64, vh));
-  QCU_TRY(t.create(P64, vh));
-  QCU_TRY(o.create(P64, vh));
-  for (int p = 0; p < 2; ++p)
-    QCU_TRY(spinor_ext_to_batch((const char *)in + p * half, op, 0, 0, x[p].ptr(), P64, lat.stream));
-  SpinorPtr none{};
-  for (int p = 0; p < 2; ++p) {
-    QCU_TRY(hop(op, P64, t.ptr(), x[1 - p].ptr(), p, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr,
-                tuned_cfg(op, P64), lat.stream, false));
-    QCU_TRY(cl_axpy(op, o.ptr(), x[p].ptr(), 0.0, false, none, 2, p, lat.stream));
-    QCU_TRY(axpby(op, -lat.kappa, t.ptr(), P64, 1.0, o.ptr(), P64, lat.stream));
-    QCU_TRY(spinor_batch_to_ext(o.ptr(), op, 0, 0, (char *)out + p * half, P64, lat.stream));
-  }
-  QCU_HIP(hipStreamSynchronize(lat.stream));
-  return 0;
+  return direct_op(lat, out, in, 2 * half_bytes(lat), 0, 1, lat.has_clover(), nullptr);
 }
 
 int qcuTrueResidual(QcuLatticeHandle h, const void *x, const void *b, double *res) {
@@ -447,6 +444,7 @@ int qcuBenchHop(QcuLatticeHandle h, int prec, int clover, int xpay, int iters, i
   LaunchCfg cfg = tuned_cfg(lat.self, prec);
   if (block > 0) cfg.block = block;
   if (remap >= 0) cfg.remap = remap;
+  if (block > 0 || remap >= 0) cfg.automatic = false;
   return bench_hop(lat.self, lat.stream, prec, clover, xpay, iters, cfg, ms);
 }
 

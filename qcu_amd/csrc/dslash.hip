@@ -18,6 +18,7 @@
 #include "qcu_batch.h"
 #include "qcu_internal.h"
 #include "qcu_reduce.h"
+#include "qcu_solver.h"
 #include "qcu_state.h"
 
 namespace qcu {
@@ -89,17 +90,52 @@ QCU_D void transport(const cplx<T> (&u)[9], const cplx<T> (&h)[3], cplx<T> (&a)[
   }
 }
 
-template <int P, int MU, int FWD>
-QCU_D void hop_dir(cplx<typename real_of<P>::type> (&d)[12], const LinkPtr &U, int pm, int li,
-                   const SpinorPtr &in, int si, typename real_of<P>::type ph) {
+// Where the spinors of a hop live.  Reading the caller's fields directly (192
+// contiguous bytes per lane, whose lines the twelve loads of a direction share)
+// costs the hop 3 % more than the internal layout; staging them through it cost
+// two more passes (70 + 100 us beside a 430 us clover hop at 32^3x64) and, as the
+// staging was allocated per call, 10 ms of hipMalloc and hipFree.
+enum HopIO {
+  IO_INT = 0,  // internal layout (batch vectors)
+  IO_EXT = 1,  // the caller's FP64 fields [Vh][4][3], one lattice and one right-hand side
+};
+
+template <int P, int IO>
+QCU_D void load_spinor(const SpinorPtr &f, int i, cplx<typename real_of<P>::type> (&v)[12]) {
+  if (IO == IO_EXT) {
+    const double2 *src = (const double2 *)f.p + (size_t)i * 12;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+      const double2 a = src[k];
+      v[k] = mk<typename real_of<P>::type>(a.x, a.y);
+    }
+  } else {
+    SpinorIO<P>::load(f, i, v);
+  }
+}
+
+template <int P, int IO>
+QCU_D void store_spinor(const SpinorPtr &f, int i, const cplx<typename real_of<P>::type> (&v)[12]) {
+  if (IO == IO_EXT) {
+    double2 *dst = (double2 *)f.p + (size_t)i * 12;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) dst[k] = make_double2(v[k].re, v[k].im);
+  } else {
+    SpinorIO<P>::store(f, i, v);
+  }
+}
+
+// the transported half spinor (a0, a1) of one direction
+template <int P, int IO, int MU, int FWD>
+QCU_D void hop_half(cplx<typename real_of<P>::type> (&a0)[3], cplx<typename real_of<P>::type> (&a1)[3],
+                    const LinkPtr &U, int pm, int li, const SpinorPtr &in, int si, typename real_of<P>::type ph) {
   typedef typename real_of<P>::type T;
   cplx<T> s[12];
-  SpinorIO<P>::load(in, si, s);
+  load_spinor<P, IO>(in, si, s);
   cplx<T> h0[3], h1[3];
   project<MU, FWD>(s, h0, h1);
   cplx<T> u[9];
   LinkIO<P>::load(U, pm, li, u);
-  cplx<T> a0[3], a1[3];
   transport<FWD>(u, h0, a0);
   transport<FWD>(u, h1, a1);
   if (MU == 3) {
@@ -109,7 +145,33 @@ QCU_D void hop_dir(cplx<typename real_of<P>::type> (&d)[12], const LinkPtr &U, i
       a1[c] = ph * a1[c];
     }
   }
+}
+
+template <int P, int IO, int MU, int FWD>
+QCU_D void hop_dir(cplx<typename real_of<P>::type> (&d)[12], const LinkPtr &U, int pm, int li,
+                   const SpinorPtr &in, int si, typename real_of<P>::type ph) {
+  cplx<typename real_of<P>::type> a0[3], a1[3];
+  hop_half<P, IO, MU, FWD>(a0, a1, U, pm, li, in, si, ph);
   accumulate<MU, FWD>(d, a0, a1);
+}
+
+// index of the neighbour of site i (half index) in direction MU, forward or
+// backward, and the sign of a hop across the time boundary.  Branch-free; a
+// site with odd full x has its x-1 neighbour at the same half index.
+template <int MU, int FWD>
+QCU_D int neighbour(const Geom &g, const Site &s, int i, int &sign) {
+  const int sy = g.lxh, sz = g.lxh * g.ly, st = sz * g.lz;
+  sign = 1;
+  if (MU == 0) {
+    if (FWD) return i + s.xodd - s.xodd * (int)(s.xh == g.lxh - 1) * g.lxh;
+    const int xe = 1 - s.xodd;
+    return i - xe + xe * (int)(s.xh == 0) * g.lxh;
+  }
+  if (MU == 1) return FWD ? i + sy - (int)(s.y == g.ly - 1) * g.ly * sy : i - sy + (int)(s.y == 0) * g.ly * sy;
+  if (MU == 2) return FWD ? i + sz - (int)(s.z == g.lz - 1) * g.lz * sz : i - sz + (int)(s.z == 0) * g.lz * sz;
+  const int edge = FWD ? (int)(s.t == g.lt - 1) : (int)(s.t == 0);
+  sign = 1 - 2 * ((int)(g.tbc < 0) & edge);
+  return FWD ? i + st - edge * g.lt * st : i - st + edge * g.lt * st;
 }
 
 struct HopKArgs {
@@ -131,15 +193,35 @@ struct HopKArgs {
     if ((G) == 1 || ((G) == 2 && ((k) & 1))) __builtin_amdgcn_sched_barrier(0);    \
   } while (0)
 
-template <int P, int CLOVER, int EPI, int RED, int G>
+// parity and block of a launch: with EPI_MAT one launch covers both parities,
+// in alternate blocks
+template <int EPI>
+QCU_D int hop_block(const HopKArgs &a, int &parity) {
+  const int b = remap_block(blockIdx.x, gridDim.x, a.remap);
+  parity = EPI == EPI_MAT ? (b & 1) : a.parity;
+  return EPI == EPI_MAT ? b >> 1 : b;
+}
+
+// the fields of a launch for one segment (and parity): EPI_MAT works on full
+// external fields
+template <int P, int IO, int EPI>
+QCU_D SpinorPtr hop_field(const SpinorPtr &f, const SegDesc &sd, int parity) {
+  if (IO == IO_INT) return seg_view(f, P, sd.voff, sd.nthr);
+  SpinorPtr v = f;
+  if (EPI == EPI_MAT) v.p = (char *)f.p + (size_t)parity * sd.g.vh * 192;
+  return v;
+}
+
+template <int P, int IO, int CLOVER, int EPI, int RED, int G>
 __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
   typedef typename real_of<P>::type T;
-  const int blk = remap_block(blockIdx.x, gridDim.x, a.remap);
+  int p;
+  const int blk = hop_block<EPI>(a, p);
   const BlockSeg bs = find_seg(a.segs, a.nseg, blk, blockDim.x);
   if (bs.seg < 0) return;  // uniform: a block past the last segment
   const SegDesc &sd = a.segs[bs.seg];
   const Geom g = sd.g;
-  const int nrhs = sd.nrhs;
+  const int nrhs = IO == IO_EXT ? 1 : sd.nrhs;
   const int t = bs.t0 + threadIdx.x;
   const int site = t / nrhs;
   const int rhs = t - site * nrhs;
@@ -149,54 +231,56 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
   cplx<T> d[12];
   double red[3] = {0, 0, 0};
   if (active) {
-    const SpinorPtr in = seg_view(a.in, P, sd.voff, sd.nthr);
+    const int q = 1 - p;
+    const SpinorPtr in = hop_field<P, IO, EPI>(a.in, sd, q);
     const LinkPtr U = sd.U[P];
     const int i = site;
-    const Site s = decode(g, i, a.parity);
-    const int p = a.parity, q = 1 - p;
-    const int sy = g.lxh, sz = g.lxh * g.ly, st_ = sz * g.lz;
+    const Site s = decode(g, i, p);
 #pragma unroll
     for (int k = 0; k < 12; ++k) d[k] = mk<T>(0, 0);
-    {
-      // branch-free index arithmetic keeps the body one basic block, so the
-      // scheduling fences below bound the live registers; a site with odd
-      // full x has its x-1 neighbour at the same half index
-      const int xe = 1 - s.xodd;
-      const int jb = i - xe + xe * (int)(s.xh == 0) * g.lxh;
-      const int jf = i + s.xodd - s.xodd * (int)(s.xh == g.lxh - 1) * g.lxh;
-      hop_dir<P, 0, 0>(d, U, q * 4 + 0, jb, in, jb * nrhs + rhs, (T)1);
-      QCU_GROUP_FENCE(G, 0);
-      hop_dir<P, 0, 1>(d, U, p * 4 + 0, i, in, jf * nrhs + rhs, (T)1);
-      QCU_GROUP_FENCE(G, 1);
-    }
-    {
-      const int jb = i - sy + (int)(s.y == 0) * g.ly * sy;
-      const int jf = i + sy - (int)(s.y == g.ly - 1) * g.ly * sy;
-      hop_dir<P, 1, 0>(d, U, q * 4 + 1, jb, in, jb * nrhs + rhs, (T)1);
-      QCU_GROUP_FENCE(G, 2);
-      hop_dir<P, 1, 1>(d, U, p * 4 + 1, i, in, jf * nrhs + rhs, (T)1);
-      QCU_GROUP_FENCE(G, 3);
-    }
-    {
-      const int jb = i - sz + (int)(s.z == 0) * g.lz * sz;
-      const int jf = i + sz - (int)(s.z == g.lz - 1) * g.lz * sz;
-      hop_dir<P, 2, 0>(d, U, q * 4 + 2, jb, in, jb * nrhs + rhs, (T)1);
-      QCU_GROUP_FENCE(G, 4);
-      hop_dir<P, 2, 1>(d, U, p * 4 + 2, i, in, jf * nrhs + rhs, (T)1);
-      QCU_GROUP_FENCE(G, 5);
-    }
-    {
-      const int jb = i - st_ + (int)(s.t == 0) * g.lt * st_;
-      const int jf = i + st_ - (int)(s.t == g.lt - 1) * g.lt * st_;
-      const int flip = (g.tbc < 0);
-      const T phb = (T)(1 - 2 * (flip & (int)(s.t == 0)));
-      const T phf = (T)(1 - 2 * (flip & (int)(s.t == g.lt - 1)));
-      hop_dir<P, 3, 0>(d, U, q * 4 + 3, jb, in, jb * nrhs + rhs, phb);
-      QCU_GROUP_FENCE(G, 6);
-      hop_dir<P, 3, 1>(d, U, p * 4 + 3, i, in, jf * nrhs + rhs, phf);
-      QCU_GROUP_FENCE(G, 7);
-    }
-    if (CLOVER) {
+    int j, sg;
+    // branch-free index arithmetic keeps the body one basic block, so the
+    // scheduling fences below bound the live registers
+    j = neighbour<0, 0>(g, s, i, sg);
+    hop_dir<P, IO, 0, 0>(d, U, q * 4 + 0, j, in, j * nrhs + rhs, (T)1);
+    QCU_GROUP_FENCE(G, 0);
+    j = neighbour<0, 1>(g, s, i, sg);
+    hop_dir<P, IO, 0, 1>(d, U, p * 4 + 0, i, in, j * nrhs + rhs, (T)1);
+    QCU_GROUP_FENCE(G, 1);
+    j = neighbour<1, 0>(g, s, i, sg);
+    hop_dir<P, IO, 1, 0>(d, U, q * 4 + 1, j, in, j * nrhs + rhs, (T)1);
+    QCU_GROUP_FENCE(G, 2);
+    j = neighbour<1, 1>(g, s, i, sg);
+    hop_dir<P, IO, 1, 1>(d, U, p * 4 + 1, i, in, j * nrhs + rhs, (T)1);
+    QCU_GROUP_FENCE(G, 3);
+    j = neighbour<2, 0>(g, s, i, sg);
+    hop_dir<P, IO, 2, 0>(d, U, q * 4 + 2, j, in, j * nrhs + rhs, (T)1);
+    QCU_GROUP_FENCE(G, 4);
+    j = neighbour<2, 1>(g, s, i, sg);
+    hop_dir<P, IO, 2, 1>(d, U, p * 4 + 2, i, in, j * nrhs + rhs, (T)1);
+    QCU_GROUP_FENCE(G, 5);
+    j = neighbour<3, 0>(g, s, i, sg);
+    hop_dir<P, IO, 3, 0>(d, U, q * 4 + 3, j, in, j * nrhs + rhs, (T)sg);
+    QCU_GROUP_FENCE(G, 6);
+    j = neighbour<3, 1>(g, s, i, sg);
+    hop_dir<P, IO, 3, 1>(d, U, p * 4 + 3, i, in, j * nrhs + rhs, (T)sg);
+    QCU_GROUP_FENCE(G, 7);
+    if (EPI == EPI_MAT) {
+      // A x - kappa d
+      cplx<T> x[12];
+      load_spinor<P, IO>(hop_field<P, IO, EPI>(a.in, sd, p), t, x);
+      if (CLOVER) {
+        T c[36];
+        clover_load_block(sd.A[p], i, 0, c);
+        clover_apply_block(c, x, 0);
+        QCU_GROUP_FENCE(G, 1);
+        clover_load_block(sd.A[p], i, 1, c);
+        clover_apply_block(c, x, 1);
+      }
+      const T kap = (T)sd.kappa;
+#pragma unroll
+      for (int k = 0; k < 12; ++k) d[k] = nmad(x[k], kap, d[k]);
+    } else if (CLOVER) {
       const CloverPtr C = sd.Cinv[P][p];
       if (P == P16) {
         T c[72];
@@ -217,7 +301,7 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
       SpinorIO<P>::load(seg_view(a.x, P, sd.voff, sd.nthr), t, x);
       const T k2 = (T)(sd.kappa * sd.kappa);
 #pragma unroll
-      for (int k = 0; k < 12; ++k) d[k] = x[k] - k2 * d[k];
+      for (int k = 0; k < 12; ++k) d[k] = nmad(x[k], k2, d[k]);
       if (RED == RED_OUT_X) {
         // <out, x> and |out|^2
 #pragma unroll
@@ -237,7 +321,7 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
         red[1] += (double)y[k].re * (double)d[k].im - (double)y[k].im * (double)d[k].re;
       }
     }
-    SpinorIO<P>::store(seg_view(a.out, P, sd.voff, sd.nthr), t, d);
+    store_spinor<P, IO>(hop_field<P, IO, EPI>(a.out, sd, p), t, d);
   }
   if (RED == RED_DOT_Y_OUT) {
     double v[2] = {red[0], red[1]};
@@ -247,45 +331,395 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
   }
 }
 
+// ---- eight waves per 64 sites ----------------------------------------------
+// The same operator with one wave per direction: a lattice too small to fill the
+// chip with one thread per site (8^4: 32 waves for 256 CUs) is bound by the
+// latency of the eight hops one after the other.  Each of the 8 waves of a block
+// transports its direction's half spinor for the block's 64 sites into LDS; then
+// wave w < 6 forms components 2w and 2w + 1 of the result (every sum in the
+// order of k_hop, so the results are the same bit for bit), applies rows of the
+// clover block and the epilogue, and stores its pair of components.
+constexpr int kSplitSites = 64;
+
+// components 2w, 2w + 1 of a spinor
+template <int P, int IO>
+QCU_D void load_pair(const SpinorPtr &f, int i, int w, cplx<typename real_of<P>::type> (&v)[2]) {
+  typedef typename real_of<P>::type T;
+  if (P == P64) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int k = 2 * w + q;
+      const double2 a = IO == IO_EXT ? ((const double2 *)f.p)[(size_t)i * 12 + k]
+                                     : ld_at<double2>(f.p, (size_t)k * f.stride * 16, (unsigned)i * 16u);
+      v[q] = mk<T>((T)a.x, (T)a.y);
+    }
+  } else if (P == P32) {
+    const float4 a = ld_at<float4>(f.p, (size_t)w * f.stride * 16, (unsigned)i * 16u);
+    v[0] = mk<T>(a.x, a.y);
+    v[1] = mk<T>(a.z, a.w);
+  } else {
+    const float nrm = ld_at<float>(f.norm, 0, (unsigned)i * 4u);
+    const uint2 a = ld_at<uint2>((char *)f.p + 8 * (w & 1), (size_t)(w >> 1) * f.stride * 16, (unsigned)i * 16u);
+    v[0] = mk<T>(nrm * h2f((unsigned short)(a.x & 0xffffu)), nrm * h2f((unsigned short)(a.x >> 16)));
+    v[1] = mk<T>(nrm * h2f((unsigned short)(a.y & 0xffffu)), nrm * h2f((unsigned short)(a.y >> 16)));
+  }
+}
+
+// m: the largest component of the whole spinor (FP16 only)
+template <int P, int IO>
+QCU_D void store_pair(const SpinorPtr &f, int i, int w, const cplx<typename real_of<P>::type> (&v)[2], float m) {
+  if (P == P64) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const int k = 2 * w + q;
+      const double2 a = make_double2(v[q].re, v[q].im);
+      if (IO == IO_EXT)
+        ((double2 *)f.p)[(size_t)i * 12 + k] = a;
+      else
+        st_at<double2>(f.p, (size_t)k * f.stride * 16, (unsigned)i * 16u, a);
+    }
+  } else if (P == P32) {
+    st_at<float4>(f.p, (size_t)w * f.stride * 16, (unsigned)i * 16u,
+                  make_float4(v[0].re, v[0].im, v[1].re, v[1].im));
+  } else {
+    const float inv = m > 0.f ? 1.0f / m : 0.f;
+    unsigned h[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) h[q] = (unsigned)f2h(v[q].re * inv) | ((unsigned)f2h(v[q].im * inv) << 16);
+    st_at<uint2>((char *)f.p + 8 * (w & 1), (size_t)(w >> 1) * f.stride * 16, (unsigned)i * 16u,
+                 make_uint2(h[0], h[1]));
+    if (w == 0) st_at<float>(f.norm, 0, (unsigned)i * 4u, m);
+  }
+}
+
+// reals 2q, 2q + 1 of chiral block b of a packed clover field, as stored
+template <int P>
+struct CloverWord;
+template <>
+struct CloverWord<P64> {
+  typedef double2 raw;
+  static QCU_D raw load(const CloverPtr &C, unsigned off, int n) {
+    return ld_at<double2>(C.p, (size_t)n * C.vh * 16, off);
+  }
+  static QCU_D cplx<double> value(raw a, float) { return mk(a.x, a.y); }
+};
+template <>
+struct CloverWord<P32> {
+  typedef float2 raw;
+  static QCU_D raw load(const CloverPtr &C, unsigned off, int n) {
+    return ld_at<float2>((char *)C.p + 8 * (n & 1), (size_t)(n >> 1) * C.vh * 16, off);
+  }
+  static QCU_D cplx<float> value(raw a, float) { return mk(a.x, a.y); }
+};
+template <>
+struct CloverWord<P16> {
+  typedef unsigned raw;
+  static QCU_D raw load(const CloverPtr &C, unsigned off, int n) {
+    return ld_at<unsigned>((char *)C.p + 4 * (n & 3), (size_t)(n >> 2) * C.vh * 16, off);
+  }
+  static QCU_D cplx<float> value(raw a, float nrm) {
+    return mk(nrm * h2f((unsigned short)(a & 0xffffu)), nrm * h2f((unsigned short)(a >> 16)));
+  }
+};
+
+// rows 2j, 2j + 1 of a chiral block: the word of both diagonals and the 9
+// off-diagonal entries (their common one once), loaded ahead of their use
+template <int P>
+struct CloverRows {
+  typedef typename real_of<P>::type T;
+  typename CloverWord<P>::raw dg, e[2][5];
+  float nrm;
+
+  // entry of column c in row 2j + q: its word
+  static QCU_D int word(int b, int j, int q, int k) {
+    const int r = 2 * j + q;
+    const int c = k < r ? k : k + 1;  // k counts the 5 columns other than r
+    const int hi = c < r ? r : c, lo = c < r ? c : r;
+    return 18 * b + 3 + hi * (hi - 1) / 2 + lo;
+  }
+  QCU_D void load(const CloverPtr &C, int i, int b, int j) {
+    const unsigned off = (unsigned)i * 16u;
+    nrm = P == P16 ? ld_at<float>(C.norm, 0, (unsigned)i * 4u) : 1.f;
+    dg = CloverWord<P>::load(C, off, 18 * b + j);
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+#pragma unroll
+      for (int k = 0; k < 5; ++k) e[q][k] = CloverWord<P>::load(C, off, word(b, j, q, k));
+  }
+  // row 2j + q times the block's six components x (in LDS, one lane per site),
+  // in the order of clover_apply_block
+  QCU_D cplx<T> row(int j, int q, const cplx<T> (*x)[kSplitSites], int lane) const {
+    const int r = 2 * j + q;
+    const cplx<T> d = CloverWord<P>::value(dg, nrm);
+    const T diag = q ? d.im : d.re;
+    const cplx<T> v = x[r][lane];
+    cplx<T> acc = scale_(diag, v);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const cplx<T> c = CloverWord<P>::value(e[q][k], nrm);
+      if (k < r)
+        cmad(acc, c, x[k][lane]);
+      else
+        cmadj(acc, c, x[k + 1][lane]);
+    }
+    return acc;
+  }
+};
+
+// component k of the sum over the eight directions' half spinors
+template <class T>
+QCU_D cplx<T> hop_sum(const cplx<T> (*half)[6][kSplitSites], int k, int lane) {
+  cplx<T> acc = mk<T>(0, 0);
+  if (k < 6) {
+#pragma unroll
+    for (int d = 0; d < 8; ++d) acc = acc + half[d][k][lane];
+    return acc;
+  }
+  // the lower spins take the upper ones' colour c with the factors of accumulate()
+  const bool s3 = k >= 9;
+  const int c = s3 ? k - 9 : k - 6;
+  const int k01 = (s3 ? 0 : 3) + c, k23 = (s3 ? 3 : 0) + c;
+  acc = acc + mul_mi(half[0][k01][lane]);
+  acc = acc + mul_i(half[1][k01][lane]);
+  const cplx<T> b1 = half[2][k01][lane], f1 = half[3][k01][lane];
+  acc = s3 ? acc - b1 : acc + b1;
+  acc = s3 ? acc + f1 : acc - f1;
+  const cplx<T> b2 = half[4][k23][lane], f2 = half[5][k23][lane];
+  acc = s3 ? acc + mul_i(b2) : acc + mul_mi(b2);
+  acc = s3 ? acc + mul_mi(f2) : acc + mul_i(f2);
+  acc = acc + half[6][k23][lane];
+  acc = acc - half[7][k23][lane];
+  return acc;
+}
+
+template <int P, int IO, int CLOVER, int EPI, int RED>
+__global__ void __launch_bounds__(8 * kSplitSites) k_hop_split(HopKArgs a) {
+  typedef typename real_of<P>::type T;
+  __shared__ cplx<T> half[8][6][kSplitSites];
+  int p;
+  const int blk = hop_block<EPI>(a, p);
+  const BlockSeg bs = find_seg(a.segs, a.nseg, blk, kSplitSites);
+  if (bs.seg < 0) return;  // uniform
+  const SegDesc &sd = a.segs[bs.seg];
+  const Geom g = sd.g;
+  const int nrhs = IO == IO_EXT ? 1 : sd.nrhs;
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int t = bs.t0 + lane;
+  const int i = t / nrhs, rhs = t - i * nrhs;
+  bool active = t < sd.nthr;
+  if (a.st && active && a.st[sd.sys0 + rhs].done) active = false;
+  const bool mine = active && w < 6;  // this wave's pair of components
+  const int cb = w / 3, cj = w - 3 * cb;  // its chiral block and rows 2 cj, 2 cj + 1 of it
+  CloverRows<P> cr;
+  if (active) {
+    const int q = 1 - p;
+    const SpinorPtr in = hop_field<P, IO, EPI>(a.in, sd, q);
+    const LinkPtr U = sd.U[P];
+    const Site s = decode(g, i, p);
+    cplx<T> a0[3], a1[3];
+    int j, sg;
+#define QCU_SPLIT_DIR(MU)                                                                 \
+  case 2 * MU:                                                                            \
+    j = neighbour<MU, 0>(g, s, i, sg);                                                    \
+    hop_half<P, IO, MU, 0>(a0, a1, U, q * 4 + MU, j, in, j * nrhs + rhs, (T)sg);          \
+    break;                                                                                \
+  case 2 * MU + 1:                                                                        \
+    j = neighbour<MU, 1>(g, s, i, sg);                                                    \
+    hop_half<P, IO, MU, 1>(a0, a1, U, p * 4 + MU, i, in, j * nrhs + rhs, (T)sg);          \
+    break;
+    switch (w) {
+      QCU_SPLIT_DIR(0)
+      QCU_SPLIT_DIR(1)
+      QCU_SPLIT_DIR(2)
+      QCU_SPLIT_DIR(3)
+    }
+#undef QCU_SPLIT_DIR
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      half[w][c][lane] = a0[c];
+      half[w][3 + c][lane] = a1[c];
+    }
+  }
+  // in flight over the barriers and the sum
+  if (CLOVER && mine) cr.load(EPI == EPI_MAT ? sd.A[p] : sd.Cinv[P][p], i, cb, cj);
+  __syncthreads();
+  cplx<T> d[2] = {mk<T>(0, 0), mk<T>(0, 0)}, x[2] = {mk<T>(0, 0), mk<T>(0, 0)};
+  if (mine) {
+#pragma unroll
+    for (int q = 0; q < 2; ++q) d[q] = hop_sum(half, 2 * w + q, lane);
+    if (EPI == EPI_MAT) load_pair<P, IO>(hop_field<P, IO, EPI>(a.in, sd, p), t, w, x);
+    if (EPI == EPI_XPAY) load_pair<P, IO_INT>(seg_view(a.x, P, sd.voff, sd.nthr), t, w, x);
+  }
+  if (CLOVER) {
+    // the clover term acts on the sum (its inverse), or on x (EPI_MAT)
+    cplx<T>(*v)[kSplitSites] = half[0];  // 12 components over the first two directions' slots
+    __syncthreads();
+    if (mine) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) v[2 * w + q][lane] = EPI == EPI_MAT ? x[q] : d[q];
+    }
+    __syncthreads();
+    if (mine) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const cplx<T> y = cr.row(cj, q, v + 6 * cb, lane);
+        if (EPI == EPI_MAT)
+          x[q] = y;
+        else
+          d[q] = y;
+      }
+    }
+  }
+  double red[3] = {0, 0, 0};
+  if (mine) {
+    if (EPI == EPI_MAT) {
+      const T kap = (T)sd.kappa;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) d[q] = nmad(x[q], kap, d[q]);
+    }
+    if (EPI == EPI_XPAY) {
+      const T k2 = (T)(sd.kappa * sd.kappa);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        d[q] = nmad(x[q], k2, d[q]);
+        if (RED == RED_OUT_X) {
+          red[0] += (double)d[q].re * (double)x[q].re + (double)d[q].im * (double)x[q].im;
+          red[1] += (double)d[q].re * (double)x[q].im - (double)d[q].im * (double)x[q].re;
+          red[2] += (double)d[q].re * (double)d[q].re + (double)d[q].im * (double)d[q].im;
+        }
+      }
+    }
+    if (RED == RED_DOT_Y_OUT) {
+      cplx<T> y[2];
+      load_pair<P, IO_INT>(seg_view(a.y, P, sd.voff, sd.nthr), t, w, y);
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        red[0] += (double)y[q].re * (double)d[q].re + (double)y[q].im * (double)d[q].im;
+        red[1] += (double)y[q].re * (double)d[q].im - (double)y[q].im * (double)d[q].re;
+      }
+    }
+  }
+  float m = 0.f;
+  if (P == P16) {  // the site's scale over all 12 components
+    __shared__ float mx[6][kSplitSites];
+    if (w < 6)
+      mx[w][lane] = fmaxf(fmaxf(fabsf((float)d[0].re), fabsf((float)d[0].im)),
+                          fmaxf(fabsf((float)d[1].re), fabsf((float)d[1].im)));
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 6; ++k) m = fmaxf(m, mx[k][lane]);
+  }
+  if (mine) store_pair<P, IO>(hop_field<P, IO, EPI>(a.out, sd, p), t, w, d, m);
+  if (RED != RED_NONE) {
+    // the six waves' sums per site, added in order, then the sites of each system
+    constexpr int NR = RED == RED_DOT_Y_OUT ? 2 : 3;
+    __shared__ double sh[NR][6][kSplitSites];
+    if (w < 6) {
+#pragma unroll
+      for (int k = 0; k < NR; ++k) sh[k][w][lane] = red[k];
+    }
+    __syncthreads();
+    if (w >= NR) return;
+    double sum = 0;
+#pragma unroll
+    for (int j = 0; j < 6; ++j) sum += sh[w][j][lane];
+    if (nrhs == 1) {
+      sum = wave_sum(sum);
+      if (lane == 0) a.partials[(size_t)blk * NR + w] = sum;
+    } else {
+      sh[w][0][lane] = sum;  // this wave's own slots
+      __builtin_amdgcn_wave_barrier();
+      if (lane < nrhs) {
+        const int j0 = ((lane - bs.t0 % nrhs) % nrhs + nrhs) % nrhs;
+        double acc = 0;
+        for (int j = j0; j < kSplitSites; j += nrhs) acc += sh[w][0][j];
+        a.partials[((size_t)lane * sd.pcap + blk) * NR + w] = acc;
+      }
+    }
+  }
+}
+
 static int total_blocks(const std::vector<SegDesc> &segs, int bsz) {
   int nb = 0;
   for (const SegDesc &d : segs) nb += (d.nthr + bsz - 1) / bsz;
   return nb;
 }
 
-template <int P, int CLOVER, int EPI, int RED>
-static int launch(const HopKArgs &a, int nb, const LaunchCfg &cfg, hipStream_t s) {
-  switch (cfg.group) {
-    case 1: hipLaunchKernelGGL((k_hop<P, CLOVER, EPI, RED, 1>), dim3(nb), dim3(cfg.block), 0, s, a); break;
-    case 2: hipLaunchKernelGGL((k_hop<P, CLOVER, EPI, RED, 2>), dim3(nb), dim3(cfg.block), 0, s, a); break;
-    default: hipLaunchKernelGGL((k_hop<P, CLOVER, EPI, RED, 0>), dim3(nb), dim3(cfg.block), 0, s, a); break;
+template <int P, int IO, int CLOVER, int EPI, int RED>
+static int launch(const HopKArgs &a, int nb, bool split, const LaunchCfg &cfg, hipStream_t s) {
+  if (split) {
+    hipLaunchKernelGGL((k_hop_split<P, IO, CLOVER, EPI, RED>), dim3(nb), dim3(8 * kSplitSites), 0, s, a);
+  } else {
+    switch (cfg.group) {
+      case 1: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 1>), dim3(nb), dim3(cfg.block), 0, s, a); break;
+      case 2: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 2>), dim3(nb), dim3(cfg.block), 0, s, a); break;
+      default: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 0>), dim3(nb), dim3(cfg.block), 0, s, a); break;
+    }
   }
   QCU_HIP(hipGetLastError());
   return 0;
 }
 
 template <int P>
-static int dispatch(const HopKArgs &a, int nb, int clover, int epi, int red, const LaunchCfg &cfg, hipStream_t s) {
+static int dispatch(const HopKArgs &a, int nb, int clover, int epi, int red, bool split, const LaunchCfg &cfg,
+                    hipStream_t s) {
+  constexpr int I = IO_INT;
   if (epi == EPI_PLAIN) {
-    return clover ? launch<P, 1, EPI_PLAIN, RED_NONE>(a, nb, cfg, s)
-                  : launch<P, 0, EPI_PLAIN, RED_NONE>(a, nb, cfg, s);
+    return clover ? launch<P, I, 1, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s)
+                  : launch<P, I, 0, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s);
   }
   if (red == RED_NONE)
-    return clover ? launch<P, 1, EPI_XPAY, RED_NONE>(a, nb, cfg, s)
-                  : launch<P, 0, EPI_XPAY, RED_NONE>(a, nb, cfg, s);
+    return clover ? launch<P, I, 1, EPI_XPAY, RED_NONE>(a, nb, split, cfg, s)
+                  : launch<P, I, 0, EPI_XPAY, RED_NONE>(a, nb, split, cfg, s);
   if (red == RED_DOT_Y_OUT)
-    return clover ? launch<P, 1, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, cfg, s)
-                  : launch<P, 0, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, cfg, s);
-  return clover ? launch<P, 1, EPI_XPAY, RED_OUT_X>(a, nb, cfg, s)
-                : launch<P, 0, EPI_XPAY, RED_OUT_X>(a, nb, cfg, s);
+    return clover ? launch<P, I, 1, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, cfg, s)
+                  : launch<P, I, 0, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, cfg, s);
+  return clover ? launch<P, I, 1, EPI_XPAY, RED_OUT_X>(a, nb, split, cfg, s)
+                : launch<P, I, 0, EPI_XPAY, RED_OUT_X>(a, nb, split, cfg, s);
+}
+
+static int check_cfg(const LaunchCfg &cfg) {
+  QCU_CHECK(cfg.block >= 64 && cfg.block <= 256 && cfg.block % 64 == 0, QCU_ERR_ARG,
+            "block size must be a multiple of 64 in [64, 256]");
+  return 0;
+}
+
+// Eight waves per 64 sites up to 32 768 virtual sites, where one thread per site
+// gives the chip less than one wave per two SIMDs.  Hop in us, split against one
+// thread per site: 8^4 Wilson FP64 4.9 / 6.9, FP32 4.3 / 6.5; 16^4 (32 768 sites)
+// Wilson FP64 8.8 / 11.3, FP32 6.3 / 8.4, FP16 6.2 / 7.7, clover FP64 13.1 / 13.8,
+// FP16 8.6 / 8.6; 16^3x24 (49 152) Wilson FP64 13.6 / 13.1, clover 18.3 / 16.6.
+constexpr long long kSplitMax = 32768;
+static bool use_split(const BatchOp &op, const LaunchCfg &cfg) {
+  return cfg.automatic && op.nvsites <= kSplitMax;
+}
+
+int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s) {
+  QCU_CHECK(op.segs.size() == 1 && op.nsys == 1, QCU_ERR_ARG, "external fields: one lattice, one right-hand side");
+  LaunchCfg cfg = tuned_cfg(op, P64);
+  QCU_TRY(check_cfg(cfg));
+  HopKArgs a{};
+  a.out.p = out;
+  a.in.p = const_cast<void *>(in);
+  a.segs = op.dev_segs;
+  a.nseg = 1;
+  a.parity = parity;
+  a.remap = cfg.remap;
+  const bool split = use_split(op, cfg);
+  const int nb = total_blocks(op.segs, split ? kSplitSites : cfg.block) * (mat ? 2 : 1);
+  const int clover = use_clover && op.has_clover;
+  if (mat)
+    return clover ? launch<P64, IO_EXT, 1, EPI_MAT, RED_NONE>(a, nb, split, cfg, s)
+                  : launch<P64, IO_EXT, 0, EPI_MAT, RED_NONE>(a, nb, split, cfg, s);
+  return clover ? launch<P64, IO_EXT, 1, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s)
+                : launch<P64, IO_EXT, 0, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s);
 }
 
 int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, int epi, SpinorPtr x, int red,
         SpinorPtr y, SysState *st, double *partials, const LaunchCfg &cfg, hipStream_t s, bool use_clover) {
   QCU_CHECK(parity == 0 || parity == 1, QCU_ERR_ARG, "parity must be 0 or 1");
   QCU_CHECK(prec >= P64 && prec <= P16, QCU_ERR_ARG, "unknown precision");
-  QCU_CHECK(cfg.block >= 64 && cfg.block <= 256 && cfg.block % 64 == 0, QCU_ERR_ARG,
-            "block size must be a multiple of 64 in [64, 256]");
+  QCU_TRY(check_cfg(cfg));
   QCU_CHECK(red == RED_NONE || (epi == EPI_XPAY && st && partials), QCU_ERR_ARG,
             "fused reductions need the xpay epilogue and solver state");
   HopKArgs a;
@@ -300,16 +734,18 @@ int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, in
   a.st = st;
   a.partials = partials;
   const int clover = use_clover && op.has_clover;
-  const int nb = total_blocks(op.segs, cfg.block);
+  const bool split = use_split(op, cfg);
+  const int bsz = split ? kSplitSites : cfg.block;
+  const int nb = total_blocks(op.segs, bsz);
   int rc;
   switch (prec) {
-    case P64: rc = dispatch<P64>(a, nb, clover, epi, red, cfg, s); break;
-    case P32: rc = dispatch<P32>(a, nb, clover, epi, red, cfg, s); break;
-    default: rc = dispatch<P16>(a, nb, clover, epi, red, cfg, s); break;
+    case P64: rc = dispatch<P64>(a, nb, clover, epi, red, split, cfg, s); break;
+    case P32: rc = dispatch<P32>(a, nb, clover, epi, red, split, cfg, s); break;
+    default: rc = dispatch<P16>(a, nb, clover, epi, red, split, cfg, s); break;
   }
   if (rc || red == RED_NONE) return rc;
-  return red == RED_DOT_Y_OUT ? finish(op, partials, cfg.block, 2, FK_ALPHA, st, nullptr, s)
-                              : finish(op, partials, cfg.block, 3, FK_OMEGA, st, nullptr, s);
+  return red == RED_DOT_Y_OUT ? finish(op, partials, bsz, 2, FK_ALPHA, st, nullptr, s)
+                              : finish(op, partials, bsz, 3, FK_OMEGA, st, nullptr, s);
 }
 
 }  // namespace qcu

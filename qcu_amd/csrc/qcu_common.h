@@ -56,16 +56,26 @@ template <class T>
 QCU_HD cplx<T> mul_i(cplx<T> a) { return mk(-a.im, a.re); }
 template <class T>
 QCU_HD cplx<T> mul_mi(cplx<T> a) { return mk(a.im, -a.re); }
-// a += b*c ; a += conj(b)*c
+// a += b*c ; a += conj(b)*c.  The fused operations are written out, so that every
+// kernel rounds these sums alike, whatever is around them.
+QCU_HD double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
+QCU_HD float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <class T>
 QCU_HD void cmad(cplx<T> &a, cplx<T> b, cplx<T> c) {
-  a.re += b.re * c.re - b.im * c.im;
-  a.im += b.re * c.im + b.im * c.re;
+#pragma clang fp contract(off)
+  a.re = a.re + fma_(b.re, c.re, -(b.im * c.im));
+  a.im = a.im + fma_(b.re, c.im, b.im * c.re);
 }
 template <class T>
 QCU_HD void cmadj(cplx<T> &a, cplx<T> b, cplx<T> c) {
-  a.re += b.re * c.re + b.im * c.im;
-  a.im += b.re * c.im - b.im * c.re;
+#pragma clang fp contract(off)
+  a.re = a.re + fma_(b.re, c.re, b.im * c.im);
+  a.im = a.im + fma_(b.re, c.im, -(b.im * c.re));
+}
+// x - k d, in one rounding per component
+template <class T>
+QCU_HD cplx<T> nmad(cplx<T> x, T k, cplx<T> d) {
+  return mk(fma_(-k, d.re, x.re), fma_(-k, d.im, x.im));
 }
 template <class T>
 QCU_HD T norm2(cplx<T> a) { return a.re * a.re + a.im * a.im; }
@@ -343,6 +353,13 @@ struct CloverIO<P16> {
   }
 };
 
+// s a, never fused into what follows
+template <class T>
+QCU_D cplx<T> scale_(T s, cplx<T> a) {
+#pragma clang fp contract(off)
+  return mk(s * a.re, s * a.im);
+}
+
 // out_b = C_b * v_b for chiral block b (spins {2b, 2b+1}) from its 36 packed reals
 template <class T>
 QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
@@ -350,7 +367,7 @@ QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
   const cplx<T> *x = v + 6 * b;
 #pragma unroll
   for (int r = 0; r < 6; ++r) {
-    cplx<T> acc = mk(cb[r] * x[r].re, cb[r] * x[r].im);
+    cplx<T> acc = scale_(cb[r], x[r]);
 #pragma unroll
     for (int col = 0; col < 6; ++col) {
       if (col < r) {

@@ -96,12 +96,15 @@ struct LaunchCfg {
   int block = 256;
   int remap = 1;
   int group = 0;  // hop scheduling groups (see dslash.hip)
+  bool automatic = true;  // no shape was tuned or pinned: dslash.hip may take its split kernel
 };
 
 // --------------------------------------------------------------------------
 // batches: the segment table (qcu_batch.h) on the host and the device
 // --------------------------------------------------------------------------
 struct Lattice;
+struct BatchOp;
+std::string tune_base(const BatchOp &op);
 struct BatchOp {
   std::vector<SegDesc> segs;
   std::vector<const Lattice *> lats;
@@ -110,6 +113,7 @@ struct BatchOp {
   int nsys = 0;
   long long nvsites = 0;
   bool has_clover = false;
+  std::string tune_base;  // see tune_key()
   // one segment per lattice with nrhs[k] right-hand sides
   int build(const std::vector<const Lattice *> &lats, const std::vector<int> &nrhs, hipStream_t s);
   int max_blocks(int bsz) const;
@@ -133,13 +137,18 @@ int spinor_ext_to_batch(const void *ext, const BatchOp &op, int seg, int rhs, Sp
 int spinor_batch_to_ext(SpinorPtr src, const BatchOp &op, int seg, int rhs, void *ext, int prec, hipStream_t s);
 
 // dslash.hip
-enum HopEpi { EPI_PLAIN = 0, EPI_XPAY = 1 };
+enum HopEpi { EPI_PLAIN = 0, EPI_XPAY = 1, EPI_MAT = 2 };
 enum HopRed { RED_NONE = 0, RED_DOT_Y_OUT = 1, RED_OUT_X = 2 };
 // out = [A_p^-1] D_{p,1-p} in                                  (EPI_PLAIN)
 // out = x - kappa^2 [A_p^-1] D_{p,1-p} in                      (EPI_XPAY)
 // RED_DOT_Y_OUT: <y,out> -> alpha update; RED_OUT_X: <out,x>,|out|^2 -> omega
 int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, int epi, SpinorPtr x, int red,
         SpinorPtr y, SysState *st, double *partials, const LaunchCfg &cfg, hipStream_t s, bool use_clover = true);
+
+// the FP64 hop on the caller's fields of a single lattice, which must not overlap:
+// out = [A_p^-1] D_{p,1-p} in on one-parity fields, or (mat) out = A in - kappa D in
+// on full ones
+int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s);
 
 // clover.hip
 // packed A and A^-1 of one parity; FP32 and FP16 copies of A^-1 where asked for

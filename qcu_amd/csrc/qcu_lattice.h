@@ -25,6 +25,10 @@ struct Lattice {
   DevBuf cinv64[2];  // packed A^-1
   DevBuf cinv32[2], cinv16[2], cinv16n[2];
   DevBuf flag;       // singular-clover counter
+  // staging of qcuDslash and qcuMatFull, made on first use and kept: half
+  // spinors of the low precisions, and a copy of an input that overlaps the output
+  Spinor stage[2];
+  DevBuf stage_in;
 
   BatchOp self;      // this lattice as a one-system batch
   std::unique_ptr<Solver> solver;

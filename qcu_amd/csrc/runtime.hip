@@ -91,6 +91,7 @@ int BatchOp::build(const std::vector<const Lattice *> &ls, const std::vector<int
   // block size a reducing kernel uses (64), the same stride for every segment
   const int pcap = max_blocks(64) + 1;
   for (SegDesc &d : segs) d.pcap = pcap;
+  tune_base = qcu::tune_base(*this);
   QCU_TRY(dseg.alloc(segs.size() * sizeof(SegDesc)));
   dev_segs = (SegDesc *)dseg.p;
   QCU_HIP(hipMemcpyAsync(dev_segs, segs.data(), segs.size() * sizeof(SegDesc), hipMemcpyHostToDevice, s));

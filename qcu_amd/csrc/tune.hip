@@ -27,10 +27,20 @@ std::atomic<unsigned long long> g_tune_gen{1};
 // graphs (which hold the launch shapes of their capture) are re-captured
 unsigned long long tune_generation() { return g_tune_gen.load(); }
 
-static void set_tuned(const std::string &key, const LaunchCfg &c) {
+static void set_tuned(const std::string &key, LaunchCfg c) {
+  c.automatic = false;
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     g_tuned[key] = c;
+  }
+  ++g_tune_gen;
+}
+
+// back to the shape that the rule of dslash.hip picks
+static void set_automatic(const std::string &key) {
+  {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    g_tuned.erase(key);
   }
   ++g_tune_gen;
 }
@@ -41,7 +51,10 @@ static int valid_cfg(int block, int remap, int group) {
   return 0;
 }
 
-std::string tune_key(const BatchOp &op, int prec) {
+// the part of a batch's table key that is the same for every precision, formed
+// once when the batch is built (asking the driver for the device costs more
+// than a small hop)
+std::string tune_base(const BatchOp &op) {
   std::string k;
   hipDeviceProp_t prop;
   int dev = current_device();
@@ -51,8 +64,13 @@ std::string tune_key(const BatchOp &op, int prec) {
     snprintf(buf, sizeof(buf), ":%dx%dx%dx%dr%d", 2 * d.g.lxh, d.g.ly, d.g.lz, d.g.lt, d.nrhs);
     k += buf;
   }
+  return k;
+}
+
+std::string tune_key(const BatchOp &op, int prec) {
+  char buf[32];
   snprintf(buf, sizeof(buf), ":p%d:c%d", prec, op.has_clover ? 1 : 0);
-  return k + buf;
+  return op.tune_base + buf;
 }
 
 LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
@@ -101,8 +119,10 @@ int bench_hop(const BatchOp &op, hipStream_t s, int prec, int clover, int xpay, 
 static int tune_op(const BatchOp &op, hipStream_t s, int prec, double *best_ms, LaunchCfg *out) {
   const int clover = op.has_clover ? 1 : 0;
   const int blocks[] = {64, 128, 256};
+  // the shape that the rule picks, then each one-thread-per-site shape
   LaunchCfg best;
   double bms = 1e30;
+  QCU_TRY(bench_hop(op, s, prec, clover, 1, 20, best, &bms));
   for (int grp = 0; grp < 3; ++grp)
     for (int b : blocks)
       for (int r = 0; r < 2; ++r) {
@@ -110,6 +130,7 @@ static int tune_op(const BatchOp &op, hipStream_t s, int prec, double *best_ms, 
         c.block = b;
         c.remap = r;
         c.group = grp;
+        c.automatic = false;
         double ms = 0;
         QCU_TRY(bench_hop(op, s, prec, clover, 1, 20, c, &ms));
         if (ms < bms) {
@@ -117,7 +138,10 @@ static int tune_op(const BatchOp &op, hipStream_t s, int prec, double *best_ms, 
           best = c;
         }
       }
-  set_tuned(tune_key(op, prec), best);
+  if (best.automatic)
+    set_automatic(tune_key(op, prec));
+  else
+    set_tuned(tune_key(op, prec), best);
   if (best_ms) *best_ms = bms;
   if (out) *out = best;
   return 0;
@@ -211,6 +235,7 @@ int qcuTuneLoad(const char *path) {
       c.block = b;
       c.remap = r;
       c.group = grp;
+      c.automatic = false;
       g_tuned[key] = c;
     }
   }
