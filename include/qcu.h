@@ -172,7 +172,9 @@ int qcuBatchTune(QcuBatchHandle h, int prec, double *best_ms);
 
 /* launch-shape autotuner: sweeps block size, XCD-aware block order and the
  * instruction-scheduling grouping of the hop kernel for this lattice and
- * precision and keeps the fastest; the table persists in a text file */
+ * precision and keeps the fastest; the table persists in a text file.  Without
+ * tuning a rule on the size and precision picks the shape, and small lattices run
+ * a kernel of their own; qcuTune keeps that choice where it is the fastest */
 int qcuTune(QcuLatticeHandle h, int prec, double *best_ms);
 int qcuTuneGet(QcuLatticeHandle h, int prec, int *block, int *remap, int *group);
 /* pins the launch shape of the hop kernel for this lattice (or batch) and

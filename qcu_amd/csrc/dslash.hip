@@ -126,7 +126,7 @@ QCU_D void store_spinor(const SpinorPtr &f, int i, const cplx<typename real_of<P
 }
 
 // the transported half spinor (a0, a1) of one direction
-template <int P, int IO, int MU, int FWD>
+template <int P, int IO, int MU, int FWD, bool NT = false>
 QCU_D void hop_half(cplx<typename real_of<P>::type> (&a0)[3], cplx<typename real_of<P>::type> (&a1)[3],
                     const LinkPtr &U, int pm, int li, const SpinorPtr &in, int si, typename real_of<P>::type ph) {
   typedef typename real_of<P>::type T;
@@ -135,7 +135,7 @@ QCU_D void hop_half(cplx<typename real_of<P>::type> (&a0)[3], cplx<typename real
   cplx<T> h0[3], h1[3];
   project<MU, FWD>(s, h0, h1);
   cplx<T> u[9];
-  LinkIO<P>::load(U, pm, li, u);
+  LinkIO<P>::template load<NT>(U, pm, li, u);
   transport<FWD>(u, h0, a0);
   transport<FWD>(u, h1, a1);
   if (MU == 3) {
@@ -147,11 +147,11 @@ QCU_D void hop_half(cplx<typename real_of<P>::type> (&a0)[3], cplx<typename real
   }
 }
 
-template <int P, int IO, int MU, int FWD>
+template <int P, int IO, int MU, int FWD, bool NT>
 QCU_D void hop_dir(cplx<typename real_of<P>::type> (&d)[12], const LinkPtr &U, int pm, int li,
                    const SpinorPtr &in, int si, typename real_of<P>::type ph) {
   cplx<typename real_of<P>::type> a0[3], a1[3];
-  hop_half<P, IO, MU, FWD>(a0, a1, U, pm, li, in, si, ph);
+  hop_half<P, IO, MU, FWD, NT>(a0, a1, U, pm, li, in, si, ph);
   accumulate<MU, FWD>(d, a0, a1);
 }
 
@@ -212,7 +212,7 @@ QCU_D SpinorPtr hop_field(const SpinorPtr &f, const SegDesc &sd, int parity) {
   return v;
 }
 
-template <int P, int IO, int CLOVER, int EPI, int RED, int G>
+template <int P, int IO, int CLOVER, int EPI, int RED, int G, bool NT>
 __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
   typedef typename real_of<P>::type T;
   int p;
@@ -222,10 +222,9 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
   const SegDesc &sd = a.segs[bs.seg];
   const Geom g = sd.g;
   const int nrhs = IO == IO_EXT ? 1 : sd.nrhs;
-  const int t = bs.t0 + threadIdx.x;
-  const int site = t / nrhs;
-  const int rhs = t - site * nrhs;
-  bool active = t < sd.nthr;
+  const int n = bs.t0 + threadIdx.x;
+  const int k = n / nrhs, rhs = n - k * nrhs;
+  bool active = n < sd.nthr;
   // a solver state, when given, stops the work of its system once it has stopped
   if (a.st && active && a.st[sd.sys0 + rhs].done) active = false;
   cplx<T> d[12];
@@ -234,36 +233,37 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
     const int q = 1 - p;
     const SpinorPtr in = hop_field<P, IO, EPI>(a.in, sd, q);
     const LinkPtr U = sd.U[P];
-    const int i = site;
-    const Site s = decode(g, i, p);
+    int i;
+    const Site s = ordered_site(g, sd.zslab[P], k, p, i);
+    const int t = i * nrhs + rhs;
 #pragma unroll
     for (int k = 0; k < 12; ++k) d[k] = mk<T>(0, 0);
     int j, sg;
     // branch-free index arithmetic keeps the body one basic block, so the
     // scheduling fences below bound the live registers
     j = neighbour<0, 0>(g, s, i, sg);
-    hop_dir<P, IO, 0, 0>(d, U, q * 4 + 0, j, in, j * nrhs + rhs, (T)1);
+    hop_dir<P, IO, 0, 0, NT>(d, U, q * 4 + 0, j, in, j * nrhs + rhs, (T)1);
     QCU_GROUP_FENCE(G, 0);
     j = neighbour<0, 1>(g, s, i, sg);
-    hop_dir<P, IO, 0, 1>(d, U, p * 4 + 0, i, in, j * nrhs + rhs, (T)1);
+    hop_dir<P, IO, 0, 1, NT>(d, U, p * 4 + 0, i, in, j * nrhs + rhs, (T)1);
     QCU_GROUP_FENCE(G, 1);
     j = neighbour<1, 0>(g, s, i, sg);
-    hop_dir<P, IO, 1, 0>(d, U, q * 4 + 1, j, in, j * nrhs + rhs, (T)1);
+    hop_dir<P, IO, 1, 0, NT>(d, U, q * 4 + 1, j, in, j * nrhs + rhs, (T)1);
     QCU_GROUP_FENCE(G, 2);
     j = neighbour<1, 1>(g, s, i, sg);
-    hop_dir<P, IO, 1, 1>(d, U, p * 4 + 1, i, in, j * nrhs + rhs, (T)1);
+    hop_dir<P, IO, 1, 1, NT>(d, U, p * 4 + 1, i, in, j * nrhs + rhs, (T)1);
     QCU_GROUP_FENCE(G, 3);
     j = neighbour<2, 0>(g, s, i, sg);
-    hop_dir<P, IO, 2, 0>(d, U, q * 4 + 2, j, in, j * nrhs + rhs, (T)1);
+    hop_dir<P, IO, 2, 0, NT>(d, U, q * 4 + 2, j, in, j * nrhs + rhs, (T)1);
     QCU_GROUP_FENCE(G, 4);
     j = neighbour<2, 1>(g, s, i, sg);
-    hop_dir<P, IO, 2, 1>(d, U, p * 4 + 2, i, in, j * nrhs + rhs, (T)1);
+    hop_dir<P, IO, 2, 1, NT>(d, U, p * 4 + 2, i, in, j * nrhs + rhs, (T)1);
     QCU_GROUP_FENCE(G, 5);
     j = neighbour<3, 0>(g, s, i, sg);
-    hop_dir<P, IO, 3, 0>(d, U, q * 4 + 3, j, in, j * nrhs + rhs, (T)sg);
+    hop_dir<P, IO, 3, 0, NT>(d, U, q * 4 + 3, j, in, j * nrhs + rhs, (T)sg);
     QCU_GROUP_FENCE(G, 6);
     j = neighbour<3, 1>(g, s, i, sg);
-    hop_dir<P, IO, 3, 1>(d, U, p * 4 + 3, i, in, j * nrhs + rhs, (T)sg);
+    hop_dir<P, IO, 3, 1, NT>(d, U, p * 4 + 3, i, in, j * nrhs + rhs, (T)sg);
     QCU_GROUP_FENCE(G, 7);
     if (EPI == EPI_MAT) {
       // A x - kappa d
@@ -271,10 +271,10 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
       load_spinor<P, IO>(hop_field<P, IO, EPI>(a.in, sd, p), t, x);
       if (CLOVER) {
         T c[36];
-        clover_load_block(sd.A[p], i, 0, c);
+        clover_load_block<NT>(sd.A[p], i, 0, c);
         clover_apply_block(c, x, 0);
         QCU_GROUP_FENCE(G, 1);
-        clover_load_block(sd.A[p], i, 1, c);
+        clover_load_block<NT>(sd.A[p], i, 1, c);
         clover_apply_block(c, x, 1);
       }
       const T kap = (T)sd.kappa;
@@ -284,15 +284,15 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
       const CloverPtr C = sd.Cinv[P][p];
       if (P == P16) {
         T c[72];
-        CloverIO<P>::load(C, i, c);
+        CloverIO<P>::template load<NT>(C, i, c);
         clover_apply_site(c, d);
       } else {
         // one chiral block at a time bounds the live registers
         T c[36];
-        clover_load_block(C, i, 0, c);
+        clover_load_block<NT>(C, i, 0, c);
         clover_apply_block(c, d, 0);
         QCU_GROUP_FENCE(G, 1);
-        clover_load_block(C, i, 1, c);
+        clover_load_block<NT>(C, i, 1, c);
         clover_apply_block(c, d, 1);
       }
     }
@@ -504,9 +504,12 @@ __global__ void __launch_bounds__(8 * kSplitSites) k_hop_split(HopKArgs a) {
   const Geom g = sd.g;
   const int nrhs = IO == IO_EXT ? 1 : sd.nrhs;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int t = bs.t0 + lane;
-  const int i = t / nrhs, rhs = t - i * nrhs;
-  bool active = t < sd.nthr;
+  const int n = bs.t0 + lane;
+  const int k = n / nrhs, rhs = n - k * nrhs;
+  bool active = n < sd.nthr;
+  int i;
+  const Site s = ordered_site(g, sd.zslab[P], k, p, i);
+  const int t = i * nrhs + rhs;
   if (a.st && active && a.st[sd.sys0 + rhs].done) active = false;
   const bool mine = active && w < 6;  // this wave's pair of components
   const int cb = w / 3, cj = w - 3 * cb;  // its chiral block and rows 2 cj, 2 cj + 1 of it
@@ -515,7 +518,6 @@ __global__ void __launch_bounds__(8 * kSplitSites) k_hop_split(HopKArgs a) {
     const int q = 1 - p;
     const SpinorPtr in = hop_field<P, IO, EPI>(a.in, sd, q);
     const LinkPtr U = sd.U[P];
-    const Site s = decode(g, i, p);
     cplx<T> a0[3], a1[3];
     int j, sg;
 #define QCU_SPLIT_DIR(MU)                                                                 \
@@ -645,37 +647,45 @@ static int total_blocks(const std::vector<SegDesc> &segs, int bsz) {
   return nb;
 }
 
+template <int P, int IO, int CLOVER, int EPI, int RED, bool NT>
+static void launch_group(const HopKArgs &a, int nb, const LaunchCfg &cfg, hipStream_t s) {
+  const dim3 n(nb), b(cfg.block);
+  switch (cfg.group) {
+    case 1: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 1, NT>), n, b, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 2, NT>), n, b, 0, s, a); break;
+    default: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 0, NT>), n, b, 0, s, a); break;
+  }
+}
+
 template <int P, int IO, int CLOVER, int EPI, int RED>
-static int launch(const HopKArgs &a, int nb, bool split, const LaunchCfg &cfg, hipStream_t s) {
+static int launch(const HopKArgs &a, int nb, bool split, bool nt, const LaunchCfg &cfg, hipStream_t s) {
   if (split) {
     hipLaunchKernelGGL((k_hop_split<P, IO, CLOVER, EPI, RED>), dim3(nb), dim3(8 * kSplitSites), 0, s, a);
+  } else if (nt) {
+    launch_group<P, IO, CLOVER, EPI, RED, true>(a, nb, cfg, s);
   } else {
-    switch (cfg.group) {
-      case 1: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 1>), dim3(nb), dim3(cfg.block), 0, s, a); break;
-      case 2: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 2>), dim3(nb), dim3(cfg.block), 0, s, a); break;
-      default: hipLaunchKernelGGL((k_hop<P, IO, CLOVER, EPI, RED, 0>), dim3(nb), dim3(cfg.block), 0, s, a); break;
-    }
+    launch_group<P, IO, CLOVER, EPI, RED, false>(a, nb, cfg, s);
   }
   QCU_HIP(hipGetLastError());
   return 0;
 }
 
 template <int P>
-static int dispatch(const HopKArgs &a, int nb, int clover, int epi, int red, bool split, const LaunchCfg &cfg,
-                    hipStream_t s) {
+static int dispatch(const HopKArgs &a, int nb, int clover, int epi, int red, bool split, bool nt,
+                    const LaunchCfg &cfg, hipStream_t s) {
   constexpr int I = IO_INT;
   if (epi == EPI_PLAIN) {
-    return clover ? launch<P, I, 1, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s)
-                  : launch<P, I, 0, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s);
+    return clover ? launch<P, I, 1, EPI_PLAIN, RED_NONE>(a, nb, split, nt, cfg, s)
+                  : launch<P, I, 0, EPI_PLAIN, RED_NONE>(a, nb, split, nt, cfg, s);
   }
   if (red == RED_NONE)
-    return clover ? launch<P, I, 1, EPI_XPAY, RED_NONE>(a, nb, split, cfg, s)
-                  : launch<P, I, 0, EPI_XPAY, RED_NONE>(a, nb, split, cfg, s);
+    return clover ? launch<P, I, 1, EPI_XPAY, RED_NONE>(a, nb, split, nt, cfg, s)
+                  : launch<P, I, 0, EPI_XPAY, RED_NONE>(a, nb, split, nt, cfg, s);
   if (red == RED_DOT_Y_OUT)
-    return clover ? launch<P, I, 1, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, cfg, s)
-                  : launch<P, I, 0, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, cfg, s);
-  return clover ? launch<P, I, 1, EPI_XPAY, RED_OUT_X>(a, nb, split, cfg, s)
-                : launch<P, I, 0, EPI_XPAY, RED_OUT_X>(a, nb, split, cfg, s);
+    return clover ? launch<P, I, 1, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, nt, cfg, s)
+                  : launch<P, I, 0, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, nt, cfg, s);
+  return clover ? launch<P, I, 1, EPI_XPAY, RED_OUT_X>(a, nb, split, nt, cfg, s)
+                : launch<P, I, 0, EPI_XPAY, RED_OUT_X>(a, nb, split, nt, cfg, s);
 }
 
 static int check_cfg(const LaunchCfg &cfg) {
@@ -694,6 +704,19 @@ static bool use_split(const BatchOp &op, const LaunchCfg &cfg) {
   return cfg.automatic && op.nvsites <= kSplitMax;
 }
 
+// Links and clover blocks are read once per launch.  Where they do not stay in
+// the 256 MB Infinity Cache from one launch to the next, non-temporal loads leave
+// more of the caches to the spinors, each of which is read eight times.  Clover
+// hop with xpay in us, plain against non-temporal: 32^3x64 FP64 457 / 431, FP32
+// 213 / 199, FP16 111 / 103; 24^3x48 FP64 142 / 131, FP32 65 / 60; but where the
+// fields fit, 24^3x48 FP16 33.7 / 36.0, Wilson FP32 43.6 / 46.2.
+static bool use_nt(const BatchOp &op, int prec, bool clover) {
+  const double real = prec == P64 ? 8 : (prec == P32 ? 4 : 2);
+  double bytes = 0;
+  for (const SegDesc &d : op.segs) bytes += (double)d.g.vh * real * (8 * 12 + (clover ? 72 : 0) + 2 * 24 * d.nrhs);
+  return bytes > 256e6;
+}
+
 int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s) {
   QCU_CHECK(op.segs.size() == 1 && op.nsys == 1, QCU_ERR_ARG, "external fields: one lattice, one right-hand side");
   LaunchCfg cfg = tuned_cfg(op, P64);
@@ -705,14 +728,14 @@ int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, b
   a.nseg = 1;
   a.parity = parity;
   a.remap = cfg.remap;
-  const bool split = use_split(op, cfg);
-  const int nb = total_blocks(op.segs, split ? kSplitSites : cfg.block) * (mat ? 2 : 1);
   const int clover = use_clover && op.has_clover;
+  const bool split = use_split(op, cfg), nt = use_nt(op, P64, clover);
+  const int nb = total_blocks(op.segs, split ? kSplitSites : cfg.block) * (mat ? 2 : 1);
   if (mat)
-    return clover ? launch<P64, IO_EXT, 1, EPI_MAT, RED_NONE>(a, nb, split, cfg, s)
-                  : launch<P64, IO_EXT, 0, EPI_MAT, RED_NONE>(a, nb, split, cfg, s);
-  return clover ? launch<P64, IO_EXT, 1, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s)
-                : launch<P64, IO_EXT, 0, EPI_PLAIN, RED_NONE>(a, nb, split, cfg, s);
+    return clover ? launch<P64, IO_EXT, 1, EPI_MAT, RED_NONE>(a, nb, split, nt, cfg, s)
+                  : launch<P64, IO_EXT, 0, EPI_MAT, RED_NONE>(a, nb, split, nt, cfg, s);
+  return clover ? launch<P64, IO_EXT, 1, EPI_PLAIN, RED_NONE>(a, nb, split, nt, cfg, s)
+                : launch<P64, IO_EXT, 0, EPI_PLAIN, RED_NONE>(a, nb, split, nt, cfg, s);
 }
 
 int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, int epi, SpinorPtr x, int red,
@@ -734,14 +757,14 @@ int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, in
   a.st = st;
   a.partials = partials;
   const int clover = use_clover && op.has_clover;
-  const bool split = use_split(op, cfg);
+  const bool split = use_split(op, cfg), nt = use_nt(op, prec, clover);
   const int bsz = split ? kSplitSites : cfg.block;
   const int nb = total_blocks(op.segs, bsz);
   int rc;
   switch (prec) {
-    case P64: rc = dispatch<P64>(a, nb, clover, epi, red, split, cfg, s); break;
-    case P32: rc = dispatch<P32>(a, nb, clover, epi, red, split, cfg, s); break;
-    default: rc = dispatch<P16>(a, nb, clover, epi, red, split, cfg, s); break;
+    case P64: rc = dispatch<P64>(a, nb, clover, epi, red, split, nt, cfg, s); break;
+    case P32: rc = dispatch<P32>(a, nb, clover, epi, red, split, nt, cfg, s); break;
+    default: rc = dispatch<P16>(a, nb, clover, epi, red, split, nt, cfg, s); break;
   }
   if (rc || red == RED_NONE) return rc;
   return red == RED_DOT_Y_OUT ? finish(op, partials, bsz, 2, FK_ALPHA, st, nullptr, s)

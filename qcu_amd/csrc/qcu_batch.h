@@ -29,6 +29,7 @@ struct SegDesc {
   int nrhs;      // interleaved right-hand sides
   int sys0;      // solver state index of rhs 0
   int nthr;      // vh * nrhs virtual sites
+  int zslab[3];  // z planes per slab of the hop kernels' site order (0: storage order), per precision
   int pcap;      // block-partial slots per right-hand side (the same for every segment of a batch)
   long long voff;  // virtual-site offset of this segment in batch vectors
   double kappa;
@@ -43,21 +44,44 @@ struct BlockSeg {
   int t0;
 };
 
+// The device table of a batch's segments is followed by their first blocks at
+// block sizes 64, 128 and 256 (nseg + 1 cumulative counts each): the search then
+// walks consecutive words instead of one cache line per segment, each a
+// dependent miss (six lattices: the hop 3 us shorter).
+constexpr int kSegBlockSizes = 3;
+QCU_HD int seg_block_size(int k) { return 64 << k; }
+
 QCU_D BlockSeg find_seg(const SegDesc *d, int nseg, int blk, int bsz) {
+  BlockSeg r;
+  if (nseg == 1) {
+    r.seg = blk * bsz < d[0].nthr ? 0 : -1;
+    r.t0 = blk * bsz;
+    return r;
+  }
+  r.seg = -1;
+  r.t0 = 0;
+  const int *first = nullptr;
+  for (int k = 0; k < kSegBlockSizes; ++k)
+    if (bsz == seg_block_size(k)) first = (const int *)(d + nseg) + k * (nseg + 1);
+  if (first) {
+    for (int s = 0; s < nseg; ++s)
+      if (blk < first[s + 1]) {
+        r.seg = s;
+        r.t0 = (blk - first[s]) * bsz;
+        return r;
+      }
+    return r;
+  }
   int acc = 0;
   for (int s = 0; s < nseg; ++s) {
     const int nb = (d[s].nthr + bsz - 1) / bsz;
     if (blk < acc + nb) {
-      BlockSeg r;
       r.seg = s;
       r.t0 = (blk - acc) * bsz;
       return r;
     }
     acc += nb;
   }
-  BlockSeg r;
-  r.seg = -1;
-  r.t0 = 0;
   return r;
 }
 

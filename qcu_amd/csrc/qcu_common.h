@@ -105,13 +105,47 @@ QCU_D Site decode(const Geom &g, int i, int parity) {
   return s;
 }
 
+// Site number k of the order in which the hop kernels visit the sites: with
+// zslab = 0 the storage order, else slabs of zslab z planes one after the other,
+// t by t within a slab (the last slab may be thinner).  i: the half-site index.
+QCU_D Site ordered_site(const Geom &g, int zslab, int k, int parity, int &i) {
+  if (zslab == 0) {
+    i = k;
+    return decode(g, k, parity);
+  }
+  const int plane = g.lxh * g.ly;
+  const int full = zslab * plane * g.lt;
+  const int slab = k / full;
+  const int left = g.lz - slab * zslab;
+  const int row = (left < zslab ? left : zslab) * plane;  // sites of one t in this slab
+  int r = k - slab * full;
+  Site s;
+  s.t = r / row;
+  r -= s.t * row;
+  const int zi = r / plane;
+  r -= zi * plane;
+  s.z = slab * zslab + zi;
+  s.y = r / g.lxh;
+  s.xh = r - s.y * g.lxh;
+  s.xodd = (s.y + s.z + s.t + parity) & 1;
+  i = (s.t * g.lz + s.z) * plane + r;
+  return s;
+}
+
 // Loads and stores address a wavefront-uniform base (component k of a field,
 // kept in scalar registers) plus a 32-bit per-lane byte offset, so that the
 // compiler can use the scalar-base / 32-bit-offset form of global memory
 // instructions instead of a 64-bit address per load and per component.
-template <class V>
+// NT: non-temporal, for data a kernel reads once.
+template <class V, bool NT = false>
 QCU_D V ld_at(const void *base, size_t comp_bytes, unsigned lane_off) {
-  return *(const V *)((const char *)base + comp_bytes + lane_off);
+  const char *p = (const char *)base + comp_bytes + lane_off;
+  if (!NT) return *(const V *)p;
+  typedef unsigned words __attribute__((ext_vector_type(sizeof(V) / 4)));
+  const words w = __builtin_nontemporal_load((const words *)p);
+  V v;
+  __builtin_memcpy(&v, &w, sizeof(V));
+  return v;
 }
 template <class V>
 QCU_D void st_at(void *base, size_t comp_bytes, unsigned lane_off, const V &v) {
@@ -251,17 +285,18 @@ QCU_D void recon_row2(cplx<T> (&u)[9]) {
   u[8] = conj(u[0] * u[4] - u[1] * u[3]);
 }
 
+// load(L, pm, i, u): (p, mu) slab index pm = p*4 + mu
 template <int P>
 struct LinkIO;
 
 template <>
 struct LinkIO<P64> {
-  // (p, mu) slab index pm = p*4 + mu
+  template <bool NT = false>
   static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<double> (&u)[9]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      double2 a = ld_at<double2>(L.a, ((size_t)pm * 6 + k) * L.vh * 16, off);
+      double2 a = ld_at<double2, NT>(L.a, ((size_t)pm * 6 + k) * L.vh * 16, off);
       u[k] = mk(a.x, a.y);
     }
     recon_row2(u);
@@ -270,11 +305,12 @@ struct LinkIO<P64> {
 
 template <>
 struct LinkIO<P32> {
+  template <bool NT = false>
   static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<float> (&u)[9]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      float4 a = ld_at<float4>(L.a, ((size_t)pm * 3 + k) * L.vh * 16, off);
+      float4 a = ld_at<float4, NT>(L.a, ((size_t)pm * 3 + k) * L.vh * 16, off);
       u[2 * k] = mk(a.x, a.y);
       u[2 * k + 1] = mk(a.z, a.w);
     }
@@ -284,9 +320,10 @@ struct LinkIO<P32> {
 
 template <>
 struct LinkIO<P16> {
+  template <bool NT = false>
   static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<float> (&u)[9]) {
-    uint4 a = ld_at<uint4>(L.a, (size_t)pm * L.vh * 16, (unsigned)i * 16u);
-    uint2 b = ld_at<uint2>(L.b, (size_t)pm * L.vh * 8, (unsigned)i * 8u);
+    uint4 a = ld_at<uint4, NT>(L.a, (size_t)pm * L.vh * 16, (unsigned)i * 16u);
+    uint2 b = ld_at<uint2, NT>(L.b, (size_t)pm * L.vh * 8, (unsigned)i * 8u);
     unsigned w[6] = {a.x, a.y, a.z, a.w, b.x, b.y};
 #pragma unroll
     for (int k = 0; k < 6; ++k)
@@ -311,11 +348,12 @@ struct CloverIO;
 
 template <>
 struct CloverIO<P64> {
+  template <bool NT = false>
   static QCU_D void load(const CloverPtr &C, int i, double (&c)[72]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 36; ++k) {
-      double2 a = ld_at<double2>(C.p, (size_t)k * C.vh * 16, off);
+      double2 a = ld_at<double2, NT>(C.p, (size_t)k * C.vh * 16, off);
       c[2 * k] = a.x;
       c[2 * k + 1] = a.y;
     }
@@ -323,11 +361,12 @@ struct CloverIO<P64> {
 };
 template <>
 struct CloverIO<P32> {
+  template <bool NT = false>
   static QCU_D void load(const CloverPtr &C, int i, float (&c)[72]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 18; ++k) {
-      float4 a = ld_at<float4>(C.p, (size_t)k * C.vh * 16, off);
+      float4 a = ld_at<float4, NT>(C.p, (size_t)k * C.vh * 16, off);
       c[4 * k] = a.x;
       c[4 * k + 1] = a.y;
       c[4 * k + 2] = a.z;
@@ -337,12 +376,13 @@ struct CloverIO<P32> {
 };
 template <>
 struct CloverIO<P16> {
+  template <bool NT = false>
   static QCU_D void load(const CloverPtr &C, int i, float (&c)[72]) {
     const unsigned off = (unsigned)i * 16u;
     const float nrm = ld_at<float>(C.norm, 0, (unsigned)i * 4u);
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-      uint4 a = ld_at<uint4>(C.p, (size_t)k * C.vh * 16, off);
+      uint4 a = ld_at<uint4, NT>(C.p, (size_t)k * C.vh * 16, off);
       unsigned w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
       for (int q2 = 0; q2 < 4; ++q2) {
@@ -392,20 +432,22 @@ QCU_D void clover_apply_site(const T (&c)[72], cplx<T> (&v)[12]) {
 }
 
 // load one chiral block (36 reals) of a packed FP64 / FP32 clover field
+template <bool NT = false>
 QCU_D void clover_load_block(const CloverPtr &C, int i, int b, double (&c)[36]) {
   const unsigned off = (unsigned)i * 16u;
 #pragma unroll
   for (int k = 0; k < 18; ++k) {
-    double2 a = ld_at<double2>(C.p, (size_t)(18 * b + k) * C.vh * 16, off);
+    double2 a = ld_at<double2, NT>(C.p, (size_t)(18 * b + k) * C.vh * 16, off);
     c[2 * k] = a.x;
     c[2 * k + 1] = a.y;
   }
 }
+template <bool NT = false>
 QCU_D void clover_load_block(const CloverPtr &C, int i, int b, float (&c)[36]) {
   const unsigned off = (unsigned)i * 16u;
 #pragma unroll
   for (int k = 0; k < 9; ++k) {
-    float4 a = ld_at<float4>(C.p, (size_t)(9 * b + k) * C.vh * 16, off);
+    float4 a = ld_at<float4, NT>(C.p, (size_t)(9 * b + k) * C.vh * 16, off);
     c[4 * k] = a.x;
     c[4 * k + 1] = a.y;
     c[4 * k + 2] = a.z;

@@ -1,4 +1,5 @@
 // runtime.hip -- errors, device buffers, resident lattice state, batches.
+#include <algorithm>
 #include <cstring>
 #include <string>
 
@@ -92,9 +93,17 @@ int BatchOp::build(const std::vector<const Lattice *> &ls, const std::vector<int
   const int pcap = max_blocks(64) + 1;
   for (SegDesc &d : segs) d.pcap = pcap;
   tune_base = qcu::tune_base(*this);
-  QCU_TRY(dseg.alloc(segs.size() * sizeof(SegDesc)));
+  std::vector<int> first;  // see find_seg()
+  for (int k = 0; k < kSegBlockSizes; ++k) {
+    const int bsz = seg_block_size(k);
+    first.push_back(0);
+    for (const SegDesc &d : segs) first.push_back(first.back() + (d.nthr + bsz - 1) / bsz);
+  }
+  const size_t nb = segs.size() * sizeof(SegDesc);
+  QCU_TRY(dseg.alloc(nb + first.size() * sizeof(int)));
   dev_segs = (SegDesc *)dseg.p;
-  QCU_HIP(hipMemcpyAsync(dev_segs, segs.data(), segs.size() * sizeof(SegDesc), hipMemcpyHostToDevice, s));
+  QCU_HIP(hipMemcpyAsync(dev_segs, segs.data(), nb, hipMemcpyHostToDevice, s));
+  QCU_HIP(hipMemcpyAsync((char *)dseg.p + nb, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice, s));
   QCU_HIP(hipStreamSynchronize(s));
   return 0;
 }
@@ -220,12 +229,32 @@ CloverPtr Lattice::clover(int p) const {
   return c;
 }
 
+// z planes per slab of the hop kernels' site order.  In storage order an XCD
+// sweeps its sites time slice by time slice and reads each spinor again one
+// slice later and one after that.  Where two such slices no longer fit an XCD's
+// 4 MB L2, slabs of about 1 MB per slice (at least 3 planes, whose outer
+// neighbours are read twice) keep those reads in it.  Clover hop with xpay in us
+// at 24^3x48 with 12 right-hand sides, storage order against slabs of 3 / 6
+// planes: FP64 947 / 761 / 788, FP32 457 / 371 / 369, FP16 352 / 309 / 307 (2
+// planes: 810, 409, 317); one right-hand side at 32^3x64 FP64 431 / 420 (8 planes).
+// FP32 there, whose slice is 1.6 MB, is 199 in storage order, 212 in slabs of 8.
+static int hop_slab(const Geom &g, int nrhs, int prec) {
+  const double site = prec == P64 ? 192 : (prec == P32 ? 96 : 52);
+  const double plane = (double)g.lxh * g.ly * nrhs * site;
+  if (plane * g.lz <= 2e6) return 0;
+  const int most = std::max(3, (int)(1e6 / plane));
+  if (most >= g.lz) return 0;
+  const int slabs = (g.lz + most - 1) / most;
+  return (g.lz + slabs - 1) / slabs;
+}
+
 SegDesc Lattice::seg_desc(int nrhs) const {
   SegDesc d;
   std::memset(&d, 0, sizeof(d));
   d.g = g;
   d.nrhs = nrhs;
   d.nthr = g.vh * nrhs;
+  for (int p = 0; p < 3; ++p) d.zslab[p] = hop_slab(g, nrhs, p);
   d.kappa = kappa;
   for (int p = 0; p < 3; ++p) {
     d.U[p] = links(p);

@@ -74,10 +74,20 @@ std::string tune_key(const BatchOp &op, int prec) {
 }
 
 LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
-  std::lock_guard<std::mutex> lk(g_tune_mu);
-  auto it = g_tuned.find(tune_key(op, prec));
-  if (it != g_tuned.end()) return it->second;
-  return LaunchCfg();
+  {
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    auto it = g_tuned.find(tune_key(op, prec));
+    if (it != g_tuned.end()) return it->second;
+  }
+  // no shape tuned or pinned: single-wave blocks refill a SIMD as soon as a wave
+  // ends (24^3x48 FP64 142 against 149 us in blocks of 256); large batches take
+  // longer blocks, which run as fast there and write fewer block partials.  The
+  // low precisions fence their directions in pairs (24^3x48 FP32 65 against 73 us
+  // unfenced), FP64 needs every load in flight (32^3x64 plain 282 against 288 us).
+  LaunchCfg c;
+  c.block = op.nvsites <= (1 << 20) ? 64 : 256;
+  c.group = prec == P64 ? 0 : 2;
+  return c;
 }
 
 // average milliseconds per launch of the hop kernel on resident fields
