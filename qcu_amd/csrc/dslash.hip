@@ -50,6 +50,37 @@ QCU_D void project(const cplx<T> (&s)[12], cplx<T> (&h0)[3], cplx<T> (&h1)[3]) {
   }
 }
 
+// the same from the stored halves of an FP16 spinor, scaled by its norm: a
+// component is norm s_a +- norm s_b in two mixed FMAs, without conversions
+template <int MU, int FWD>
+QCU_D void project_raw(const _Float16 (&s)[24], float nrm, cplx<float> (&h0)[3], cplx<float> (&h1)[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    // base spin a, partner b, factor: +-1 (f = 0) or +-i (f = 1)
+    auto comb = [&](int a, int b, int f, int sgn) {
+      const int ka = 2 * (3 * a + c), kb = 2 * (3 * b + c);
+      const float re = nrm * (float)s[ka], im = nrm * (float)s[ka + 1];
+      const float n = sgn > 0 ? nrm : -nrm;
+      if (f == 0) return mk(fma_(n, (float)s[kb], re), fma_(n, (float)s[kb + 1], im));
+      return mk(fma_(-n, (float)s[kb + 1], re), fma_(n, (float)s[kb], im));
+    };
+    const int w = FWD ? -1 : 1;  // sign of the gamma term
+    if (MU == 0) {
+      h0[c] = comb(0, 3, 1, w);
+      h1[c] = comb(1, 2, 1, w);
+    } else if (MU == 1) {
+      h0[c] = comb(0, 3, 0, -w);
+      h1[c] = comb(1, 2, 0, w);
+    } else if (MU == 2) {
+      h0[c] = comb(0, 2, 1, w);
+      h1[c] = comb(1, 3, 1, -w);
+    } else {
+      h0[c] = comb(0, 2, 0, w);
+      h1[c] = comb(1, 3, 0, w);
+    }
+  }
+}
+
 // add the reconstructed 4-spinor of the transported half spinor (a0, a1)
 template <int MU, int FWD, class T>
 QCU_D void accumulate(cplx<T> (&d)[12], const cplx<T> (&a0)[3], const cplx<T> (&a1)[3]) {
@@ -74,7 +105,7 @@ QCU_D void accumulate(cplx<T> (&d)[12], const cplx<T> (&a0)[3], const cplx<T> (&
 }
 
 // a = U h (FWD) or U^dag h
-template <int FWD, class T>
+template <int FWD, bool CHAIN, class T>
 QCU_D void transport(const cplx<T> (&u)[9], const cplx<T> (&h)[3], cplx<T> (&a)[3]) {
 #pragma unroll
   for (int r = 0; r < 3; ++r) {
@@ -82,9 +113,9 @@ QCU_D void transport(const cplx<T> (&u)[9], const cplx<T> (&h)[3], cplx<T> (&a)[
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       if (FWD)
-        cmad(acc, u[r * 3 + c], h[c]);
+        cmad_<CHAIN>(acc, u[r * 3 + c], h[c]);
       else
-        cmadj(acc, u[c * 3 + r], h[c]);
+        cmadj_<CHAIN>(acc, u[c * 3 + r], h[c]);
     }
     a[r] = acc;
   }
@@ -130,14 +161,20 @@ template <int P, int IO, int MU, int FWD, bool NT = false>
 QCU_D void hop_half(cplx<typename real_of<P>::type> (&a0)[3], cplx<typename real_of<P>::type> (&a1)[3],
                     const LinkPtr &U, int pm, int li, const SpinorPtr &in, int si, typename real_of<P>::type ph) {
   typedef typename real_of<P>::type T;
-  cplx<T> s[12];
-  load_spinor<P, IO>(in, si, s);
   cplx<T> h0[3], h1[3];
-  project<MU, FWD>(s, h0, h1);
+  if constexpr (P == P16) {
+    _Float16 s[24];
+    const float nrm = SpinorIO<P16>::load_raw(in, si, s);
+    project_raw<MU, FWD>(s, nrm, h0, h1);
+  } else {
+    cplx<T> s[12];
+    load_spinor<P, IO>(in, si, s);
+    project<MU, FWD>(s, h0, h1);
+  }
   cplx<T> u[9];
   LinkIO<P>::template load<NT>(U, pm, li, u);
-  transport<FWD>(u, h0, a0);
-  transport<FWD>(u, h1, a1);
+  transport<FWD, P == P16>(u, h0, a0);
+  transport<FWD, P == P16>(u, h1, a1);
   if (MU == 3) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
@@ -282,10 +319,12 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
       for (int k = 0; k < 12; ++k) d[k] = nmad(x[k], kap, d[k]);
     } else if (CLOVER) {
       const CloverPtr C = sd.Cinv[P][p];
-      if (P == P16) {
+      if constexpr (P == P16) {
         T c[72];
-        CloverIO<P>::template load<NT>(C, i, c);
-        clover_apply_site(c, d);
+        const float nrm = CloverIO<P>::template load<NT>(C, i, c);
+        clover_apply_site<true>(c, d);
+#pragma unroll
+        for (int k = 0; k < 12; ++k) d[k] = scale_(nrm, d[k]);
       } else {
         // one chiral block at a time bounds the live registers
         T c[36];
@@ -401,7 +440,7 @@ struct CloverWord<P64> {
   static QCU_D raw load(const CloverPtr &C, unsigned off, int n) {
     return ld_at<double2>(C.p, (size_t)n * C.vh * 16, off);
   }
-  static QCU_D cplx<double> value(raw a, float) { return mk(a.x, a.y); }
+  static QCU_D cplx<double> value(raw a) { return mk(a.x, a.y); }
 };
 template <>
 struct CloverWord<P32> {
@@ -409,7 +448,7 @@ struct CloverWord<P32> {
   static QCU_D raw load(const CloverPtr &C, unsigned off, int n) {
     return ld_at<float2>((char *)C.p + 8 * (n & 1), (size_t)(n >> 1) * C.vh * 16, off);
   }
-  static QCU_D cplx<float> value(raw a, float) { return mk(a.x, a.y); }
+  static QCU_D cplx<float> value(raw a) { return mk(a.x, a.y); }
 };
 template <>
 struct CloverWord<P16> {
@@ -417,8 +456,8 @@ struct CloverWord<P16> {
   static QCU_D raw load(const CloverPtr &C, unsigned off, int n) {
     return ld_at<unsigned>((char *)C.p + 4 * (n & 3), (size_t)(n >> 2) * C.vh * 16, off);
   }
-  static QCU_D cplx<float> value(raw a, float nrm) {
-    return mk(nrm * h2f((unsigned short)(a & 0xffffu)), nrm * h2f((unsigned short)(a >> 16)));
+  static QCU_D cplx<float> value(raw a) {
+    return mk(h2f((unsigned short)(a & 0xffffu)), h2f((unsigned short)(a >> 16)));
   }
 };
 
@@ -450,19 +489,19 @@ struct CloverRows {
   // in the order of clover_apply_block
   QCU_D cplx<T> row(int j, int q, const cplx<T> (*x)[kSplitSites], int lane) const {
     const int r = 2 * j + q;
-    const cplx<T> d = CloverWord<P>::value(dg, nrm);
+    const cplx<T> d = CloverWord<P>::value(dg);
     const T diag = q ? d.im : d.re;
     const cplx<T> v = x[r][lane];
     cplx<T> acc = scale_(diag, v);
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
-      const cplx<T> c = CloverWord<P>::value(e[q][k], nrm);
+      const cplx<T> c = CloverWord<P>::value(e[q][k]);
       if (k < r)
-        cmad(acc, c, x[k][lane]);
+        cmad_<P == P16>(acc, c, x[k][lane]);
       else
-        cmadj(acc, c, x[k + 1][lane]);
+        cmadj_<P == P16>(acc, c, x[k + 1][lane]);
     }
-    return acc;
+    return P == P16 ? scale_((T)nrm, acc) : acc;
   }
 };
 

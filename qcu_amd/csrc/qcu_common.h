@@ -72,6 +72,29 @@ QCU_HD void cmadj(cplx<T> &a, cplx<T> b, cplx<T> c) {
   a.re = a.re + fma_(b.re, c.re, b.im * c.im);
   a.im = a.im + fma_(b.re, c.im, -(b.im * c.re));
 }
+// cmad / cmadj, or with CHAIN the products as chained FMAs: 2 instructions per
+// component instead of 3, at one more rounding.  For the FP16 fields, whose hop
+// is near its vector rate (24^3x48 with 12 right-hand sides 356 against 310 us)
+// and whose halves the FMAs take unconverted; the FP32 hop is slower with it
+// (380 against 395 us: longer dependent chains).
+template <bool CHAIN, class T>
+QCU_HD void cmad_(cplx<T> &a, cplx<T> b, cplx<T> c) {
+  if (CHAIN) {
+    a.re = fma_(-b.im, c.im, fma_(b.re, c.re, a.re));
+    a.im = fma_(b.im, c.re, fma_(b.re, c.im, a.im));
+  } else {
+    cmad(a, b, c);
+  }
+}
+template <bool CHAIN, class T>
+QCU_HD void cmadj_(cplx<T> &a, cplx<T> b, cplx<T> c) {
+  if (CHAIN) {
+    a.re = fma_(b.im, c.im, fma_(b.re, c.re, a.re));
+    a.im = fma_(-b.im, c.re, fma_(b.re, c.im, a.im));
+  } else {
+    cmadj(a, b, c);
+  }
+}
 // x - k d, in one rounding per component
 template <class T>
 QCU_HD cplx<T> nmad(cplx<T> x, T k, cplx<T> d) {
@@ -236,6 +259,17 @@ QCU_D unsigned short f2h(float f) { return __half_as_ushort(__float2half_rn(f));
 template <>
 struct SpinorIO<P16> {
   typedef float real;
+  // the stored halves and their scale: an FMA takes a half operand as it is
+  // (v_fma_mix_f32), so kernels that go on with products need not convert it
+  static QCU_D float load_raw(const SpinorPtr &f, int i, _Float16 (&h)[24]) {
+    const unsigned off = (unsigned)i * 16u;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint4 a = ld_at<uint4>(f.p, (size_t)k * f.stride * 16, off);
+      __builtin_memcpy(&h[8 * k], &a, 16);
+    }
+    return ld_at<float>(f.norm, 0, (unsigned)i * 4u);
+  }
   static QCU_D void load(const SpinorPtr &f, int i, cplx<float> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
     const float nrm = ld_at<float>(f.norm, 0, (unsigned)i * 4u);
@@ -284,6 +318,17 @@ QCU_D void recon_row2(cplx<T> (&u)[9]) {
   u[7] = conj(u[2] * u[3] - u[0] * u[5]);
   u[8] = conj(u[0] * u[4] - u[1] * u[3]);
 }
+// the same with chained FMAs
+QCU_D cplx<float> cross_chain(cplx<float> a, cplx<float> b, cplx<float> c, cplx<float> d) {  // conj(a b - c d)
+  const float re = fma_(c.im, d.im, fma_(-c.re, d.re, fma_(-a.im, b.im, a.re * b.re)));
+  const float im = fma_(c.im, d.re, fma_(c.re, d.im, fma_(-a.im, b.re, -(a.re * b.im))));
+  return mk(re, im);
+}
+QCU_D void recon_row2_chain(cplx<float> (&u)[9]) {
+  u[6] = cross_chain(u[1], u[5], u[2], u[4]);
+  u[7] = cross_chain(u[2], u[3], u[0], u[5]);
+  u[8] = cross_chain(u[0], u[4], u[1], u[3]);
+}
 
 // load(L, pm, i, u): (p, mu) slab index pm = p*4 + mu
 template <int P>
@@ -328,7 +373,7 @@ struct LinkIO<P16> {
 #pragma unroll
     for (int k = 0; k < 6; ++k)
       u[k] = mk(h2f((unsigned short)(w[k] & 0xffffu)), h2f((unsigned short)(w[k] >> 16)));
-    recon_row2(u);
+    recon_row2_chain(u);
   }
 };
 
@@ -376,20 +421,19 @@ struct CloverIO<P32> {
 };
 template <>
 struct CloverIO<P16> {
+  // the stored halves and their scale, which the caller applies to the product
   template <bool NT = false>
-  static QCU_D void load(const CloverPtr &C, int i, float (&c)[72]) {
+  static QCU_D float load(const CloverPtr &C, int i, float (&c)[72]) {
     const unsigned off = (unsigned)i * 16u;
-    const float nrm = ld_at<float>(C.norm, 0, (unsigned)i * 4u);
+    _Float16 h[72];
 #pragma unroll
     for (int k = 0; k < 9; ++k) {
-      uint4 a = ld_at<uint4, NT>(C.p, (size_t)k * C.vh * 16, off);
-      unsigned w[4] = {a.x, a.y, a.z, a.w};
-#pragma unroll
-      for (int q2 = 0; q2 < 4; ++q2) {
-        c[8 * k + 2 * q2] = nrm * h2f((unsigned short)(w[q2] & 0xffffu));
-        c[8 * k + 2 * q2 + 1] = nrm * h2f((unsigned short)(w[q2] >> 16));
-      }
+      const uint4 a = ld_at<uint4, NT>(C.p, (size_t)k * C.vh * 16, off);
+      __builtin_memcpy(&h[8 * k], &a, 16);
     }
+#pragma unroll
+    for (int k = 0; k < 72; ++k) c[k] = (float)h[k];
+    return ld_at<float>(C.norm, 0, (unsigned)i * 4u);
   }
 };
 
@@ -401,7 +445,7 @@ QCU_D cplx<T> scale_(T s, cplx<T> a) {
 }
 
 // out_b = C_b * v_b for chiral block b (spins {2b, 2b+1}) from its 36 packed reals
-template <class T>
+template <bool CHAIN = false, class T>
 QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
   cplx<T> o[6];
   const cplx<T> *x = v + 6 * b;
@@ -412,10 +456,10 @@ QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
     for (int col = 0; col < 6; ++col) {
       if (col < r) {
         int k = 6 + 2 * (r * (r - 1) / 2 + col);
-        cmad(acc, mk(cb[k], cb[k + 1]), x[col]);
+        cmad_<CHAIN>(acc, mk(cb[k], cb[k + 1]), x[col]);
       } else if (col > r) {
         int k = 6 + 2 * (col * (col - 1) / 2 + r);
-        cmadj(acc, mk(cb[k], cb[k + 1]), x[col]);
+        cmadj_<CHAIN>(acc, mk(cb[k], cb[k + 1]), x[col]);
       }
     }
     o[r] = acc;
@@ -425,10 +469,10 @@ QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
 }
 
 // out = C * v for one site (both chiral blocks)
-template <class T>
+template <bool CHAIN, class T>
 QCU_D void clover_apply_site(const T (&c)[72], cplx<T> (&v)[12]) {
-  clover_apply_block(c, v, 0);
-  clover_apply_block(c + 36, v, 1);
+  clover_apply_block<CHAIN>(c, v, 0);
+  clover_apply_block<CHAIN>(c + 36, v, 1);
 }
 
 // load one chiral block (36 reals) of a packed FP64 / FP32 clover field
