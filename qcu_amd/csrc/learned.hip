@@ -747,7 +747,20 @@ __global__ void __launch_bounds__(256) k_net_wgrad(NetWgradArgs a) {
 // instead of from HBM once per term.  XCD k takes the site blocks
 // k nsb / 8 .. (k + 1) nsb / 8 - 1, so at each step of the waves' sweep it
 // works on one contiguous stretch of sites (their y neighbours included).
-constexpr int kWgBlocks = 1024;  // blocks per term (a multiple of 8)
+constexpr int kWgBlocks = 1024;  // most blocks per term (a multiple of 8)
+
+// Blocks per term, a multiple of 8.  Each leaves an 8 KiB sum that
+// k_net_wgrad_fin reads again, so a block takes at least 16 steps of 32 sites;
+// smaller lattices take up to 88 blocks, which with 9 terms and 3 blocks per CU
+// fill the chip once (16^3x32, 8 -> 8: 1024 blocks 282 + 80 us for the sum, 256
+// blocks 270 + 6 us).
+static int wgrad_blocks(int vh) {
+  const int steps = (2 * vh + 31) / 32;
+  int n = steps / 16;
+  if (n < 88) n = steps < 88 ? steps : 88;
+  n = (n + 7) & ~7;
+  return n < kWgBlocks ? n : kWgBlocks;
+}
 
 template <int MT, int NT, bool SPLIT, bool LDS>
 __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *part) {
@@ -1080,45 +1093,51 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
   }
 }
 
-// gW[t][o][i][s][s2] = sum over the blocks of term t, FP64 accumulation in block
-// order, times the inverse operand scales of the split products (null maxima:
-// unscaled FP32 products)
+// gW[t][o][i][s][s2] = sum over the blocks of term t, FP64 accumulation in a
+// fixed order, times the inverse operand scales of the split products (null
+// maxima: unscaled FP32 products).  One block per (t, mt, nt, s): its lanes are
+// the 64 entries (o, i, s2) that lie together, and its waves take the blocks in
+// turn.  (One thread per entry left 36 blocks to read 75 MB: 80 us.)
+constexpr int kFinWaves = 16;
 template <int MT, int NT>
-__global__ void k_net_wgrad_fin(const float *part, int nblk, int cin, int cout, float2 *gW, const unsigned *gmax,
-                                const unsigned *amax) {
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;  // over 9 * cout * cin * 16
-  const int total = 9 * cout * cin * 16;
-  if (idx >= total) return;
-  const int e = idx % 16, s = e >> 2, s2 = e & 3;
-  const int ci = (idx / 16) % cin;
-  const int o = (idx / 16 / cin) % cout;
-  const int t = idx / 16 / cin / cout;
+__global__ void __launch_bounds__(64 * kFinWaves) k_net_wgrad_fin(const float *part, int nblk, int cin, int cout,
+                                                                  float2 *gW, const unsigned *gmax,
+                                                                  const unsigned *amax) {
   constexpr int NREG = MT * NT * 2 * 4;
-  const int mt = o >> 2, nt = ci >> 2;
-  const int lane = (o & 3) * 16 + (ci & 3) * 4 + s2;
+  __shared__ double sh[2][kFinWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  int e = blockIdx.x;
+  const int s = e & 3;
+  e >>= 2;
+  const int nt = e % NT;
+  e /= NT;
+  const int mt = e % MT, t = e / MT;
   const int r = ((mt * NT + nt) * 2) * 4 + s;
-  // 8 interleaved FP64 sums (block b into sum b % 8) keep 16 loads in flight;
-  // they are combined in a fixed order, so the result is the same every run
-  constexpr int kAcc = 8;
-  double re[kAcc] = {}, im[kAcc] = {};
   const float *src = part + ((size_t)t * nblk * NREG + r) * 64 + lane;
   const size_t bstride = (size_t)NREG * 64;
-  int b = 0;
-  for (; b + kAcc <= nblk; b += kAcc)
+  double re[4] = {}, im[4] = {};
+  int b = wave;
+  for (; b + 3 * kFinWaves < nblk; b += 4 * kFinWaves)
 #pragma unroll
-    for (int k = 0; k < kAcc; ++k) {
-      re[k] += src[(b + k) * bstride];
-      im[k] += src[(b + k) * bstride + 4 * 64];
+    for (int k = 0; k < 4; ++k) {
+      re[k] += src[(b + k * kFinWaves) * bstride];
+      im[k] += src[(b + k * kFinWaves) * bstride + 4 * 64];
     }
-  for (; b < nblk; ++b) {
-    re[b % kAcc] += src[b * bstride];
-    im[b % kAcc] += src[b * bstride + 4 * 64];
+  for (; b < nblk; b += kFinWaves) {
+    re[0] += src[b * bstride];
+    im[0] += src[b * bstride + 4 * 64];
   }
+  sh[0][wave][lane] = (re[0] + re[1]) + (re[2] + re[3]);
+  sh[1][wave][lane] = (im[0] + im[1]) + (im[2] + im[3]);
+  __syncthreads();
+  if (wave) return;
+  const int o = 4 * mt + (lane >> 4), ci = 4 * nt + ((lane >> 2) & 3), s2 = lane & 3;
+  if (o >= cout || ci >= cin) return;
   double sr = 0, si = 0;
 #pragma unroll
-  for (int k = 0; k < kAcc; ++k) {
-    sr += re[k];
-    si += im[k];
+  for (int k = 0; k < kFinWaves; ++k) {
+    sr += sh[0][k][lane];
+    si += sh[1][k][lane];
   }
   if (gmax) {
     const double inv = 1.0 / ((double)pow2_scale(__uint_as_float(*gmax), 14) *
@@ -1126,7 +1145,7 @@ __global__ void k_net_wgrad_fin(const float *part, int nblk, int cin, int cout, 
     sr *= inv;
     si *= inv;
   }
-  gW[idx] = make_float2((float)sr, (float)si);
+  gW[(((size_t)t * cout + o) * cin + ci) * 16 + 4 * s + s2] = make_float2((float)sr, (float)si);
 }
 
 // second stage: gW[t][o][ci][16] = sum over blocks (FP64 accumulation)
@@ -1254,22 +1273,23 @@ __global__ void k_g5_xpay(SpinorPtr out, SpinorPtr r, SpinorPtr u, float k2, flo
   SpinorIO<P32>::store(out, i, rv);
 }
 
-// res = y - b (FP32 odd), |res|^2 into partials per block (FP64)
-__global__ void k_sub_norm(SpinorPtr res, SpinorPtr y, SpinorPtr b, float bscale, int vh, double *partials) {
+// res = y - b (FP32 odd); |res|^2 and |b|^2 per block into partials (FP64)
+__global__ void k_sub_norms(SpinorPtr res, SpinorPtr y, SpinorPtr b, int vh, double *partials) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  double acc[1] = {0};
+  double acc[2] = {0, 0};
   if (i < vh) {
     cf yv[12], bv[12];
     SpinorIO<P32>::load(y, i, yv);
     SpinorIO<P32>::load(b, i, bv);
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
-      yv[k] = mk(yv[k].re - bscale * bv[k].re, yv[k].im - bscale * bv[k].im);
+      yv[k] = mk(yv[k].re - bv[k].re, yv[k].im - bv[k].im);
       acc[0] += (double)yv[k].re * yv[k].re + (double)yv[k].im * yv[k].im;
+      acc[1] += (double)bv[k].re * bv[k].re + (double)bv[k].im * bv[k].im;
     }
     SpinorIO<P32>::store(res, i, yv);
   }
-  block_partial<1>(acc, partials, blockIdx.x);
+  block_partial<2>(acc, partials, blockIdx.x);
 }
 
 // FP32 odd vector <- external one-parity complex128 field, scaled
@@ -1382,6 +1402,7 @@ struct Net : Precond {
   DevBuf fpk2;                  // its packed operands (net_pack_fuse), then its inverse scale
   unsigned long long wver = 1;  // weight version (bumped on every change of W)
   unsigned long long packed_ver = 0;
+  unsigned long long packed_t_ver = 0;  // the same for Wt and its packed operands
   size_t field_bytes() const { return (size_t)lat->g.vh * 2 * 96; }  // one channel, both parities
   // layer k (or its transpose, dir 1: cin <-> cout) runs on the split kernel
   bool split_layer(int k, int dir) const {
@@ -1505,7 +1526,7 @@ int Net::init(Lattice *l, int nlayers, const int *ch, uint64_t seed, double init
   QCU_TRY(gbuf[0].alloc(cmax * field_bytes()));
   QCU_TRY(gbuf[1].alloc(cmax * field_bytes()));
   QCU_TRY(tmp.alloc((size_t)6 * lat->g.vh * 96));
-  QCU_TRY(red.alloc(((size_t)lat->g.vh / 64 + 16) * 8));
+  QCU_TRY(red.alloc(((size_t)lat->g.vh / 64 + 16) * 8));  // at least two sums per 256 sites
   // weight-gradient partials: combos (9 cin * groups) * blocks * CO*32 floats
   size_t wp = 0;
   for (int k = 0; k < nl; ++k) {
@@ -1858,19 +1879,21 @@ int Net::forward(const SysState *st, hipStream_t s, bool odd_only_last, int zero
 // gout_last: gradient w.r.t. act[nl]; accumulates nothing, writes gW (this sample)
 int Net::backward(SpinorPtr gout, hipStream_t s, bool want_grad_in, SpinorPtr grad_in, int gout_zero_par,
                   int act0_zero_par) {
-  // conjugate-transposed weights for the data gradient
-  for (int k = 0; k < nl; ++k) {
-    const int total = 9 * chan[k] * chan[k + 1] * 16;
-    hipLaunchKernelGGL(k_net_transpose, dim3((unsigned)ndiv(total, 256)), dim3(256), 0, s,
-                       (const float2 *)W.p + woff[k], (float2 *)Wt.p + woff[k], chan[k], chan[k + 1]);
-  }
-  QCU_HIP(hipGetLastError());
   bool any = false;
   for (int k = 0; k < nl; ++k) any = any || split_layer(k, 1);
-  if (any) {
-    QCU_TRY(pack_split(1, s));
-    QCU_TRY(reset_max(1, s));
+  // conjugate-transposed weights for the data gradient, once per weight version
+  // (the samples of a training batch share them)
+  if (packed_t_ver != wver) {
+    for (int k = 0; k < nl; ++k) {
+      const int total = 9 * chan[k] * chan[k + 1] * 16;
+      hipLaunchKernelGGL(k_net_transpose, dim3((unsigned)ndiv(total, 256)), dim3(256), 0, s,
+                         (const float2 *)W.p + woff[k], (float2 *)Wt.p + woff[k], chan[k], chan[k + 1]);
+    }
+    QCU_HIP(hipGetLastError());
+    if (any) QCU_TRY(pack_split(1, s));
+    packed_t_ver = wver;
   }
+  if (any) QCU_TRY(reset_max(1, s));
   SpinorPtr gcur = gout;
   int ping = 0;
   for (int k = nl - 1; k >= 0; --k) {
@@ -1897,18 +1920,18 @@ int Net::backward(SpinorPtr gout, hipStream_t s, bool want_grad_in, SpinorPtr gr
     if (use_mfma) {
       const int mt = (cout + 3) / 4, nt = (cin + 3) / 4;
       static_assert(kWgBlocks % 8 == 0, "term blocks of a site block share an XCD");
-      const dim3 grid(9 * kWgBlocks);
+      const int nwb = wgrad_blocks(lat->g.vh);
+      const dim3 grid(9 * nwb);
       float *pp = (float *)wpart.p;
       float2 *dst = (float2 *)gW.p + woff[k];
-      const dim3 fg((unsigned)ndiv(total, 256));
       auto run = [&](auto mtc, auto ntc, auto splitc) {
         constexpr int MT_ = decltype(mtc)::value, NT_ = decltype(ntc)::value;
         if (wg_lds)
           hipLaunchKernelGGL((k_net_wgrad_mfma<MT_, NT_, decltype(splitc)::value, true>), grid, dim3(256), 0, s, a, pp);
         else
           hipLaunchKernelGGL((k_net_wgrad_mfma<MT_, NT_, decltype(splitc)::value, false>), grid, dim3(256), 0, s, a, pp);
-        hipLaunchKernelGGL((k_net_wgrad_fin<MT_, NT_>), fg, dim3(256), 0, s, (const float *)pp, kWgBlocks, cin, cout,
-                           dst, a.gmax, a.amax);
+        hipLaunchKernelGGL((k_net_wgrad_fin<MT_, NT_>), dim3(9 * MT_ * NT_ * 4), dim3(64 * kFinWaves), 0, s,
+                           (const float *)pp, nwb, cin, cout, dst, a.gmax, a.amax);
       };
       using I1 = std::integral_constant<int, 1>;
       using I2 = std::integral_constant<int, 2>;
@@ -2032,20 +2055,7 @@ struct NetTrainer {
     Lattice &lat = *net.lat;
     const int vh = lat.g.vh, bs = 256;
     const unsigned nb = (unsigned)ndiv(vh, bs);
-    // |b|^2
-    double *red = (double *)net.red.p;
-    hipLaunchKernelGGL(k_sub_norm, dim3(nb), dim3(bs), 0, s, odd(5), odd(0), odd(0), 0.f, vh, red);
-    QCU_HIP(hipGetLastError());
-    std::vector<double> h(nb);
-    QCU_HIP(hipMemcpyAsync(h.data(), red, nb * 8, hipMemcpyDeviceToHost, s));
-    QCU_HIP(hipStreamSynchronize(s));
-    double b2 = 0;
-    for (double x : h) b2 += x;
-    if (!(b2 > 0)) {
-      *loss = 0;
-      return 0;
-    }
-    // y = K b / |b|
+    // y = K b
     QCU_TRY(net.load_input(odd(0), P32, nullptr, s));
     // only the odd part of the output enters the loss: the last layer runs on
     // the odd sites only, as in the preconditioner
@@ -2053,13 +2063,22 @@ struct NetTrainer {
     hipLaunchKernelGGL(k_net_extract<P32>, dim3(nb), dim3(bs), 0, s, odd(1), net.act_ptr(net.nl), vh, nullptr);
     QCU_HIP(hipGetLastError());
     QCU_TRY(mhat32(lat, odd(2), odd(1), odd(3), s));
-    // res = Mhat K b - b, unnormalised, then scaled
-    hipLaunchKernelGGL(k_sub_norm, dim3(nb), dim3(bs), 0, s, odd(4), odd(2), odd(0), 1.f, vh, red);
+    // res = Mhat K b - b, with both norms in one pass and one wait
+    double *red = (double *)net.red.p;
+    hipLaunchKernelGGL(k_sub_norms, dim3(nb), dim3(bs), 0, s, odd(4), odd(2), odd(0), vh, red);
     QCU_HIP(hipGetLastError());
-    QCU_HIP(hipMemcpyAsync(h.data(), red, nb * 8, hipMemcpyDeviceToHost, s));
+    std::vector<double> h(2 * (size_t)nb);
+    QCU_HIP(hipMemcpyAsync(h.data(), red, h.size() * 8, hipMemcpyDeviceToHost, s));
     QCU_HIP(hipStreamSynchronize(s));
-    double r2 = 0;
-    for (double x : h) r2 += x;
+    double r2 = 0, b2 = 0;
+    for (unsigned k = 0; k < nb; ++k) {
+      r2 += h[2 * k];
+      b2 += h[2 * k + 1];
+    }
+    if (!(b2 > 0)) {
+      *loss = 0;
+      return 0;
+    }
     *loss = r2 / b2;
     if (!grad) return 0;
     // dL/d(K b) on odd sites = 2 Mhat^dag res / |b|^2 ; zero on even sites
