@@ -44,7 +44,9 @@ QCU_D void zero12(cplx<RT<P>> (&v)[12]) {
 // per-thread view of a batch: segment, local virtual site, system
 struct TCtx {
   const SegDesc *sd;
-  int t, t0, sys, nrhs;
+  int t, t0, sys, nrhs, nthr, pcap;
+  long long voff;
+  double kappa;
   bool valid;   // inside a segment
   bool active;  // valid and its system still running (or no state given)
 };
@@ -55,23 +57,31 @@ QCU_D TCtx tctx(const SegDesc *segs, int nseg, const SysState *st) {
   c.valid = false;
   c.active = false;
   c.sd = nullptr;
+  c.nthr = c.pcap = 0;
+  c.voff = 0;
+  c.kappa = 0;
   c.t0 = bs.t0;
   c.nrhs = 1;
   c.t = 0;
   c.sys = 0;
   if (bs.seg < 0) return c;
+  // values, read before any store (see SegPart)
   c.sd = segs + bs.seg;
   c.nrhs = c.sd->nrhs;
+  c.nthr = c.sd->nthr;
+  c.pcap = c.sd->pcap;
+  c.voff = c.sd->voff;
+  c.kappa = c.sd->kappa;
   c.t = bs.t0 + threadIdx.x;
   c.sys = c.sd->sys0 + c.t % c.nrhs;
-  c.valid = c.t < c.sd->nthr;
+  c.valid = c.t < c.nthr;
   c.active = c.valid && (!st || st[c.sys].done == 0);
   return c;
 }
 
 template <int P>
 QCU_D SpinorPtr view(const SpinorPtr &f, const TCtx &c) {
-  return seg_view(f, P, c.sd->voff, c.sd->nthr);
+  return seg_view(f, P, c.voff, c.nthr);
 }
 
 // ---------------------------------------------------------------- epilogues
@@ -140,7 +150,7 @@ __global__ void __launch_bounds__(256) k_bicg_init(SpinorPtr r, SpinorPtr rt, Sp
     zero12<Px>(zx);
     SpinorIO<Px>::store(view<Px>(x, c), c.t, zx);
   }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // p = r + beta (p - omega v)
@@ -220,7 +230,7 @@ __global__ void __launch_bounds__(256) k_xr_update(SpinorPtr x, SpinorPtr r, Spi
     }
     SpinorIO<P>::store(view<P>(r, c), c.t, ss);
   }
-  block_partial_rhs<3>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<3>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // two-vector reductions: <a, b> with |a|^2 (omega of the preconditioned method)
@@ -243,7 +253,7 @@ __global__ void __launch_bounds__(256) k_dot2(SpinorPtr a_, SpinorPtr b_, const 
                           : (double)b[k].re * b[k].re + (double)b[k].im * b[k].im;
     }
   }
-  block_partial_rhs<3>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<3>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // y = a x + b y (all systems)
@@ -279,7 +289,7 @@ __global__ void __launch_bounds__(256) k_xmy_norm(SpinorPtr b, SpinorPtr r, cons
     }
     SpinorIO<P64>::store(view<P64>(r, c), c.t, rr);
   }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 template <int P>
@@ -293,7 +303,7 @@ __global__ void __launch_bounds__(256) k_norm2(SpinorPtr x, const SegDesc *segs,
 #pragma unroll
     for (int k = 0; k < 12; ++k) acc[0] += (double)xx[k].re * xx[k].re + (double)xx[k].im * xx[k].im;
   }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // out = C (x + a y) in FP64; a = kappa of the segment when a_is_kappa;
@@ -304,7 +314,7 @@ __global__ void __launch_bounds__(256) k_cl_axpy(SpinorPtr out, SpinorPtr x, dou
   if (!c.valid) return;
   cplx<double> xx[12];
   SpinorIO<P64>::load(view<P64>(x, c), c.t, xx);
-  const double aa = a_is_kappa ? c.sd->kappa : a;
+  const double aa = a_is_kappa ? c.kappa : a;
   if (aa != 0.0) {
     cplx<double> yy[12];
     SpinorIO<P64>::load(view<P64>(y, c), c.t, yy);
@@ -345,7 +355,7 @@ __global__ void __launch_bounds__(256) k_residual(SpinorPtr b, SpinorPtr x, Spin
       clover_load_block(A, site, 1, cb);
       clover_apply_block(cb, xx, 1);
     }
-    const double kappa = c.sd->kappa;
+    const double kappa = c.kappa;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
       cplx<double> r = bb[k] - (xx[k] - kappa * tt[k]);
@@ -353,7 +363,7 @@ __global__ void __launch_bounds__(256) k_residual(SpinorPtr b, SpinorPtr x, Spin
       acc[1] += norm2(bb[k]);
     }
   }
-  block_partial_rhs<2>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<2>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // ---------------------------------------------------------------- CG on the normal equations (FP64)
@@ -379,7 +389,7 @@ __global__ void __launch_bounds__(256) k_cg_xr(SpinorPtr x, SpinorPtr r, SpinorP
     SpinorIO<P64>::store(view<P64>(x, c), c.t, xx);
     SpinorIO<P64>::store(view<P64>(r, c), c.t, rr);
   }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // p = z + beta p
@@ -424,7 +434,7 @@ __global__ void __launch_bounds__(256) k_cg_z(SpinorPtr z, SpinorPtr r, SpinorPt
   if (!c.sd) return;
   double acc[1] = {0};
   if (c.active) {
-    const double k2 = c.sd->kappa * c.sd->kappa;
+    const double k2 = c.kappa * c.kappa;
     cplx<double> rr[12], yy[12];
     SpinorIO<P64>::load(view<P64>(r, c), c.t, rr);
     SpinorIO<P64>::load(view<P64>(y, c), c.t, yy);
@@ -436,7 +446,7 @@ __global__ void __launch_bounds__(256) k_cg_z(SpinorPtr z, SpinorPtr r, SpinorPt
     }
     SpinorIO<P64>::store(view<P64>(z, c), c.t, rr);
   }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // |q|^2 per system of the running systems
@@ -450,7 +460,7 @@ __global__ void __launch_bounds__(256) k_cg_norm(SpinorPtr q, const SegDesc *seg
 #pragma unroll
     for (int k = 0; k < 12; ++k) acc[0] += norm2(v[k]);
   }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.sd->pcap);
+  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // ---------------------------------------------------------------- finishing kernel

@@ -52,36 +52,65 @@ constexpr int kSegBlockSizes = 3;
 QCU_HD int seg_block_size(int k) { return 64 << k; }
 
 QCU_D BlockSeg find_seg(const SegDesc *d, int nseg, int blk, int bsz) {
-  BlockSeg r;
-  if (nseg == 1) {
-    r.seg = blk * bsz < d[0].nthr ? 0 : -1;
-    r.t0 = blk * bsz;
-    return r;
-  }
-  r.seg = -1;
-  r.t0 = 0;
-  const int *first = nullptr;
-  for (int k = 0; k < kSegBlockSizes; ++k)
-    if (bsz == seg_block_size(k)) first = (const int *)(d + nseg) + k * (nseg + 1);
-  if (first) {
-    for (int s = 0; s < nseg; ++s)
-      if (blk < first[s + 1]) {
-        r.seg = s;
-        r.t0 = (blk - first[s]) * bsz;
-        return r;
+  int seg = 0, first = 0;
+  if (nseg > 1) {
+    seg = -1;
+    const int table = bsz == 64 ? 0 : (bsz == 128 ? 1 : (bsz == 256 ? 2 : -1));
+    if (table >= 0) {
+      const int *cum = (const int *)(d + nseg) + table * (nseg + 1);
+      for (int s = 0; s < nseg; ++s) {
+        const int next = cum[s + 1];
+        if (blk < next) {
+          seg = s;
+          break;
+        }
+        first = next;
       }
-    return r;
-  }
-  int acc = 0;
-  for (int s = 0; s < nseg; ++s) {
-    const int nb = (d[s].nthr + bsz - 1) / bsz;
-    if (blk < acc + nb) {
-      r.seg = s;
-      r.t0 = (blk - acc) * bsz;
-      return r;
+    } else {
+      for (int s = 0; s < nseg; ++s) {
+        const int next = first + (d[s].nthr + bsz - 1) / bsz;
+        if (blk < next) {
+          seg = s;
+          break;
+        }
+        first = next;
+      }
     }
-    acc += nb;
   }
+  // wavefront-uniform, and said so: what is read through it comes by scalar loads
+  BlockSeg r;
+  r.seg = __builtin_amdgcn_readfirstlane(seg);
+  r.t0 = __builtin_amdgcn_readfirstlane((blk - first) * bsz);
+  if (r.seg >= 0 && r.t0 >= d[r.seg].nthr) r.seg = -1;
+  return r;
+}
+
+// What a kernel of precision P working on output parity p needs of a segment, as
+// values: a SegDesc reached through its pointer would be read again, by vector
+// loads, after every store that might have changed it.
+struct SegPart {
+  Geom g;
+  int nrhs, sys0, nthr, zslab, pcap;
+  long long voff;
+  double kappa;
+  LinkPtr U;
+  CloverPtr Cinv, A;
+};
+template <int P>
+QCU_D SegPart seg_part(const SegDesc *d, int seg, int p) {
+  const SegDesc &s = d[seg];
+  SegPart r;
+  r.g = s.g;
+  r.nrhs = s.nrhs;
+  r.sys0 = s.sys0;
+  r.nthr = s.nthr;
+  r.zslab = s.zslab[P];
+  r.pcap = s.pcap;
+  r.voff = s.voff;
+  r.kappa = s.kappa;
+  r.U = s.U[P];
+  r.Cinv = s.Cinv[P][p];
+  r.A = s.A[p];
   return r;
 }
 

@@ -159,20 +159,26 @@ QCU_D Site ordered_site(const Geom &g, int zslab, int k, int parity, int &i) {
 // kept in scalar registers) plus a 32-bit per-lane byte offset, so that the
 // compiler can use the scalar-base / 32-bit-offset form of global memory
 // instructions instead of a 64-bit address per load and per component.
-// NT: non-temporal, for data a kernel reads once.
+// NT: non-temporal, for data a kernel reads once.  The global address space is
+// stated: the compiler cannot know it of a base that was itself read from memory
+// (a segment's links and clover blocks), and would use flat loads, which return
+// out of order and make every wait a full one.
+#define QCU_GLOBAL __attribute__((address_space(1)))
 template <class V, bool NT = false>
 QCU_D V ld_at(const void *base, size_t comp_bytes, unsigned lane_off) {
-  const char *p = (const char *)base + comp_bytes + lane_off;
-  if (!NT) return *(const V *)p;
   typedef unsigned words __attribute__((ext_vector_type(sizeof(V) / 4)));
-  const words w = __builtin_nontemporal_load((const words *)p);
+  const QCU_GLOBAL words *p = (const QCU_GLOBAL words *)((const QCU_GLOBAL char *)base + comp_bytes + lane_off);
+  const words w = NT ? __builtin_nontemporal_load(p) : *p;
   V v;
   __builtin_memcpy(&v, &w, sizeof(V));
   return v;
 }
 template <class V>
 QCU_D void st_at(void *base, size_t comp_bytes, unsigned lane_off, const V &v) {
-  *(V *)((char *)base + comp_bytes + lane_off) = v;
+  typedef unsigned words __attribute__((ext_vector_type(sizeof(V) / 4)));
+  words w;
+  __builtin_memcpy(&w, &v, sizeof(V));
+  *(QCU_GLOBAL words *)((QCU_GLOBAL char *)base + comp_bytes + lane_off) = w;
 }
 // the same as a non-temporal store: for fields written once and read by a
 // later kernel (the network's activations and term fields), which then need
@@ -336,14 +342,19 @@ struct LinkIO;
 
 template <>
 struct LinkIO<P64> {
+  // rows 0 and 1 only
   template <bool NT = false>
-  static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<double> (&u)[9]) {
+  static QCU_D void rows(const LinkPtr &L, int pm, int i, cplx<double> (&u)[9]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
       double2 a = ld_at<double2, NT>(L.a, ((size_t)pm * 6 + k) * L.vh * 16, off);
       u[k] = mk(a.x, a.y);
     }
+  }
+  template <bool NT = false>
+  static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<double> (&u)[9]) {
+    rows<NT>(L, pm, i, u);
     recon_row2(u);
   }
 };
@@ -351,7 +362,7 @@ struct LinkIO<P64> {
 template <>
 struct LinkIO<P32> {
   template <bool NT = false>
-  static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<float> (&u)[9]) {
+  static QCU_D void rows(const LinkPtr &L, int pm, int i, cplx<float> (&u)[9]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -359,6 +370,10 @@ struct LinkIO<P32> {
       u[2 * k] = mk(a.x, a.y);
       u[2 * k + 1] = mk(a.z, a.w);
     }
+  }
+  template <bool NT = false>
+  static QCU_D void load(const LinkPtr &L, int pm, int i, cplx<float> (&u)[9]) {
+    rows<NT>(L, pm, i, u);
     recon_row2(u);
   }
 };

@@ -145,6 +145,12 @@ enum HopRed { RED_NONE = 0, RED_DOT_Y_OUT = 1, RED_OUT_X = 2 };
 int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, int epi, SpinorPtr x, int red,
         SpinorPtr y, SysState *st, double *partials, const LaunchCfg &cfg, hipStream_t s, bool use_clover = true);
 
+// whether hop() takes the kernel with eight waves per 64 sites
+bool hop_is_split(const BatchOp &op, const LaunchCfg &cfg);
+// that kernel's second half of the Schur operator (out = x - kappa^2 A^-1 D in on the
+// odd sites) with its block partials (RED_DOT_Y_OUT: 2 values, RED_OUT_X: 3), not finished
+int hop_split_red(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, SpinorPtr x, int red, SpinorPtr y,
+                  SysState *st, double *partials, hipStream_t s);
 // the FP64 hop on the caller's fields of a single lattice, which must not overlap:
 // out = [A_p^-1] D_{p,1-p} in on one-parity fields, or (mat) out = A in - kappa D in
 // on full ones
@@ -197,6 +203,15 @@ int residual_parity(const BatchOp &op, SpinorPtr b, SpinorPtr x, SpinorPtr t, in
 // gen.hip
 int gen_gauge(void *ext, const Geom &g, double eps, uint64_t seed, hipStream_t s);
 int gen_gauss(void *ext, long n_complex, uint64_t seed, hipStream_t s);
+
+// iterate.hip: n BiCGSTAB iterations of small batches in five launches each
+struct SplitIter {
+  SpinorPtr p[2];      // p[0] holds p before and (n even) after the iterations
+  SpinorPtr r, rt, v, s, t, tmp, x;
+  SysState *st[2];     // st[0]: the solver's states; st[1]: scratch
+  double *part[2];     // block partials, (max_blocks(64) + 1) * kMaxRhs * 3 doubles each
+};
+int split_iterations(const BatchOp &op, int prec, const SplitIter &v, int n, hipStream_t s);
 
 // CG on the normal equations (FP64, per-system device scalars)
 int cg_xr(const BatchOp &op, SpinorPtr x, SpinorPtr r, SpinorPtr p, SpinorPtr q, SysState *st, double *partials,

@@ -14,10 +14,28 @@ namespace qcu {
 
 constexpr int kMaxWaves = 16;  // up to 1024 threads per block
 
+template <int CTRL>
+QCU_D double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+QCU_D double lane_value(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Sum over the 64 lanes, in every lane; all lanes must be active.  Within a row
+// of 16 lanes the partner comes by DPP (1 and 2 lanes away by quad permutes; the
+// mirrors of 8 and 16 lanes reach the other half, whose lanes all hold its sum),
+// the four rows by lane reads: the tree of a butterfly of exchanges, whose six
+// LDS round trips took 0.4 us.
 QCU_D double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
-  return v;
+  v += dpp_move<0xB1>(v);   // quad_perm 1,0,3,2
+  v += dpp_move<0x4E>(v);   // quad_perm 2,3,0,1
+  v += dpp_move<0x141>(v);  // row_half_mirror
+  v += dpp_move<0x140>(v);  // row_mirror
+  return (lane_value(v, 0) + lane_value(v, 16)) + (lane_value(v, 32) + lane_value(v, 48));
 }
 
 // Sums v over the block and stores it as partials[slot * NR + k].  Must be

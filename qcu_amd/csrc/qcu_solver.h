@@ -27,6 +27,8 @@ struct Precond {
 struct VecSet {
   int prec = P64, px = P64;
   Spinor r, rt, p, v, s, t, tmp, x, ph, sh;
+  Spinor p2;         // small batches (iterate.hip), made on first use: the other p,
+  DevBuf split_buf;  // the other states and two sets of block partials
   std::map<long, hipGraphExec_t> graphs;
   unsigned long long graph_net = 0;  // uid of the preconditioner the graphs were captured with
   unsigned long long graph_tune = 0; // tune_generation() when the graphs were captured

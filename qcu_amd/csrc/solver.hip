@@ -160,11 +160,45 @@ static int enqueue_iteration(Solver &S, VecSet &V, Precond *K) {
   return 0;
 }
 
-static int run_chunk(Solver &S, VecSet &V, Precond *K, int chunk, bool use_graph) {
-  if (!use_graph) {
-    for (int k = 0; k < chunk; ++k) QCU_TRY(enqueue_iteration(S, V, K));
+// `n` iterations: small batches without a preconditioner in five launches each
+// (FP64, FP32; an even number, since p changes places with every iteration)
+static bool split_chunk(const Solver &S, const VecSet &V, const Precond *K, int n) {
+  return !K && V.prec != P16 && V.px == V.prec && n % 2 == 0 && hop_is_split(*S.op, tuned_cfg(*S.op, V.prec));
+}
+
+static int prepare_split(Solver &S, VecSet &V) {
+  QCU_TRY(V.p2.create(V.prec, S.n));
+  const size_t part = (size_t)(S.op->max_blocks(64) + 1) * kMaxRhs * 3 * sizeof(double);
+  return V.split_buf.alloc(2 * part + S.nsys * sizeof(SysState));
+}
+
+static int enqueue_chunk(Solver &S, VecSet &V, Precond *K, int n) {
+  if (!split_chunk(S, V, K, n)) {
+    for (int k = 0; k < n; ++k) QCU_TRY(enqueue_iteration(S, V, K));
     return 0;
   }
+  const size_t part = (size_t)(S.op->max_blocks(64) + 1) * kMaxRhs * 3;
+  double *buf = (double *)V.split_buf.p;
+  SplitIter it;
+  it.p[0] = V.p.ptr();
+  it.p[1] = V.p2.ptr();
+  it.r = V.r.ptr();
+  it.rt = V.rt.ptr();
+  it.v = V.v.ptr();
+  it.s = V.s.ptr();
+  it.t = V.t.ptr();
+  it.tmp = V.tmp.ptr();
+  it.x = V.x.ptr();
+  it.st[0] = S.st;
+  it.st[1] = (SysState *)(buf + 2 * part);
+  it.part[0] = buf;
+  it.part[1] = buf + part;
+  return split_iterations(*S.op, V.prec, it, n, S.stream);
+}
+
+static int run_chunk(Solver &S, VecSet &V, Precond *K, int chunk, bool use_graph) {
+  if (split_chunk(S, V, K, chunk)) QCU_TRY(prepare_split(S, V));
+  if (!use_graph) return enqueue_chunk(S, V, K, chunk);
   if (V.graph_tune != tune_generation()) {
     // the graphs hold the launch shapes of their capture: a newly tuned (or
     // set) shape needs new graphs
@@ -189,8 +223,7 @@ static int run_chunk(Solver &S, VecSet &V, Precond *K, int chunk, bool use_graph
   if (it == V.graphs.end()) {
     hipGraph_t graph;
     QCU_HIP(hipStreamBeginCapture(S.stream, hipStreamCaptureModeThreadLocal));
-    int rc = 0;
-    for (int k = 0; k < chunk && !rc; ++k) rc = enqueue_iteration(S, V, K);
+    const int rc = enqueue_chunk(S, V, K, chunk);
     hipError_t e = hipStreamEndCapture(S.stream, &graph);
     if (rc) return rc;
     QCU_HIP(e);
