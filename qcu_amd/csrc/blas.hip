@@ -105,16 +105,13 @@ QCU_D void fin_init(SysState *st, double rr) {
 }
 
 // after a reliable update replaced r by the recomputed residual:
-// rho = <r~, r>, beta = (rho / rho_prev) (alpha / omega), rr_ref = |r|^2
+// rho = <r~, r>, beta = (rho / rho_prev) (alpha / omega), rr_ref = |r|^2 (whether
+// the system goes on is the host's decision)
 QCU_D void fin_reliable(SysState *st, double rre, double rim, double rr) {
   st->rho[0] = rre;
   st->rho[1] = rim;
   st->rr = rr;
   st->rr_ref = rr;
-  if (!isfinite(rr)) {
-    st->done = 2;
-    return;
-  }
   double q1[2], q2[2];
   cdiv(st->rho, st->rho_prev, q1);
   cdiv(st->alpha, st->omega, q2);
@@ -123,7 +120,6 @@ QCU_D void fin_reliable(SysState *st, double rre, double rim, double rr) {
     st->beta[0] = 0;  // restart the search direction
     st->beta[1] = 0;
   }
-  st->done = (rr < st->rr_stop) ? 1 : 0;
 }
 
 // ---------------------------------------------------------------- kernels
@@ -273,6 +269,48 @@ __global__ void __launch_bounds__(256) k_axpby(double a, SpinorPtr x, double b, 
   SpinorIO<Py>::store(view<Py>(y, c), c.t, yy);
 }
 
+// y += x (FP64), x = 0: a reliable update takes the correction into the solution
+template <int Px>
+__global__ void __launch_bounds__(256) k_fold(SpinorPtr x, SpinorPtr y, const SegDesc *segs, int nseg) {
+  const TCtx c = tctx(segs, nseg, nullptr);
+  if (!c.valid) return;
+  cplx<RT<Px>> xx[12];
+  cplx<double> yy[12];
+  SpinorIO<Px>::load(view<Px>(x, c), c.t, xx);
+  SpinorIO<P64>::load(view<P64>(y, c), c.t, yy);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) yy[k] = mk(yy[k].re + (double)xx[k].re, yy[k].im + (double)xx[k].im);
+  SpinorIO<P64>::store(view<P64>(y, c), c.t, yy);
+  zero12<Px>(xx);
+  SpinorIO<Px>::store(view<Px>(x, c), c.t, xx);
+}
+
+// r = the FP64 residual in the solver's precision, <r~, r> and |r|^2 of the stored
+// r per system
+template <int P>
+__global__ void __launch_bounds__(256) k_reliable(SpinorPtr r, SpinorPtr rt, SpinorPtr r64, const SegDesc *segs, int nseg,
+                           double *partials) {
+  const TCtx c = tctx(segs, nseg, nullptr);
+  if (!c.sd) return;
+  double acc[3] = {0, 0, 0};
+  if (c.valid) {
+    cplx<double> s[12];
+    SpinorIO<P64>::load(view<P64>(r64, c), c.t, s);
+    cplx<RT<P>> b[12], a[12];
+    cvt<P, P64>(s, b);
+    SpinorIO<P>::store(view<P>(r, c), c.t, b);
+    if constexpr (P == P16) SpinorIO<P16>::round(b);
+    SpinorIO<P>::load(view<P>(rt, c), c.t, a);
+#pragma unroll
+    for (int k = 0; k < 12; ++k) {
+      acc[0] += (double)a[k].re * b[k].re + (double)a[k].im * b[k].im;
+      acc[1] += (double)a[k].re * b[k].im - (double)a[k].im * b[k].re;
+      acc[2] += (double)b[k].re * b[k].re + (double)b[k].im * b[k].im;
+    }
+  }
+  block_partial_rhs<3>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
+}
+
 // r = b - r (FP64), |r|^2 per system
 __global__ void __launch_bounds__(256) k_xmy_norm(SpinorPtr b, SpinorPtr r, const SegDesc *segs, int nseg, double *partials) {
   const TCtx c = tctx(segs, nseg, nullptr);
@@ -292,47 +330,43 @@ __global__ void __launch_bounds__(256) k_xmy_norm(SpinorPtr b, SpinorPtr r, cons
   block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
-template <int P>
-__global__ void __launch_bounds__(256) k_norm2(SpinorPtr x, const SegDesc *segs, int nseg, double *partials) {
+// out = C (x + a y) in FP64; a = kappa of the segment when a_is_kappa;
+// which: 0 identity, 1 inverse clover of the parity, 2 clover of the parity;
+// NORM: |x|^2 per system as well
+template <int NORM>
+__global__ void __launch_bounds__(256) k_cl_axpy(SpinorPtr out, SpinorPtr x, double a, int a_is_kappa, SpinorPtr y, int which, int parity,
+                          const SegDesc *segs, int nseg, double *partials) {
   const TCtx c = tctx(segs, nseg, nullptr);
-  if (!c.sd) return;
+  if (NORM ? !c.sd : !c.valid) return;
   double acc[1] = {0};
   if (c.valid) {
-    cplx<RT<P>> xx[12];
-    SpinorIO<P>::load(view<P>(x, c), c.t, xx);
+    cplx<double> xx[12];
+    SpinorIO<P64>::load(view<P64>(x, c), c.t, xx);
+    if (NORM) {
 #pragma unroll
-    for (int k = 0; k < 12; ++k) acc[0] += (double)xx[k].re * xx[k].re + (double)xx[k].im * xx[k].im;
-  }
-  block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
-}
-
-// out = C (x + a y) in FP64; a = kappa of the segment when a_is_kappa;
-// which: 0 identity, 1 inverse clover of the parity, 2 clover of the parity
-__global__ void __launch_bounds__(256) k_cl_axpy(SpinorPtr out, SpinorPtr x, double a, int a_is_kappa, SpinorPtr y, int which, int parity,
-                          const SegDesc *segs, int nseg) {
-  const TCtx c = tctx(segs, nseg, nullptr);
-  if (!c.valid) return;
-  cplx<double> xx[12];
-  SpinorIO<P64>::load(view<P64>(x, c), c.t, xx);
-  const double aa = a_is_kappa ? c.kappa : a;
-  if (aa != 0.0) {
-    cplx<double> yy[12];
-    SpinorIO<P64>::load(view<P64>(y, c), c.t, yy);
+      for (int k = 0; k < 12; ++k) acc[0] += norm2(xx[k]);
+    }
+    const double aa = a_is_kappa ? c.kappa : a;
+    if (aa != 0.0) {
+      cplx<double> yy[12];
+      SpinorIO<P64>::load(view<P64>(y, c), c.t, yy);
 #pragma unroll
-    for (int k = 0; k < 12; ++k) xx[k] = xx[k] + aa * yy[k];
+      for (int k = 0; k < 12; ++k) xx[k] = xx[k] + aa * yy[k];
+    }
+    CloverPtr C{};
+    if (which == 1) C = c.sd->Cinv[P64][parity];
+    if (which == 2) C = c.sd->A[parity];
+    if (C.p) {
+      const int site = c.t / c.nrhs;
+      double cb[36];
+      clover_load_block(C, site, 0, cb);
+      clover_apply_block(cb, xx, 0);
+      clover_load_block(C, site, 1, cb);
+      clover_apply_block(cb, xx, 1);
+    }
+    SpinorIO<P64>::store(view<P64>(out, c), c.t, xx);
   }
-  CloverPtr C{};
-  if (which == 1) C = c.sd->Cinv[P64][parity];
-  if (which == 2) C = c.sd->A[parity];
-  if (C.p) {
-    const int site = c.t / c.nrhs;
-    double cb[36];
-    clover_load_block(C, site, 0, cb);
-    clover_apply_block(cb, xx, 0);
-    clover_load_block(C, site, 1, cb);
-    clover_apply_block(cb, xx, 1);
-  }
-  SpinorIO<P64>::store(view<P64>(out, c), c.t, xx);
+  if (NORM) block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
 // |b - (A x - kappa t)|^2 and |b|^2 per system on one parity
@@ -483,8 +517,7 @@ __global__ void __launch_bounds__(1024) k_finish(const double *partials, const S
     acc_b += n;
   }
   if (seg < 0) return;
-  if (st && (kind == FK_ALPHA || kind == FK_OMEGA || kind == FK_RHO || kind == FK_RELIABLE || kind == FK_CG_ALPHA ||
-             kind == FK_CG_RHO) &&
+  if (st && (kind == FK_ALPHA || kind == FK_OMEGA || kind == FK_RHO || kind == FK_CG_ALPHA || kind == FK_CG_RHO) &&
       st[sys].done)
     return;
   // this system's partials are contiguous: slots r * pcap + blk0 .. + nb - 1;
@@ -654,9 +687,27 @@ int omega_dot(const BatchOp &op, SpinorPtr t, SpinorPtr s_, int prec, SysState *
   return dot2<1>(op, t, s_, prec, st, partials, FK_OMEGA, s);
 }
 
-int reliable_dot(const BatchOp &op, SpinorPtr rt, SpinorPtr r, int prec, SysState *st, double *partials,
-                 hipStream_t s) {
-  return dot2<0>(op, rt, r, prec, st, partials, FK_RELIABLE, s);
+int fold(const BatchOp &op, SpinorPtr x, int px, SpinorPtr y, hipStream_t s) {
+  const int bs = 256, nb = batch_blocks(op, bs);
+  QCU_CHECK(px == P64 || px == P32, QCU_ERR_ARG, "fold: bad precision");
+  if (px == P64)
+    hipLaunchKernelGGL(k_fold<P64>, dim3(nb), dim3(bs), 0, s, x, y, QCU_SEGS);
+  else
+    hipLaunchKernelGGL(k_fold<P32>, dim3(nb), dim3(bs), 0, s, x, y, QCU_SEGS);
+  QCU_HIP(hipGetLastError());
+  return 0;
+}
+
+int reliable_residual(const BatchOp &op, SpinorPtr r, SpinorPtr rt, SpinorPtr r64, int prec, SysState *st,
+                      double *partials, hipStream_t s) {
+  const int bs = 256, nb = batch_blocks(op, bs);
+  switch (prec) {
+    case P64: hipLaunchKernelGGL(k_reliable<P64>, dim3(nb), dim3(bs), 0, s, r, rt, r64, QCU_SEGS, partials); break;
+    case P32: hipLaunchKernelGGL(k_reliable<P32>, dim3(nb), dim3(bs), 0, s, r, rt, r64, QCU_SEGS, partials); break;
+    default: hipLaunchKernelGGL(k_reliable<P16>, dim3(nb), dim3(bs), 0, s, r, rt, r64, QCU_SEGS, partials); break;
+  }
+  QCU_HIP(hipGetLastError());
+  return finish(op, partials, bs, 3, FK_RELIABLE, st, nullptr, s);
 }
 
 int axpby(const BatchOp &op, double a, SpinorPtr x, int px, double b, SpinorPtr y, int py, hipStream_t s) {
@@ -695,23 +746,19 @@ int xmy_norm(const BatchOp &op, SpinorPtr b, SpinorPtr r, SysState *st, double *
   return finish(op, partials, bs, 1, store ? FK_STORE_TMP : FK_NONE, st, nullptr, s);
 }
 
-int norm2_dev(const BatchOp &op, SpinorPtr x, int px, double *out_dev, double *partials, hipStream_t s) {
-  const int bs = 256, nb = batch_blocks(op, bs);
-  switch (px) {
-    case P64: hipLaunchKernelGGL(k_norm2<P64>, dim3(nb), dim3(bs), 0, s, x, QCU_SEGS, partials); break;
-    case P32: hipLaunchKernelGGL(k_norm2<P32>, dim3(nb), dim3(bs), 0, s, x, QCU_SEGS, partials); break;
-    default: hipLaunchKernelGGL(k_norm2<P16>, dim3(nb), dim3(bs), 0, s, x, QCU_SEGS, partials); break;
-  }
-  QCU_HIP(hipGetLastError());
-  return finish(op, partials, bs, 1, FK_STORE, nullptr, out_dev, s);
-}
-
 int cl_axpy(const BatchOp &op, SpinorPtr out, SpinorPtr x, double a, bool a_is_kappa, SpinorPtr y, int which,
-            int parity, hipStream_t s) {
+            int parity, hipStream_t s, double *norm, double *partials) {
   const int bs = 256, nb = batch_blocks(op, bs);
-  hipLaunchKernelGGL(k_cl_axpy, dim3(nb), dim3(bs), 0, s, out, x, a, (int)a_is_kappa, y, which, parity, QCU_SEGS);
+  if (!norm) {
+    hipLaunchKernelGGL(k_cl_axpy<0>, dim3(nb), dim3(bs), 0, s, out, x, a, (int)a_is_kappa, y, which, parity, QCU_SEGS,
+                       partials);
+    QCU_HIP(hipGetLastError());
+    return 0;
+  }
+  hipLaunchKernelGGL(k_cl_axpy<1>, dim3(nb), dim3(bs), 0, s, out, x, a, (int)a_is_kappa, y, which, parity, QCU_SEGS,
+                     partials);
   QCU_HIP(hipGetLastError());
-  return 0;
+  return finish(op, partials, bs, 1, FK_STORE, nullptr, norm, s);
 }
 
 int cg_xr(const BatchOp &op, SpinorPtr x, SpinorPtr r, SpinorPtr p, SpinorPtr q, SysState *st, double *partials,
@@ -752,11 +799,11 @@ int cg_qnorm(const BatchOp &op, SpinorPtr q, SysState *st, double *partials, hip
 }
 
 int residual_parity(const BatchOp &op, SpinorPtr b, SpinorPtr x, SpinorPtr t, int parity, double *partials,
-                    double *out, hipStream_t s) {
+                    double *out, bool add, hipStream_t s) {
   const int bs = 256, nb = batch_blocks(op, bs);
   hipLaunchKernelGGL(k_residual, dim3(nb), dim3(bs), 0, s, b, x, t, parity, QCU_SEGS, partials);
   QCU_HIP(hipGetLastError());
-  return finish(op, partials, bs, 2, FK_ACCUM, nullptr, out, s);
+  return finish(op, partials, bs, 2, add ? FK_ACCUM : FK_STORE, nullptr, out, s);
 }
 
 #undef QCU_SEGS

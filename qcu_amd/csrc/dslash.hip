@@ -162,6 +162,15 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
         }
       }
     }
+    if (RED == RED_RES) {
+      cplx<T> y[12];
+      SpinorIO<P>::load(seg_view(a.y, P, sd.voff, sd.nthr), t, y);
+#pragma unroll
+      for (int k = 0; k < 12; ++k) {
+        d[k] = y[k] - d[k];
+        red[0] += (double)norm2(d[k]);
+      }
+    }
     if (RED == RED_DOT_Y_OUT) {
       cplx<T> y[12];
       SpinorIO<P>::load(seg_view(a.y, P, sd.voff, sd.nthr), t, y);
@@ -178,6 +187,9 @@ __global__ void __launch_bounds__(256) k_hop(HopKArgs a) {
     block_partial_rhs<2>(v, a.partials, blk, bs.t0, nrhs, sd.pcap);
   } else if (RED == RED_OUT_X) {
     block_partial_rhs<3>(red, a.partials, blk, bs.t0, nrhs, sd.pcap);
+  } else if (RED == RED_RES) {
+    double v[1] = {red[0]};
+    block_partial_rhs<1>(v, a.partials, blk, bs.t0, nrhs, sd.pcap);
   }
 }
 
@@ -245,7 +257,7 @@ __global__ void __launch_bounds__(8 * kSplitSites) k_hop_split(HopKArgs a) {
     if (CLOVER) cr.load(EPI == EPI_MAT ? sd.A : sd.Cinv, i, cb, cj);
     if (EPI == EPI_MAT) load_pair<P, IO>(hop_field<P, IO, EPI>(a.in, sd, p), t, w, x);
     if (EPI == EPI_XPAY) load_pair<P, IO_INT>(seg_view(a.x, P, sd.voff, sd.nthr), t, w, x);
-    if (RED == RED_DOT_Y_OUT) load_pair<P, IO_INT>(seg_view(a.y, P, sd.voff, sd.nthr), t, w, y);
+    if (RED == RED_DOT_Y_OUT || RED == RED_RES) load_pair<P, IO_INT>(seg_view(a.y, P, sd.voff, sd.nthr), t, w, y);
   }
   __syncthreads();
   if (mine) {
@@ -291,6 +303,13 @@ __global__ void __launch_bounds__(8 * kSplitSites) k_hop_split(HopKArgs a) {
         }
       }
     }
+    if (RED == RED_RES) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        d[q] = y[q] - d[q];
+        red[0] += (double)norm2(d[q]);
+      }
+    }
     if (RED == RED_DOT_Y_OUT) {
 #pragma unroll
       for (int q = 0; q < 2; ++q) {
@@ -312,7 +331,7 @@ __global__ void __launch_bounds__(8 * kSplitSites) k_hop_split(HopKArgs a) {
   if (mine) store_pair<P, IO>(hop_field<P, IO, EPI>(a.out, sd, p), t, w, d, m);
   if (RED != RED_NONE) {
     // the six waves' sums per site, added in order, then the sites of each system
-    constexpr int NR = RED == RED_DOT_Y_OUT ? 2 : 3;
+    constexpr int NR = RED == RED_RES ? 1 : (RED == RED_DOT_Y_OUT ? 2 : 3);
     __shared__ double sh[NR][6][kSplitSites];
     if (w < 6) {
 #pragma unroll
@@ -362,6 +381,11 @@ static int dispatch(const HopKArgs &a, int nb, int clover, int epi, int red, boo
   if (red == RED_NONE)
     return clover ? launch<P, I, 1, EPI_XPAY, RED_NONE>(a, nb, split, nt, cfg, s)
                   : launch<P, I, 0, EPI_XPAY, RED_NONE>(a, nb, split, nt, cfg, s);
+  if constexpr (P == P64) {
+    if (red == RED_RES)
+      return clover ? launch<P, I, 1, EPI_XPAY, RED_RES>(a, nb, split, nt, cfg, s)
+                    : launch<P, I, 0, EPI_XPAY, RED_RES>(a, nb, split, nt, cfg, s);
+  }
   if (red == RED_DOT_Y_OUT)
     return clover ? launch<P, I, 1, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, nt, cfg, s)
                   : launch<P, I, 0, EPI_XPAY, RED_DOT_Y_OUT>(a, nb, split, nt, cfg, s);
@@ -444,6 +468,7 @@ int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, in
   QCU_TRY(check_cfg(cfg));
   QCU_CHECK(red == RED_NONE || (epi == EPI_XPAY && st && partials), QCU_ERR_ARG,
             "fused reductions need the xpay epilogue and solver state");
+  QCU_CHECK(red != RED_RES || prec == P64, QCU_ERR_ARG, "residuals are formed in FP64");
   HopKArgs a;
   a.out = out;
   a.in = in;
@@ -453,7 +478,7 @@ int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, in
   a.nseg = (int)op.segs.size();
   a.parity = parity;
   a.remap = cfg.remap;
-  a.st = st;
+  a.st = red == RED_RES ? nullptr : st;  // residuals of every system, stopped or not
   a.partials = partials;
   const int clover = use_clover && op.has_clover;
   const bool split = hop_is_split(op, cfg), nt = use_nt(op, prec, clover);
@@ -466,6 +491,7 @@ int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, in
     default: rc = dispatch<P16>(a, nb, clover, epi, red, split, nt, cfg, s); break;
   }
   if (rc || red == RED_NONE) return rc;
+  if (red == RED_RES) return finish(op, partials, bsz, 1, FK_STORE_TMP, st, nullptr, s);
   return red == RED_DOT_Y_OUT ? finish(op, partials, bsz, 2, FK_ALPHA, st, nullptr, s)
                               : finish(op, partials, bsz, 3, FK_OMEGA, st, nullptr, s);
 }

@@ -276,6 +276,15 @@ struct SpinorIO<P16> {
     }
     return ld_at<float>(f.norm, 0, (unsigned)i * 4u);
   }
+  // v as load() gives it back after store()
+  static QCU_D void round(cplx<float> (&v)[12]) {
+    float m = 0.f;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) m = fmaxf(m, fmaxf(fabsf(v[k].re), fabsf(v[k].im)));
+    const float inv = m > 0.f ? 1.0f / m : 0.f;
+#pragma unroll
+    for (int k = 0; k < 12; ++k) v[k] = mk(m * h2f(f2h(v[k].re * inv)), m * h2f(f2h(v[k].im * inv)));
+  }
   static QCU_D void load(const SpinorPtr &f, int i, cplx<float> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
     const float nrm = ld_at<float>(f.norm, 0, (unsigned)i * 4u);

@@ -135,13 +135,17 @@ size_t gauge_hash_scratch_bytes();
 int spinor_ext_to_batch(const void *ext, const BatchOp &op, int seg, int rhs, SpinorPtr dst, int prec,
                         hipStream_t s);
 int spinor_batch_to_ext(SpinorPtr src, const BatchOp &op, int seg, int rhs, void *ext, int prec, hipStream_t s);
+// external full-lattice fields ext[k] of every system k <-> FP64 batch vectors of both parities
+int systems_to_batch(const void *const *ext, const BatchOp &op, SpinorPtr even, SpinorPtr odd, hipStream_t s);
+int batch_to_systems(SpinorPtr even, SpinorPtr odd, const BatchOp &op, void *const *ext, hipStream_t s);
 
 // dslash.hip
 enum HopEpi { EPI_PLAIN = 0, EPI_XPAY = 1, EPI_MAT = 2 };
-enum HopRed { RED_NONE = 0, RED_DOT_Y_OUT = 1, RED_OUT_X = 2 };
+enum HopRed { RED_NONE = 0, RED_DOT_Y_OUT = 1, RED_OUT_X = 2, RED_RES = 3 };
 // out = [A_p^-1] D_{p,1-p} in                                  (EPI_PLAIN)
 // out = x - kappa^2 [A_p^-1] D_{p,1-p} in                      (EPI_XPAY)
-// RED_DOT_Y_OUT: <y,out> -> alpha update; RED_OUT_X: <out,x>,|out|^2 -> omega
+// RED_DOT_Y_OUT: <y,out> -> alpha update; RED_OUT_X: <out,x>,|out|^2 -> omega;
+// RED_RES (FP64, all systems): out = y - (x - kappa^2 ...), |out|^2 -> st->tmp[0]
 int hop(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, int parity, int epi, SpinorPtr x, int red,
         SpinorPtr y, SysState *st, double *partials, const LaunchCfg &cfg, hipStream_t s, bool use_clover = true);
 
@@ -182,23 +186,25 @@ int bicg_xr_update(const BatchOp &op, SpinorPtr x, int px, SpinorPtr r, SpinorPt
 int bicg_xr_update_pc(const BatchOp &op, SpinorPtr x, int px, SpinorPtr r, SpinorPtr rt, SpinorPtr ph, SpinorPtr sh,
                       SpinorPtr s_, SpinorPtr t, int prec, SysState *st, double *partials, hipStream_t s);
 int omega_dot(const BatchOp &op, SpinorPtr t, SpinorPtr s_, int prec, SysState *st, double *partials, hipStream_t s);
-int reliable_dot(const BatchOp &op, SpinorPtr rt, SpinorPtr r, int prec, SysState *st, double *partials,
-                 hipStream_t s);
+// y += x (y FP64), x = 0
+int fold(const BatchOp &op, SpinorPtr x, int px, SpinorPtr y, hipStream_t s);
+// r = r64 in the solver's precision, then rho, beta, rr and rr_ref of every system
+int reliable_residual(const BatchOp &op, SpinorPtr r, SpinorPtr rt, SpinorPtr r64, int prec, SysState *st,
+                      double *partials, hipStream_t s);
 // y = a*x + b*y  (real a, b; mixed precisions allowed)
 int axpby(const BatchOp &op, double a, SpinorPtr x, int px, double b, SpinorPtr y, int py, hipStream_t s);
 int spinor_convert(const BatchOp &op, SpinorPtr dst, int pdst, SpinorPtr src, int psrc, hipStream_t s);
 int zero_spinor(const BatchOp &op, SpinorPtr x, int px, hipStream_t s);
 // r = b - r (FP64); store: |r|^2 of system k into st[k].tmp[0]
 int xmy_norm(const BatchOp &op, SpinorPtr b, SpinorPtr r, SysState *st, double *partials, int store, hipStream_t s);
-// out_dev[k] = |x_k|^2
-int norm2_dev(const BatchOp &op, SpinorPtr x, int px, double *out_dev, double *partials, hipStream_t s);
 // out = C (x + a y) in FP64 (a = kappa of each segment when a_is_kappa);
-// which: 0 identity, 1 inverse clover, 2 clover of the parity
+// which: 0 identity, 1 inverse clover, 2 clover of the parity; norm (with
+// partials): |x|^2 of every system as well
 int cl_axpy(const BatchOp &op, SpinorPtr out, SpinorPtr x, double a, bool a_is_kappa, SpinorPtr y, int which,
-            int parity, hipStream_t s);
-// out[2k] += |b - (A x - kappa t)|^2, out[2k+1] += |b|^2 of system k, one parity
+            int parity, hipStream_t s, double *norm = nullptr, double *partials = nullptr);
+// out[2k] = |b - (A x - kappa t)|^2, out[2k+1] = |b|^2 of system k, one parity (add: +=)
 int residual_parity(const BatchOp &op, SpinorPtr b, SpinorPtr x, SpinorPtr t, int parity, double *partials,
-                    double *out, hipStream_t s);
+                    double *out, bool add, hipStream_t s);
 
 // gen.hip
 int gen_gauge(void *ext, const Geom &g, double eps, uint64_t seed, hipStream_t s);

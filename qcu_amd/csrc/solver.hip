@@ -248,12 +248,51 @@ static int write_states(Solver &S) {
   return 0;
 }
 
+// How many iterations until a running system needs the host: from the mean
+// decrease of its residual per iteration so far.  Iterations launched beyond that
+// only run kernels that return at once, but each costs its launches (60 us at
+// 32^3x64, where a reliable update every 3 or 4 iterations would waste as many).
+struct Pace {
+  std::vector<double> lrr, rate;  // log |r|^2 when last seen, its decrease per iteration (0: unknown)
+  std::vector<int> iter;
+  Pace(const SysState *hs, int nsys) : lrr(nsys), rate(nsys, 0.0), iter(nsys) { restarted(hs, nsys); }
+  void restarted(const SysState *hs, int nsys) {
+    for (int k = 0; k < nsys; ++k) {
+      lrr[k] = std::log(hs[k].rr);
+      iter[k] = hs[k].iter;
+    }
+  }
+  void seen(const SysState *hs, int nsys) {
+    for (int k = 0; k < nsys; ++k) {
+      const int n = hs[k].iter - iter[k];
+      if (n <= 0) continue;
+      const double l = std::log(hs[k].rr);
+      rate[k] = (lrr[k] - l) / n;
+      lrr[k] = l;
+      iter[k] = hs[k].iter;
+    }
+  }
+  int next(const SysState *hs, int nsys, int chunk, bool pairs) const {
+    int n = 1;
+    for (int k = 0; k < nsys; ++k) {
+      if (hs[k].done != 0) continue;
+      const double target = std::max(hs[k].rr_stop, hs[k].delta2 * hs[k].rr_ref);
+      const double need = (std::log(hs[k].rr) - std::log(target)) / rate[k];
+      // unknown, or no decrease: half a chunk where updates are expected, else all of it
+      int m = hs[k].delta2 > 0 ? (chunk + 1) / 2 : chunk;
+      if (rate[k] > 0 && std::isfinite(need)) m = need >= chunk ? chunk : (need > 1 ? (int)std::ceil(need) : 1);
+      n = std::max(n, m);
+    }
+    return pairs ? (n + 1) & ~1 : n;
+  }
+};
+
 // Solve Mhat x_o = bhat (bhat in S.bh) for the systems with active[k]; the
 // solution accumulates in S.xo (FP64): the iterated correction V.x is folded
 // into it at every reliable update.  warm: start from the current S.xo.
 // A system stops when |bhat - Mhat x_o|^2 < target2[k] (recomputed in FP64).
 static int schur_solve(Solver &S, int prec, const std::vector<double> &target2, double delta, int max_iter,
-                       int chunk, bool use_graph, Precond *K, bool warm, const std::vector<int> &active,
+                       int chunk, bool adaptive, bool use_graph, Precond *K, bool warm, const std::vector<int> &active,
                        std::vector<SolveStats> &stats) {
   const BatchOp &op = *S.op;
   const int nsys = S.nsys;
@@ -284,7 +323,10 @@ static int schur_solve(Solver &S, int prec, const std::vector<double> &target2, 
   trace.mark("  init");
   std::vector<int> stuck(nsys, 0);
   for (int k = 0; k < nsys; ++k) stats[k] = SolveStats{0, 0, 0, 0};
+  Pace pace(hs, nsys);
+  const bool pairs = split_chunk(S, *V, K, 2);  // iterations come in pairs
   int iters = 0;
+  bool folded = false;  // V.x is zero
   for (;;) {
     bool running = false, pending = false;
     for (int k = 0; k < nsys; ++k) {
@@ -293,25 +335,34 @@ static int schur_solve(Solver &S, int prec, const std::vector<double> &target2, 
     }
     if (!running && !pending) break;
     if (!pending) {
-      const int n = std::min(chunk, max_iter - iters);
+      const int n = std::min(adaptive ? pace.next(hs, nsys, chunk, pairs) : chunk, max_iter - iters);
       if (n <= 0) break;
+      folded = false;
       QCU_TRY(run_chunk(S, *V, K, n, use_graph && n == chunk));
       QCU_TRY(read_states(S));
+      pace.seen(hs, nsys);
       for (int k = 0; k < nsys; ++k) iters = std::max(iters, hs[k].iter);
       trace.mark("  chunk");
       continue;
     }
-    // reliable update of every system still in the batch: fold the
-    // correction into the FP64 solution and recompute the residual in FP64
-    // (this is also the convergence check)
+    // reliable update of every system still in the batch: fold the correction into
+    // the FP64 solution and recompute the residual in FP64 (this is also the
+    // convergence check), with the scalars of a continued recurrence
     std::vector<int> why(nsys);
     for (int k = 0; k < nsys; ++k) why[k] = hs[k].done;
-    QCU_TRY(axpby(op, 1.0, V->x.ptr(), V->px, 1.0, S.xo.ptr(), P64, S.stream));
-    QCU_TRY(zero_spinor(op, V->x.ptr(), V->px, S.stream));
-    QCU_TRY(apply_mhat64(S, S.r64.ptr(), S.xo.ptr(), S.t64.ptr()));
-    QCU_TRY(xmy_norm(op, S.bh.ptr(), S.r64.ptr(), S.st, S.partials, 1, S.stream));
+    QCU_TRY(fold(op, V->x.ptr(), V->px, S.xo.ptr(), S.stream));
+    folded = true;
+    {
+      const LaunchCfg cfg = tuned_cfg(op, P64);
+      SpinorPtr none{};
+      QCU_TRY(hop(op, P64, S.t64.ptr(), S.xo.ptr(), 0, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr, cfg,
+                  S.stream));
+      QCU_TRY(hop(op, P64, S.r64.ptr(), S.t64.ptr(), 1, EPI_XPAY, S.xo.ptr(), RED_RES, S.bh.ptr(), S.st, S.partials,
+                  cfg, S.stream));
+    }
+    QCU_TRY(reliable_residual(op, V->r.ptr(), V->rt.ptr(), S.r64.ptr(), prec, S.st, S.partials, S.stream));
     QCU_TRY(read_states(S));
-    bool restart = false;
+    bool restart = false, left = false;
     for (int k = 0; k < nsys; ++k) {
       if (why[k] == 4) continue;
       stats[k].reliable += 1;
@@ -330,9 +381,13 @@ static int schur_solve(Solver &S, int prec, const std::vector<double> &target2, 
       }
       if (d == 0 && why[k] == 1) hs[k].rr_stop = std::min(hs[k].rr_stop, target2[k]) * 0.01;
       if (d == 0 && why[k] == 2) restart = true;
+      left = left || d == 0;
       hs[k].done = d;
     }
-    QCU_TRY(spinor_convert(op, V->r.ptr(), prec, S.r64.ptr(), P64, S.stream));
+    if (!left) {
+      trace.mark("  reliable update");
+      break;
+    }
     if (restart) {
       // a breakdown restarts the Krylov spaces of the batch from the current residuals
       QCU_TRY(spinor_convert(op, V->rt.ptr(), prec, S.r64.ptr(), P64, S.stream));
@@ -344,14 +399,17 @@ static int schur_solve(Solver &S, int prec, const std::vector<double> &target2, 
         hs[k].alpha[0] = hs[k].omega[0] = 1;
         hs[k].alpha[1] = hs[k].omega[1] = 0;
       }
+      QCU_TRY(write_states(S));
+      QCU_TRY(reliable_residual(op, V->r.ptr(), V->rt.ptr(), S.r64.ptr(), prec, S.st, S.partials, S.stream));
+      QCU_TRY(read_states(S));
     }
+    for (int k = 0; k < nsys; ++k)
+      if (hs[k].done == 0) hs[k].done = !std::isfinite(hs[k].rr) ? 2 : (hs[k].rr < hs[k].rr_stop ? 1 : 0);
     QCU_TRY(write_states(S));
-    QCU_TRY(reliable_dot(op, V->rt.ptr(), V->r.ptr(), prec, S.st, S.partials, S.stream));
-    QCU_TRY(read_states(S));
+    pace.restarted(hs, nsys);
     trace.mark("  reliable update");
   }
-  QCU_TRY(axpby(op, 1.0, V->x.ptr(), V->px, 1.0, S.xo.ptr(), P64, S.stream));
-  QCU_TRY(zero_spinor(op, V->x.ptr(), V->px, S.stream));
+  if (!folded) QCU_TRY(fold(op, V->x.ptr(), V->px, S.xo.ptr(), S.stream));
   for (int k = 0; k < nsys; ++k) stats[k].iters = std::max(stats[k].iters, hs[k].iter);
   return 0;
 }
@@ -432,61 +490,26 @@ static int cgnr_solve(Solver &S, const std::vector<double> &target2, int max_ite
   return 0;
 }
 
-// per-system |b - M x|^2 and |b|^2 of the internal FP64 fields into S.host_scal[2k], [2k+1]
-static int residuals_internal(Solver &S, SpinorPtr xe, SpinorPtr xo, SpinorPtr be, SpinorPtr bo, SpinorPtr t) {
+// per-system |b - M x|^2 and |b|^2 of the internal FP64 fields into S.host_scal[2k],
+// [2k+1]; te: D_eo x_o where the caller has it, else formed in t
+static int residuals_internal(Solver &S, SpinorPtr xe, SpinorPtr xo, SpinorPtr be, SpinorPtr bo, SpinorPtr t,
+                              const SpinorPtr *te) {
   const BatchOp &op = *S.op;
   const LaunchCfg cfg = tuned_cfg(op, P64);
   SpinorPtr none{};
-  QCU_HIP(hipMemsetAsync(S.dscal, 0, 2 * S.nsys * sizeof(double), S.stream));
-  QCU_TRY(hop(op, P64, t, xo, 0, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr, cfg, S.stream, false));
-  QCU_TRY(residual_parity(op, be, xe, t, 0, S.partials, S.dscal, S.stream));
+  if (!te) QCU_TRY(hop(op, P64, t, xo, 0, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr, cfg, S.stream, false));
+  QCU_TRY(residual_parity(op, be, xe, te ? *te : t, 0, S.partials, S.dscal, false, S.stream));
   QCU_TRY(hop(op, P64, t, xe, 1, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr, cfg, S.stream, false));
-  QCU_TRY(residual_parity(op, bo, xo, t, 1, S.partials, S.dscal, S.stream));
+  QCU_TRY(residual_parity(op, bo, xo, t, 1, S.partials, S.dscal, true, S.stream));
   QCU_HIP(hipMemcpyAsync(S.host_scal, S.dscal, 2 * S.nsys * sizeof(double), hipMemcpyDeviceToHost, S.stream));
   QCU_HIP(hipStreamSynchronize(S.stream));
   return 0;
 }
 
-static void system_of(const BatchOp &op, int k, int *seg, int *rhs) {
-  for (size_t s = 0; s < op.segs.size(); ++s) {
-    if (k >= op.segs[s].sys0 && k < op.segs[s].sys0 + op.segs[s].nrhs) {
-      *seg = (int)s;
-      *rhs = k - op.segs[s].sys0;
-      return;
-    }
-  }
-  *seg = -1;
-  *rhs = 0;
-}
-
-static int load_systems(Solver &S, const void *const *ext, SpinorPtr even, SpinorPtr odd) {
-  const BatchOp &op = *S.op;
-  for (int k = 0; k < S.nsys; ++k) {
-    int seg, rhs;
-    system_of(op, k, &seg, &rhs);
-    const size_t half = (size_t)op.segs[seg].g.vh * 12 * 16;
-    QCU_TRY(spinor_ext_to_batch(ext[k], op, seg, rhs, even, P64, S.stream));
-    QCU_TRY(spinor_ext_to_batch((const char *)ext[k] + half, op, seg, rhs, odd, P64, S.stream));
-  }
-  return 0;
-}
-
-static int store_systems(Solver &S, void *const *ext, SpinorPtr even, SpinorPtr odd) {
-  const BatchOp &op = *S.op;
-  for (int k = 0; k < S.nsys; ++k) {
-    int seg, rhs;
-    system_of(op, k, &seg, &rhs);
-    const size_t half = (size_t)op.segs[seg].g.vh * 12 * 16;
-    QCU_TRY(spinor_batch_to_ext(even, op, seg, rhs, ext[k], P64, S.stream));
-    QCU_TRY(spinor_batch_to_ext(odd, op, seg, rhs, (char *)ext[k] + half, P64, S.stream));
-  }
-  return 0;
-}
-
 int true_residuals(Solver &S, const void *const *x_ext, const void *const *b_ext, double *res) {
-  QCU_TRY(load_systems(S, x_ext, S.xe.ptr(), S.xo.ptr()));
-  QCU_TRY(load_systems(S, b_ext, S.be.ptr(), S.bo.ptr()));
-  QCU_TRY(residuals_internal(S, S.xe.ptr(), S.xo.ptr(), S.be.ptr(), S.bo.ptr(), S.r64.ptr()));
+  QCU_TRY(systems_to_batch(x_ext, *S.op, S.xe.ptr(), S.xo.ptr(), S.stream));
+  QCU_TRY(systems_to_batch(b_ext, *S.op, S.be.ptr(), S.bo.ptr(), S.stream));
+  QCU_TRY(residuals_internal(S, S.xe.ptr(), S.xo.ptr(), S.be.ptr(), S.bo.ptr(), S.r64.ptr(), nullptr));
   for (int k = 0; k < S.nsys; ++k) {
     const double num = S.host_scal[2 * k], den = S.host_scal[2 * k + 1];
     res[k] = den > 0 ? sqrt(num / den) : sqrt(num);
@@ -499,17 +522,15 @@ int full_solve(Solver &S, void *const *x_ext, const void *const *b_ext, const Qc
   const int nsys = S.nsys;
   auto t0 = std::chrono::steady_clock::now();
   PhaseTrace trace(S.stream);
-  QCU_TRY(load_systems(S, b_ext, S.be.ptr(), S.bo.ptr()));
+  QCU_TRY(systems_to_batch(b_ext, op, S.be.ptr(), S.bo.ptr(), S.stream));
   // bhat = Ao^-1 (b_o + kappa D_oe Ae^-1 b_e)
   const LaunchCfg cfg = tuned_cfg(op, P64);
   SpinorPtr none{};
-  QCU_TRY(cl_axpy(op, S.t64.ptr(), S.be.ptr(), 0.0, false, none, 1, 0, S.stream));
+  // (with |b|^2 per system for the stopping rule)
+  QCU_TRY(cl_axpy(op, S.t64.ptr(), S.be.ptr(), 0.0, false, none, 1, 0, S.stream, S.dscal, S.partials));
   QCU_TRY(hop(op, P64, S.r64.ptr(), S.t64.ptr(), 1, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr, cfg, S.stream,
               false));
-  QCU_TRY(cl_axpy(op, S.bh.ptr(), S.bo.ptr(), 0.0, true, S.r64.ptr(), 1, 1, S.stream));
-  // |b|^2 per system for the stopping rule
-  QCU_TRY(norm2_dev(op, S.be.ptr(), P64, S.dscal, S.partials, S.stream));
-  QCU_TRY(norm2_dev(op, S.bo.ptr(), P64, S.dscal + nsys, S.partials, S.stream));
+  QCU_TRY(cl_axpy(op, S.bh.ptr(), S.bo.ptr(), 0.0, true, S.r64.ptr(), 1, 1, S.stream, S.dscal + nsys, S.partials));
   QCU_HIP(hipMemcpyAsync(S.host_scal, S.dscal, 2 * nsys * sizeof(double), hipMemcpyDeviceToHost, S.stream));
   QCU_HIP(hipStreamSynchronize(S.stream));
   std::vector<double> target2(nsys), res(nsys, INFINITY);
@@ -519,9 +540,8 @@ int full_solve(Solver &S, void *const *x_ext, const void *const *b_ext, const Qc
     target2[k] = prm.legacy_stop ? prm.tol : 0.25 * prm.tol * prm.tol * b2;
   }
   trace.mark("b_hat + norms");
-  // iterations per graph: a preconditioned solve reaches a reliable update
-  // every 2-4 iterations, and the rest of an 8-iteration graph would only
-  // launch kernels that return at once (measured: 4 is 1-2 % faster there)
+  // iterations per graph: a preconditioned solve reaches a reliable update every
+  // 2-4; unless the caller set a length, fewer are launched where fewer are expected
   const int chunk = prm.chunk > 0 ? prm.chunk : (prm.precond ? 4 : 8);
   const int max_iter = prm.max_iter > 0 ? prm.max_iter : 10000;
   const double delta = prm.reliable_delta > 0 ? prm.reliable_delta : 0.1;
@@ -537,8 +557,8 @@ int full_solve(Solver &S, void *const *x_ext, const void *const *b_ext, const Qc
     if (prm.method == QCU_METHOD_CGNR)
       QCU_TRY(cgnr_solve(S, target2, std::max(budget, 0), chunk, warm, active, st));
     else
-      QCU_TRY(schur_solve(S, prm.precision, target2, delta, std::max(budget, 0), chunk, prm.use_graph != 0, K,
-                          warm, active, st));
+      QCU_TRY(schur_solve(S, prm.precision, target2, delta, std::max(budget, 0), chunk, prm.chunk <= 0,
+                          prm.use_graph != 0, K, warm, active, st));
     trace.mark("schur solve");
     bool stalled = false;
     for (int k = 0; k < nsys; ++k) {
@@ -561,7 +581,8 @@ int full_solve(Solver &S, void *const *x_ext, const void *const *b_ext, const Qc
     QCU_TRY(hop(op, P64, S.t64.ptr(), S.xo.ptr(), 0, EPI_PLAIN, none, RED_NONE, none, nullptr, nullptr, cfg, S.stream,
                 false));
     QCU_TRY(cl_axpy(op, S.xe.ptr(), S.be.ptr(), 0.0, true, S.t64.ptr(), 1, 0, S.stream));
-    QCU_TRY(residuals_internal(S, S.xe.ptr(), S.xo.ptr(), S.be.ptr(), S.bo.ptr(), S.r64.ptr()));
+    const SpinorPtr te = S.t64.ptr();
+    QCU_TRY(residuals_internal(S, S.xe.ptr(), S.xo.ptr(), S.be.ptr(), S.bo.ptr(), S.r64.ptr(), &te));
     trace.mark("x_e + true residual");
     bool again = false;
     for (int k = 0; k < nsys; ++k) {
@@ -576,7 +597,7 @@ int full_solve(Solver &S, void *const *x_ext, const void *const *b_ext, const Qc
     }
     if (!again) break;
   }
-  QCU_TRY(store_systems(S, x_ext, S.xe.ptr(), S.xo.ptr()));
+  QCU_TRY(batch_to_systems(S.xe.ptr(), S.xo.ptr(), op, x_ext, S.stream));
   QCU_HIP(hipStreamSynchronize(S.stream));
   const double secs = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
   if (info) {
