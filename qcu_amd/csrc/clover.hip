@@ -220,7 +220,7 @@ struct CloverKArgs {
   Geom g;
   double coeff;
   CloverOut out[2];  // per parity
-  int *bad;
+  int *bad;  // host memory: set to 1 by a plain store
 };
 
 // The term is built in two launches, each over both parities (neighbouring
@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(2 * kCloverSites) k_clover(CloverKArgs a) {
   if (in) {
     pack6(m, buf);
     store6(o.clov, g.vh, i, w, buf);
-    if (invert6(m)) atomicAdd(a.bad, 1);
+    if (invert6(m)) *(volatile int *)a.bad = 1;
     pack6(m, buf);
     store6(o.cinv64, g.vh, i, w, buf);
     if (o.cinv32) {
@@ -369,7 +369,7 @@ __global__ void __launch_bounds__(2 * kCloverSites) k_clover(CloverKArgs a) {
   }
 }
 
-int clover_build(const LinkPtr &U64, const Geom &g, double coeff, const CloverOut (&out)[2], int *bad_dev,
+int clover_build(const LinkPtr &U64, const Geom &g, double coeff, const CloverOut (&out)[2], int *bad,
                  hipStream_t s) {
   CloverKArgs a;
   a.U = U64;
@@ -377,7 +377,7 @@ int clover_build(const LinkPtr &U64, const Geom &g, double coeff, const CloverOu
   a.coeff = coeff;
   a.out[0] = out[0];
   a.out[1] = out[1];
-  a.bad = bad_dev;
+  a.bad = bad;
   const int nb = 2 * ((g.vh + kCloverSites - 1) / kCloverSites);
   hipLaunchKernelGGL(k_clover_field, dim3(nb), dim3(6 * kCloverSites), 0, s, a);
   hipLaunchKernelGGL(k_clover, dim3(nb), dim3(2 * kCloverSites), 0, s, a);

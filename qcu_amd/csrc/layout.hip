@@ -10,23 +10,103 @@
 
 namespace qcu {
 
+// ---- content hash of an external gauge field -------------------------------
+// A 64-bit summary of every bit of the field, position-dependent, used by the
+// reference-named entry points to keep converted links and the clover term
+// while the caller's gauge is unchanged.  Each complex entry k with bit
+// patterns (a, b) is mixed with k and the mixed words are added modulo 2^64;
+// addition commutes, so the result does not depend on the block order, and a
+// load of the field forms it on the way.
+QCU_D unsigned long long hash_mix(unsigned long long a, unsigned long long b, unsigned long long k) {
+  unsigned long long x = a * 0x9E3779B97F4A7C15ull + b * 0xC2B2AE3D27D4EB4Full + k * 0x165667B19E3779F9ull;
+  x ^= x >> 29;
+  x *= 0xBF58476D1CE4E5B9ull;
+  x ^= x >> 32;
+  x *= 0x94D049BB133111EBull;
+  return x ^ (x >> 29);
+}
+
+QCU_D unsigned long long hash_entry(double2 v, long k) {
+  return hash_mix((unsigned long long)__double_as_longlong(v.x), (unsigned long long)__double_as_longlong(v.y),
+                  (unsigned long long)k);
+}
+
+// sum of h over the 256 threads of a block, in thread 0
+QCU_D unsigned long long block_hash(unsigned long long h) {
+  __shared__ unsigned long long sh[256];
+  sh[threadIdx.x] = h;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+    __syncthreads();
+  }
+  return sh[0];
+}
+
+constexpr int kHashBlocks = 1024;
+
+__global__ void __launch_bounds__(256) k_gauge_hash(const double2 *ext, long n, unsigned long long *part) {
+  unsigned long long h = 0;
+  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x)
+    h += hash_entry(ext[k], k);
+  h = block_hash(h);
+  if (threadIdx.x == 0) part[blockIdx.x] = h;
+}
+
+__global__ void __launch_bounds__(256) k_hash_sum(const unsigned long long *part, int n, unsigned long long *out) {
+  unsigned long long h = 0;
+  for (int k = threadIdx.x; k < n; k += blockDim.x) h += part[k];
+  h = block_hash(h);
+  if (threadIdx.x == 0) *out = h;
+}
+
+static int hash_sum(const void *part, long n, unsigned long long *out, hipStream_t s) {
+  hipLaunchKernelGGL(k_hash_sum, dim3(1), dim3(256), 0, s, (const unsigned long long *)part, (int)n, out);
+  QCU_HIP(hipGetLastError());
+  return 0;
+}
+
+int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, hipStream_t s) {
+  const long n = 36L * 2 * g.vh;  // complex entries: [4][2][Vh][3][3]
+  hipLaunchKernelGGL(k_gauge_hash, dim3(kHashBlocks), dim3(256), 0, s, (const double2 *)ext, n,
+                     (unsigned long long *)scratch);
+  QCU_HIP(hipGetLastError());
+  return hash_sum(scratch, kHashBlocks, out, s);
+}
+
+static long gauge_blocks(const Geom &g) { return (8L * g.vh + 255) / 256; }
+
+size_t gauge_hash_scratch_bytes(const Geom &g) {
+  const long nb = gauge_blocks(g);
+  return (nb > kHashBlocks ? nb : kHashBlocks) * sizeof(unsigned long long);
+}
+
 // Links in every precision the lattice keeps, from one read of the field.
 // 256 consecutive links (36 KiB) are staged through LDS with whole-line loads,
 // then each thread takes rows 0 and 1 of its own link (a stride of 36 banks
 // between lanes: no conflicts for 16-byte reads) and writes them
 // component-planar.  HBM bound: 144 bytes read and 168 written per link with
 // all three precisions.
-template <int M>  // bit k: precision k
+template <int M, bool HASH>  // M bit k: precision k; HASH: partial content hashes as well
 __global__ void __launch_bounds__(256) k_gauge_in(const double2 *ext, Geom g, GaugeOut o) {
   __shared__ double2 sh[256 * 9];
   const int vh = g.vh;
   const long total = 8L * vh;
   const long n0 = (long)blockIdx.x * 256;
   const int m = (int)(total - n0 < 256 ? total - n0 : 256) * 9;  // entries of this block
+  unsigned long long h = 0;
 #pragma unroll
   for (int q = 0; q < 9; ++q) {
     const int k = q * 256 + threadIdx.x;
-    if (k < m) sh[k] = ext[n0 * 9 + k];
+    if (k < m) {
+      const double2 v = ext[n0 * 9 + k];
+      sh[k] = v;
+      if (HASH) h += hash_entry(v, n0 * 9 + k);
+    }
+  }
+  if (HASH) {
+    h = block_hash(h);
+    if (threadIdx.x == 0) o.hash[blockIdx.x] = h;
   }
   __syncthreads();
   const long n = n0 + threadIdx.x;
@@ -60,80 +140,24 @@ __global__ void __launch_bounds__(256) k_gauge_in(const double2 *ext, Geom g, Ga
 }
 
 int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeOut &o, hipStream_t s) {
-  const long n = 8L * g.vh;
-  const dim3 nb((unsigned)((n + 255) / 256)), bs(256);
+  const dim3 nb((unsigned)gauge_blocks(g)), bs(256);
   const double2 *e = (const double2 *)ext;
+  if (o.hash) {
+    QCU_CHECK(mask == 1, QCU_ERR_ARG, "bad precision mask");
+    hipLaunchKernelGGL((k_gauge_in<1, true>), nb, bs, 0, s, e, g, o);
+    QCU_HIP(hipGetLastError());
+    return hash_sum(o.hash, nb.x, o.hash_out, s);
+  }
   switch (mask) {
-    case 1: hipLaunchKernelGGL(k_gauge_in<1>, nb, bs, 0, s, e, g, o); break;
-    case 3: hipLaunchKernelGGL(k_gauge_in<3>, nb, bs, 0, s, e, g, o); break;
-    case 5: hipLaunchKernelGGL(k_gauge_in<5>, nb, bs, 0, s, e, g, o); break;
-    case 7: hipLaunchKernelGGL(k_gauge_in<7>, nb, bs, 0, s, e, g, o); break;
+    case 1: hipLaunchKernelGGL((k_gauge_in<1, false>), nb, bs, 0, s, e, g, o); break;
+    case 3: hipLaunchKernelGGL((k_gauge_in<3, false>), nb, bs, 0, s, e, g, o); break;
+    case 5: hipLaunchKernelGGL((k_gauge_in<5, false>), nb, bs, 0, s, e, g, o); break;
+    case 7: hipLaunchKernelGGL((k_gauge_in<7, false>), nb, bs, 0, s, e, g, o); break;
     default: set_error(QCU_ERR_ARG, "bad precision mask"); return QCU_ERR_ARG;
   }
   QCU_HIP(hipGetLastError());
   return 0;
 }
-
-// ---- content hash of an external gauge field -------------------------------
-// A 64-bit summary of every bit of the field, position-dependent, used by the
-// reference-named entry points to keep converted links and the clover term
-// while the caller's gauge is unchanged.  Each complex entry k with bit
-// patterns (a, b) is mixed with k and the mixed words are added modulo 2^64;
-// addition commutes, so the result does not depend on the block order.
-QCU_D unsigned long long hash_mix(unsigned long long a, unsigned long long b, unsigned long long k) {
-  unsigned long long x = a * 0x9E3779B97F4A7C15ull + b * 0xC2B2AE3D27D4EB4Full + k * 0x165667B19E3779F9ull;
-  x ^= x >> 29;
-  x *= 0xBF58476D1CE4E5B9ull;
-  x ^= x >> 32;
-  x *= 0x94D049BB133111EBull;
-  return x ^ (x >> 29);
-}
-
-constexpr int kHashBlocks = 1024;
-
-__global__ void __launch_bounds__(256) k_gauge_hash(const double2 *ext, long n, unsigned long long *part) {
-  unsigned long long h = 0;
-  for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += (long)gridDim.x * blockDim.x) {
-    const double2 v = ext[k];
-    h += hash_mix((unsigned long long)__double_as_longlong(v.x), (unsigned long long)__double_as_longlong(v.y),
-                  (unsigned long long)k);
-  }
-  __shared__ unsigned long long sh[256];
-  sh[threadIdx.x] = h;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
-}
-
-__global__ void __launch_bounds__(256) k_hash_sum(unsigned long long *part, int n) {
-  __shared__ unsigned long long sh[256];
-  unsigned long long h = 0;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) h += part[k];
-  sh[threadIdx.x] = h;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) part[n] = sh[0];
-}
-
-// scratch: (kHashBlocks + 1) 64-bit words of device memory
-int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, hipStream_t s) {
-  const long n = 36L * 2 * g.vh;  // complex entries: [4][2][Vh][3][3]
-  unsigned long long *part = (unsigned long long *)scratch;
-  hipLaunchKernelGGL(k_gauge_hash, dim3(kHashBlocks), dim3(256), 0, s, (const double2 *)ext, n, part);
-  hipLaunchKernelGGL(k_hash_sum, dim3(1), dim3(256), 0, s, part, kHashBlocks);
-  QCU_HIP(hipGetLastError());
-  QCU_HIP(hipMemcpyAsync(out, part + kHashBlocks, sizeof(*out), hipMemcpyDeviceToHost, s));
-  QCU_HIP(hipStreamSynchronize(s));
-  return 0;
-}
-
-size_t gauge_hash_scratch_bytes() { return (kHashBlocks + 1) * sizeof(unsigned long long); }
 
 // external one-parity field [Vh][4][3] <-> system (segment seg, rhs r) of a batch vector
 template <int P>

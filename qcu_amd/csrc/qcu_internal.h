@@ -114,6 +114,10 @@ struct BatchOp {
   long long nvsites = 0;
   bool has_clover = false;
   std::string tune_base;  // see tune_key()
+  std::vector<char> uploaded;  // contents of the device table
+  // the launch shapes last looked up, valid for tune generation cfg_gen
+  mutable LaunchCfg cfg[3];
+  mutable unsigned long long cfg_gen[3] = {0, 0, 0};
   // one segment per lattice with nrhs[k] right-hand sides
   int build(const std::vector<const Lattice *> &lats, const std::vector<int> &nrhs, hipStream_t s);
   int max_blocks(int bsz) const;
@@ -125,12 +129,16 @@ struct BatchOp {
 // layout.hip
 struct GaugeOut {
   void *u64, *u32, *u16a, *u16b;
+  // with mask 1: scratch of gauge_hash_scratch_bytes() and where the content
+  // hash of the field goes, or null
+  unsigned long long *hash, *hash_out;
 };
 // mask bit k: links of precision k are written (bit 0, FP64, always set)
 int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeOut &out, hipStream_t s);
-// 64-bit content hash of an external gauge field (scratch: gauge_hash_scratch_bytes() of device memory)
+// 64-bit content hash of an external gauge field into *out (memory the device can
+// write); scratch: gauge_hash_scratch_bytes() of device memory
 int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, hipStream_t s);
-size_t gauge_hash_scratch_bytes();
+size_t gauge_hash_scratch_bytes(const Geom &g);
 // external one-parity field <-> system (seg, rhs) of a batch vector
 int spinor_ext_to_batch(const void *ext, const BatchOp &op, int seg, int rhs, SpinorPtr dst, int prec,
                         hipStream_t s);
@@ -169,8 +177,8 @@ struct CloverOut {
   void *cinv16;    // or null
   float *cinv16n;
 };
-// both parities from FP64 internal links; *bad_dev counts singular blocks
-int clover_build(const LinkPtr &U64, const Geom &g, double coeff, const CloverOut (&out)[2], int *bad_dev,
+// both parities from FP64 internal links; *bad (host memory) becomes 1 at a singular block
+int clover_build(const LinkPtr &U64, const Geom &g, double coeff, const CloverOut (&out)[2], int *bad,
                  hipStream_t s);
 
 // blas.hip (every reduction is per system and finishes with finish())

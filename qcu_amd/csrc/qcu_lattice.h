@@ -24,7 +24,7 @@ struct Lattice {
   DevBuf clov64[2];  // packed A (for the true residual)
   DevBuf cinv64[2];  // packed A^-1
   DevBuf cinv32[2], cinv16[2], cinv16n[2];
-  DevBuf flag;       // singular-clover counter
+  int *bad = nullptr;  // a singular clover block was met (pinned host memory)
   // staging of qcuDslash and qcuMatFull, made on first use and kept: half
   // spinors of the low precisions, and a copy of an input that overlaps the output
   Spinor stage[2];
@@ -35,7 +35,10 @@ struct Lattice {
 
   int init(const int L_[4], double kappa_, double csw_, int tbc);
   // prec_mask bit k: keep links (and clover inverse) in precision k
-  int load_gauge(const void *gauge_ext_dev, int prec_mask = 7);
+  // hash (with mask 1): scratch for, and the place of, the field's content hash; the
+  // hash is there when the call returns
+  int load_gauge(const void *gauge_ext_dev, int prec_mask = 7, unsigned long long *hash_scratch = nullptr,
+                 unsigned long long *hash = nullptr);
   bool has_clover() const { return csw != 0.0; }
   LinkPtr links(int prec) const;
   CloverPtr clover_inv(int prec, int parity) const;

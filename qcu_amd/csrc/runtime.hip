@@ -93,18 +93,24 @@ int BatchOp::build(const std::vector<const Lattice *> &ls, const std::vector<int
   const int pcap = max_blocks(64) + 1;
   for (SegDesc &d : segs) d.pcap = pcap;
   tune_base = qcu::tune_base(*this);
+  for (unsigned long long &gen : cfg_gen) gen = 0;
   std::vector<int> first;  // see find_seg()
   for (int k = 0; k < kSegBlockSizes; ++k) {
     const int bsz = seg_block_size(k);
     first.push_back(0);
     for (const SegDesc &d : segs) first.push_back(first.back() + (d.nthr + bsz - 1) / bsz);
   }
-  const size_t nb = segs.size() * sizeof(SegDesc);
-  QCU_TRY(dseg.alloc(nb + first.size() * sizeof(int)));
+  const size_t nb = segs.size() * sizeof(SegDesc), nf = first.size() * sizeof(int);
+  std::vector<char> table(nb + nf);
+  std::memcpy(table.data(), segs.data(), nb);
+  std::memcpy(table.data() + nb, first.data(), nf);
+  if (dseg.p && table == uploaded) return 0;  // a reloaded lattice keeps its buffers
+  uploaded.clear();
+  QCU_TRY(dseg.alloc(table.size()));
   dev_segs = (SegDesc *)dseg.p;
-  QCU_HIP(hipMemcpyAsync(dev_segs, segs.data(), nb, hipMemcpyHostToDevice, s));
-  QCU_HIP(hipMemcpyAsync((char *)dseg.p + nb, first.data(), first.size() * sizeof(int), hipMemcpyHostToDevice, s));
+  QCU_HIP(hipMemcpyAsync(dev_segs, table.data(), table.size(), hipMemcpyHostToDevice, s));
   QCU_HIP(hipStreamSynchronize(s));
+  uploaded.swap(table);
   return 0;
 }
 
@@ -136,11 +142,11 @@ int Lattice::init(const int L_[4], double kappa_, double csw_, int tbc) {
   device = current_device();
   QCU_CHECK(device >= 0, QCU_ERR_STATE, "no HIP device");
   QCU_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
-  QCU_TRY(flag.alloc(256));
+  QCU_HIP(hipHostMalloc((void **)&bad, sizeof(int), hipHostMallocDefault));
   return 0;
 }
 
-int Lattice::load_gauge(const void *ext, int mask) {
+int Lattice::load_gauge(const void *ext, int mask, unsigned long long *hash_scratch, unsigned long long *hash) {
   QCU_CHECK(ext != nullptr, QCU_ERR_ARG, "gauge pointer is null");
   const size_t vh = g.vh;
   mask |= 1;  // FP64 links are always kept (clover build, reliable updates)
@@ -155,10 +161,9 @@ int Lattice::load_gauge(const void *ext, int mask) {
     QCU_TRY(U16a.alloc(8 * vh * 16));
     QCU_TRY(U16b.alloc(8 * vh * 8));
   }
-  QCU_TRY(gauge_ext_to_internal(ext, g, mask, GaugeOut{U64.p, U32.p, U16a.p, U16b.p}, stream));
+  QCU_TRY(gauge_ext_to_internal(ext, g, mask, GaugeOut{U64.p, U32.p, U16a.p, U16b.p, hash_scratch, hash}, stream));
   if (has_clover()) {
-    int *bad = (int *)flag.p;
-    QCU_HIP(hipMemsetAsync(bad, 0, sizeof(int), stream));
+    *bad = 0;  // nothing of an earlier load is in flight
     CloverOut out[2];
     for (int p = 0; p < 2; ++p) {
       QCU_TRY(clov64[p].alloc(vh * 72 * 8));
@@ -176,12 +181,9 @@ int Lattice::load_gauge(const void *ext, int mask) {
       }
     }
     QCU_TRY(clover_build(links(P64), g, kappa * csw, out, bad, stream));
-    int hbad = 0;
-    QCU_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, stream));
-    QCU_HIP(hipStreamSynchronize(stream));
-    QCU_CHECK(hbad == 0, QCU_ERR_STATE, "singular clover block");
   }
   QCU_HIP(hipStreamSynchronize(stream));
+  QCU_CHECK(!has_clover() || *(volatile int *)bad == 0, QCU_ERR_STATE, "singular clover block");
   // the lattice's own one-system batch table is built from a loaded lattice
   prec_mask = mask;
   gauge_loaded = true;
@@ -268,6 +270,7 @@ SegDesc Lattice::seg_desc(int nrhs) const {
 
 Lattice::~Lattice() {
   solver.reset();
+  if (bad) (void)hipHostFree(bad);
   if (stream) (void)hipStreamDestroy(stream);
 }
 

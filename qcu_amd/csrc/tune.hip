@@ -55,10 +55,21 @@ static int valid_cfg(int block, int remap, int group) {
 // once when the batch is built (asking the driver for the device costs more
 // than a small hop)
 std::string tune_base(const BatchOp &op) {
+  static std::mutex mu;
+  static std::map<int, std::string> names;  // device names, asked for once
   std::string k;
-  hipDeviceProp_t prop;
-  int dev = current_device();
-  if (dev >= 0 && hipGetDeviceProperties(&prop, dev) == hipSuccess) k = prop.gcnArchName;
+  {
+    std::lock_guard<std::mutex> lk(mu);
+    const int dev = current_device();
+    auto it = names.find(dev);
+    if (it == names.end()) {
+      hipDeviceProp_t prop;
+      if (dev >= 0 && hipGetDeviceProperties(&prop, dev) == hipSuccess) k = prop.gcnArchName;
+      names[dev] = k;
+    } else {
+      k = it->second;
+    }
+  }
   char buf[96];
   for (const SegDesc &d : op.segs) {
     snprintf(buf, sizeof(buf), ":%dx%dx%dx%dr%d", 2 * d.g.lxh, d.g.ly, d.g.lz, d.g.lt, d.nrhs);
@@ -73,7 +84,7 @@ std::string tune_key(const BatchOp &op, int prec) {
   return op.tune_base + buf;
 }
 
-LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
+static LaunchCfg find_cfg(const BatchOp &op, int prec) {
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
     auto it = g_tuned.find(tune_key(op, prec));
@@ -88,6 +99,15 @@ LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
   c.block = op.nvsites <= (1 << 20) ? 64 : 256;
   c.group = prec == P64 ? 0 : 2;
   return c;
+}
+
+LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
+  const unsigned long long gen = tune_generation();
+  if (op.cfg_gen[prec] != gen) {
+    op.cfg[prec] = find_cfg(op, prec);
+    op.cfg_gen[prec] = gen;
+  }
+  return op.cfg[prec];
 }
 
 // average milliseconds per launch of the hop kernel on resident fields
