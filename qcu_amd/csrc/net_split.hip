@@ -946,14 +946,30 @@ __global__ void __launch_bounds__(256) k_net_pack_second(const float2 *W1, const
   }
 }
 
-// MIX: the epilogue also writes the next layer's single-output term fields
-// (fused_epilogue with the hop terms' operands in global memory, the site
-// term's in LDS)
-template <int WAVES, bool MIX>
+// Both parities of this layer, or one half of a 1-8-8-8-1 preconditioner.  There
+// only the odd network output is kept, so that with L2 the second layer's odd
+// sites, by the same linearity, the last layer's hop fields at even sites are
+//   Z_t(x) = sum_u (W4_t W3_u) T_u L2(x + u) + sum_u G_{t,u} T_u in(x + u),
+//   G_{t,u} = (W4_t W3_8 + W4_8 W3_t) E_u,
+// and its site field at odd z is W4_8 W3_8 L2(z): two kernels of this one shape,
+// one over odd sites (SECOND_ODD: L2, and its site field in the epilogue) and one
+// over even sites (SECOND_TAIL: the 8 fields Z_t take the place of 8 output
+// channels).  The second layer's even sites and the third layer are never formed.
+// The composed matrices are FP64 sums rounded to FP32 once per weight version
+// (k_net_compose_tail).  One application, against the second layer on both
+// parities with the last layer's composed fields in its epilogue, the third layer on
+// its even sites with the last one's in its epilogue, and a gather of two sets of
+// fields: 24^3x48 1129 -> 947 us (second 556 -> 413, third 403 -> 403, gather 125 ->
+// 70), 32^3x64 3245 -> 2660, 16^3x32 251 -> 214.  Both are bound by the loads of the
+// 8-channel field (4-5 times its size reaches them) and by the vector units' work on
+// it (transports and splits, half of the time); loads two steps ahead, or all
+// terms of two channels before the next two, measured no faster.
+enum { SECOND_BOTH, SECOND_ODD, SECOND_TAIL };
+template <int WAVES, int MODE>
 __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
   typedef SplitShape<32> SH;
   constexpr int NH = 8 * 2 * 4 * 2 * 64;  // the second layer's hop-term operands (split packing, terms 0..7)
-  constexpr int N2 = MIX ? 4 * 2 * 64 : 0;  // the mixing's site-term operands (8 KiB: 156 KiB in all)
+  constexpr int N2 = MODE == SECOND_ODD ? 4 * 2 * 64 : 0;  // the site field's operands (8 KiB: 156 KiB in all)
   __shared__ uint4 lw[NH + kFirstPackOps + N2];
   if (a.st && a.st->done) return;  // uniform over the grid
   for (int k = threadIdx.x; k < NH; k += blockDim.x) lw[k] = a.Ah[k];
@@ -966,8 +982,9 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
   const float s0 = pow2_scale(__uint_as_float(*a.in_max), 14);
   const float s1 = pow2_scale(__uint_as_float(*a.l1_max), 14);
   const float oe = a.winv[0] / s0;    // even sites: E against the input
-  const float oo = a.winvh[0] / s1;   // odd sites: the hop terms against L1
-  const float rs = (a.winv[1] * s1) / (a.winvh[0] * s0);  // the site term's part -> the hop terms' scale
+  const float oo = a.winvh[0] / s1;   // the hop terms against L1
+  // the input's part (site term S, or G) -> the hop terms' scale
+  const float rs = (a.winv[MODE == SECOND_TAIL ? 0 : 1] * s1) / (a.winvh[0] * s0);
   const int lane = threadIdx.x & 63, gq = lane >> 5, n = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t field = (size_t)g.vh * 96, plane = (size_t)g.vh * 16;
@@ -1058,27 +1075,25 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
   float4 lraw[3], vb[6];
   const SlabOrder sl = slab_order(g, WAVES, wave);
   // chunk c: the lane's site (lanes past the last site compute a copy of a
-  // valid site and store nothing) and the even pass's first loads
+  // valid site and store nothing) and the first pass's first loads
   auto begin = [&](int c) {
     const int base = slab_chunk(sl, g, c) * 32;
     i = base + n;
     ok = i < g.vh;
     if (!ok) i = base;
-    se = decode(g, i, 0);
-    tg = term_geo_u(g, se, i, 0, term_const(g, gq));
-    load_link(tg, lraw);
-    load_in(vb, tg.j);
+    if constexpr (MODE == SECOND_ODD) {
+      load_in(vb, i);
+    } else {
+      se = decode(g, i, 0);
+      tg = term_geo_u(g, se, i, 0, term_const(g, gq));
+      load_link(tg, lraw);
+      load_in(vb, tg.j);
+    }
   };
-  const int cstep = sl.cstep, cend = sl.cend;
-  int c = sl.c0;
-  if (c < cend) begin(c);
-#pragma unroll 1
-  for (; c < cend; c += cstep) {
-    const int ic = i;
-    const bool okc = ok;
-    // even output sites: K step ks = the hops in direction ks of the input
-    // (forward on lane group 0, backward on group 1) against E
-    clear();
+  // the input's 8 hops at even site ic: K step ks = the hops in direction ks
+  // (forward on lane group 0, backward on group 1); next() issues the following
+  // pass's first loads
+  auto input_hops = [&](int ic, auto next) {
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
       cf m[9], v[4][3];
@@ -1090,52 +1105,50 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
         tg = term_geo_u(g, se, ic, 0, term_const(g, 2 * (ks + 1) + gq));
         load_link(tg, lraw);
         load_in(vb, tg.j);
-      } else if constexpr (!MIX) {
-        load_in(vb, ic);  // the odd pass's site term: the site's own input
+      } else {
+        next();
       }
       __builtin_amdgcn_sched_barrier(0);
       products(v, le + (ks * 2) * 2 * 64, 2 * 64);
     }
-    if (okc) store(ic, 0, oe);
-    if constexpr (MIX) {
-      // the hop-term fields of the single-output mixing; the odd pass's site
-      // operand is loaded once the accumulators are split
-      const MixOut mo{a.A2, ls2, a.winv2, a.mix};
-      fused_epilogue(mo, acc, oe, ic, 0, okc, gq, lane, field, plane, [&]() { load_in(vb, ic); });
+  };
+  // the input's part of the accumulators -> the hop terms' scale
+  auto rescale = [&]() {
+#pragma unroll
+    for (int cc = 0; cc < 3; ++cc) {
+      acc[cc][0] *= rs;
+      acc[cc][1] *= rs;
     }
-    // odd output sites: the site term S on lane group 0 first, then the
-    // accumulators take the hop terms' scale and the 8 hop terms follow
-    // against the first layer's even sites (the term's link and the next K
-    // step's channels loaded one step ahead, as in k_net_layer_split)
-    const Site so = decode(g, ic, 1);
-    clear();
-    {
-      cf v[4][3];
-      unpack(vb, v);
-      __builtin_amdgcn_sched_barrier(0);
-      tg = term_geo(g, so, ic, 1, 0);
-      load_link(tg, lraw);
-      load_l1(vb, tg, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      const float f = gq == 0 ? s0 : 0.f;
+  };
+  // the site term S of an odd site on lane group 0; next() as above
+  auto site_term = [&](auto next) {
+    cf v[4][3];
+    unpack(vb, v);
+    __builtin_amdgcn_sched_barrier(0);
+    next();
+    __builtin_amdgcn_sched_barrier(0);
+    const float f = gq == 0 ? s0 : 0.f;
 #pragma unroll
-      for (int s2 = 0; s2 < 4; ++s2)
+    for (int s2 = 0; s2 < 4; ++s2)
 #pragma unroll
-        for (int cc = 0; cc < 3; ++cc) v[s2][cc] = f * v[s2][cc];
-      products(v, le + (4 * 2) * 2 * 64, 2 * 64);
-#pragma unroll
-      for (int cc = 0; cc < 3; ++cc) {
-        acc[cc][0] *= rs;
-        acc[cc][1] *= rs;
-      }
-    }
+      for (int cc = 0; cc < 3; ++cc) v[s2][cc] = f * v[s2][cc];
+    products(v, le + (4 * 2) * 2 * 64, 2 * 64);
+  };
+  auto first_hop = [&](const Site &so, int ic, int p) {
+    tg = term_geo(g, so, ic, p, 0);
+    load_link(tg, lraw);
+    load_l1(vb, tg, 0);
+  };
+  // the 8 hop terms against the 8 channels (the term's link and the next K
+  // step's channels loaded one step ahead, as in k_net_layer_split)
+  auto hop_terms = [&](const Site &so, int ic, int p) {
 #pragma unroll 1
     for (int t = 0; t < 8; ++t) {
       cf m[9];
       term_matrix(lraw, 1, tg.fwd, tg.ph * s1, m);
       TermGeo ng = tg;
       if (t + 1 < 8) {
-        ng = term_geo(g, so, ic, 1, t + 1);
+        ng = term_geo(g, so, ic, p, t + 1);
         load_link(ng, lraw);
       }
 #pragma unroll
@@ -1151,10 +1164,41 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
       }
       tg = ng;
     }
-    if constexpr (MIX) {
+  };
+  const int cstep = sl.cstep, cend = sl.cend;
+  int c = sl.c0;
+  if (c < cend) begin(c);
+#pragma unroll 1
+  for (; c < cend; c += cstep) {
+    const int ic = i;
+    const bool okc = ok;
+    clear();
+    if constexpr (MODE == SECOND_TAIL) {
+      // even sites: G against the input, then the accumulators take the hop
+      // terms' scale and the hop terms follow
+      input_hops(ic, [&]() { first_hop(se, ic, 0); });
+      rescale();
+      hop_terms(se, ic, 0);
+      if (c + cstep < cend) begin(c + cstep);  // the next chunk's first loads, ahead of the stores
+      if (okc) store(ic, 0, oo);
+      continue;
+    }
+    if constexpr (MODE == SECOND_BOTH) {
+      // even sites: the input's hops against E
+      input_hops(ic, [&]() { load_in(vb, ic); });
+      if (okc) store(ic, 0, oe);
+      clear();
+    }
+    // odd sites: the site term S first, then the 8 hop terms against the first
+    // layer's even sites
+    const Site so = decode(g, ic, 1);
+    site_term([&]() { first_hop(so, ic, 1); });
+    rescale();
+    hop_terms(so, ic, 1);
+    if constexpr (MODE == SECOND_ODD) {
       if (okc) store(ic, 1, oo);
-      // the site-term field; the next chunk's first loads once the accumulators are split
-      const MixOut mo{a.A2, ls2, a.winv2, a.mix};
+      // the site field; the next chunk's first loads once the accumulators are split
+      const MixOut mo{ls2, ls2, a.winv2, a.mix};
       fused_epilogue(mo, acc, oo, ic, 1, okc, gq, lane, field, plane, [&]() {
         if (c + cstep < cend) begin(c + cstep);
       });
@@ -1166,27 +1210,67 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
   if (a.out_max) record_max(a.out_max, omax);
 }
 
-// The last layer's site term composed with the layer before it:
-// Wc[u][0][i] = W4_8[0][j] W3_u[j][i] (sum over j and the inner spin), the
-// weights of a single-output layer over that layer's input (u = 0..8), laid
-// out as a (cin 8, cout 1) layer for net_pack_fuse.  FP64 sums, FP32 result.
-__global__ void __launch_bounds__(256) k_net_compose_last(const float2 *W3, const float2 *W4, float2 *Wc) {
-  for (int e = threadIdx.x; e < 9 * 8 * 16; e += blockDim.x) {
-    const int u = e >> 7, i = (e >> 4) & 7, s = (e >> 2) & 3, s2 = e & 3;
-    double re = 0.0, im = 0.0;
+// The composed matrices of a 1-8-8-8-1 preconditioner (see k_net_second), as
+// weights in the layout of an 8 -> 8, a 1 -> 8 and an 8 -> 1 layer:
+//   C[u][t][i] = W4_t W3_u          (u, t = 0..7; u = 8: zero)
+//   G[u][t][0] = (W4_t W3_8 + W4_8 W3_t) (W2_u W1_8 + W2_8 W1_u)   (u = 8: zero)
+//   S[8][0][i] = W4_8 W3_8          (other terms zero)
+// FP64 sums, rounded to FP32.  Block u forms the matrices of term u.
+__global__ void __launch_bounds__(256) k_net_compose_tail(const float2 *W1, const float2 *W2, const float2 *W3,
+                                                          const float2 *W4, float2 *C, float2 *G, float2 *S) {
+  __shared__ double2 M[8 * 8 * 16], E[8 * 16];
+  const int u = blockIdx.x, tid = threadIdx.x;
+  // sum_j sum_sp A[j][s][sp] B[j][sp][s2], j strides as and bs (in spin matrices)
+  auto mul = [](const float2 *A, int as, const float2 *B, int bs, int s, int s2, double2 &r) {
     for (int j = 0; j < 8; ++j)
       for (int sp = 0; sp < 4; ++sp) {
-        const float2 a = W4[((size_t)8 * 8 + j) * 16 + s * 4 + sp];
-        const float2 b = W3[(((size_t)u * 8 + j) * 8 + i) * 16 + sp * 4 + s2];
-        re += (double)a.x * b.x - (double)a.y * b.y;
-        im += (double)a.x * b.y + (double)a.y * b.x;
+        const float2 x = A[(size_t)j * as * 16 + s * 4 + sp], y = B[(size_t)j * bs * 16 + sp * 4 + s2];
+        r.x += (double)x.x * y.x - (double)x.y * y.y;
+        r.y += (double)x.x * y.y + (double)x.y * y.x;
       }
-    Wc[e] = make_float2((float)re, (float)im);
+  };
+  auto w3 = [&](int t, int i) { return W3 + ((size_t)t * 64 + i) * 16; };  // outputs j: stride 8
+  auto w4 = [&](int t) { return W4 + (size_t)t * 8 * 16; };                // inputs j: stride 1
+  auto f32 = [](double2 v) { return make_float2((float)v.x, (float)v.y); };
+  for (int e = tid; e < 8 * 8 * 16; e += 256) {
+    const int t = e >> 7, i = (e >> 4) & 7, s = (e >> 2) & 3, s2 = e & 3;
+    double2 c = make_double2(0.0, 0.0), m = c;
+    if (u < 8) {
+      mul(w4(t), 1, w3(u, i), 8, s, s2, c);
+      mul(w4(t), 1, w3(8, i), 8, s, s2, m);
+      mul(w4(8), 1, w3(t, i), 8, s, s2, m);
+    }
+    M[e] = m;
+    C[(size_t)u * 1024 + e] = f32(c);
+  }
+  if (tid < 8 * 16) {
+    const int i = tid >> 4, s = (tid >> 2) & 3, s2 = tid & 3;
+    double2 v = make_double2(0.0, 0.0), w = v;
+    if (u < 8) {
+      mul(W2 + ((size_t)u * 64 + i * 8) * 16, 1, W1 + (size_t)8 * 8 * 16, 1, s, s2, v);
+      mul(W2 + ((size_t)8 * 64 + i * 8) * 16, 1, W1 + (size_t)u * 8 * 16, 1, s, s2, v);
+    } else {
+      mul(w4(8), 1, w3(8, i), 8, s, s2, w);
+    }
+    E[tid] = v;
+    S[(size_t)u * 128 + tid] = f32(w);
+  }
+  __syncthreads();
+  if (tid < 8 * 16) {
+    const int t = tid >> 4, s = (tid >> 2) & 3, s2 = tid & 3;
+    double2 v = make_double2(0.0, 0.0);
+    for (int i = 0; i < 8; ++i)
+      for (int sp = 0; sp < 4; ++sp) {
+        const double2 x = M[(t * 8 + i) * 16 + s * 4 + sp], y = E[i * 16 + sp * 4 + s2];
+        v.x += x.x * y.x - x.y * y.y;
+        v.y += x.x * y.y + x.y * y.x;
+      }
+    G[(size_t)u * 128 + tid] = f32(v);
   }
 }
 
-int net_compose_last(const float2 *W3, const float2 *W4, float2 *Wc, hipStream_t s) {
-  hipLaunchKernelGGL(k_net_compose_last, dim3(1), dim3(256), 0, s, W3, W4, Wc);
+int net_compose_tail(const float2 *const (&W)[4], float2 *C, float2 *G, float2 *S, hipStream_t s) {
+  hipLaunchKernelGGL(k_net_compose_tail, dim3(9), dim3(256), 0, s, W[0], W[1], W[2], W[3], C, G, S);
   QCU_HIP(hipGetLastError());
   return 0;
 }
@@ -1197,7 +1281,7 @@ int net_pack_second(const float2 *W1, const float2 *W2, void *Apk, float *winv, 
   return 0;
 }
 
-int net_layer_second(const NetSecondArgs &a, hipStream_t s) {
+int net_layer_second(const NetSecondArgs &a, int part, hipStream_t s) {
   QCU_CHECK((size_t)a.g.vh * 96 * 2 + (size_t)a.g.vh * 16 < ((size_t)1 << 32), QCU_ERR_DIMS,
             "net: lattice too large for the second layer");
   static int ncu = 0;
@@ -1207,13 +1291,16 @@ int net_layer_second(const NetSecondArgs &a, hipStream_t s) {
     QCU_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
     if (ncu <= 0) ncu = 256;
   }
-  // 8 waves per block, one block per CU (the operands fill 148 KiB of its LDS, 156 KiB with the mixing)
+  // 8 waves per block, one block per CU (the operands fill 148 or 156 KiB of its LDS)
   constexpr int waves = 8;
   const int nchunk = (a.g.vh + 31) / 32;
   int nblk = ncu;
   if (nchunk < nblk * waves) nblk = (nchunk + waves - 1) / waves;
-  if (a.A2) hipLaunchKernelGGL((k_net_second<waves, true>), dim3(nblk), dim3(64 * waves), 0, s, a);
-  else hipLaunchKernelGGL((k_net_second<waves, false>), dim3(nblk), dim3(64 * waves), 0, s, a);
+  switch (part) {
+    case 0: hipLaunchKernelGGL((k_net_second<waves, SECOND_BOTH>), dim3(nblk), dim3(64 * waves), 0, s, a); break;
+    case 1: hipLaunchKernelGGL((k_net_second<waves, SECOND_ODD>), dim3(nblk), dim3(64 * waves), 0, s, a); break;
+    default: hipLaunchKernelGGL((k_net_second<waves, SECOND_TAIL>), dim3(nblk), dim3(64 * waves), 0, s, a); break;
+  }
   QCU_HIP(hipGetLastError());
   return 0;
 }

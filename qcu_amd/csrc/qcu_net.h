@@ -218,34 +218,38 @@ int net_pack_first(const float2 *W, void *Apk, float *winv, hipStream_t s);
 int net_layer_first(const NetFirstArgs &a, hipStream_t s, bool even_only = false);
 
 // the second layer (8 -> 8) after a first layer on an input zero on the even
-// sites, with the first layer's odd sites left implicit (net_layer_second):
-// even outputs from the input alone, odd outputs from the first layer's even
-// sites and the input
+// sites, with the first layer's odd sites left implicit (net_layer_second).
+// part 0: even outputs from the input alone, odd outputs from the first layer's
+// even sites and the input.  part 1: the odd outputs only, and the last layer's
+// site field of a 1-8-8-8-1 network at them (mix).  part 2: that network's last
+// hop fields at even sites from the second layer's odd sites (l1) and the input,
+// in place of output channels (out: term t in slot t)
 struct NetSecondArgs {
   const char *in;           // the network input (channel 0 of both parities; the odd sites are read)
-  const char *l1;           // the first layer's 8 channels (both parities; the even sites are read)
+  const char *l1;           // 8 channels (both parities): the first layer's even sites, or (part 2) the second
+                            // layer's odd sites, are read
   char *out;                // the 8 output channels
-  const uint4 *A;           // combined operands E_t, S (net_pack_second)
-  const float *winv;        // their inverse scales: [0] E, [1] S
-  const uint4 *Ah;          // the second layer's own split operands (net_pack_split; terms 0..7 used)
+  const uint4 *A;           // combined operands E_t, S (net_pack_second), or G (net_pack_first)
+  const float *winv;        // their inverse scales: [0] E or G, [1] S
+  const uint4 *Ah;          // the hop terms' split operands (net_pack_split; terms 0..7 used)
   const float *winvh;       // their inverse scale
   const unsigned *in_max;   // largest |component| of the input (float bits)
-  const unsigned *l1_max;   // that of the first layer's even sites
+  const unsigned *l1_max;   // that of l1's sites read
   unsigned *out_max;        // receives that of the output (or null)
   LinkPtr U;                // FP32 links
   Geom g;
   const SysState *st;       // early-out flag of a captured solver iteration (or null)
-  // optional: the last layer's site-term mixing composed with the next layer,
-  // written as the single-output layer's term fields (hop terms at even
-  // sites, the site term at odd ones; see NetSplitArgs); null A2: none
+  // part 1: packed operands of the site field (net_pack_fuse), their inverse scale,
+  // and the term fields (written: the site term at the odd sites)
   const uint4 *A2 = nullptr;
   const float *winv2 = nullptr;
   char *mix = nullptr;
 };
 int net_pack_second(const float2 *W1, const float2 *W2, void *Apk, float *winv, hipStream_t s);
-// Wc[u][0][i][4x4] = W4_8[0][j] W3_u[j][i] (8 -> 8 layer W3, 8 -> 1 layer W4; u = 0..8)
-int net_compose_last(const float2 *W3, const float2 *W4, float2 *Wc, hipStream_t s);
-int net_layer_second(const NetSecondArgs &a, hipStream_t s);
+// matrices of net_layer_second's parts 1 and 2, composed of the weights W of a
+// 1-8-8-8-1 network: C an 8 -> 8, G a 1 -> 8 and S an 8 -> 1 layer's weights
+int net_compose_tail(const float2 *const (&W)[4], float2 *C, float2 *G, float2 *S, hipStream_t s);
+int net_layer_second(const NetSecondArgs &a, int part, hipStream_t s);
 
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 
