@@ -942,7 +942,12 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
     float4 *sG = smem, *sV = smem + 48 * 32;
     float2 *sM = (float2 *)(smem + 2 * 48 * 32);  // the term's colour matrix at each site of the step
     const int tid = threadIdx.x;
-    const int fs = tid & 31;  // the thread's site in a step; its planes: (tid >> 5) + 8 r
+    // the thread's site in a step; its planes: (tid >> 5) + 8 r.  Plane b holds its
+    // sites rotated by b mod 8: a matrix-core operand is read at one site from 16
+    // planes (4 channels x 4 spins) at once, which would all lie in the same banks,
+    // and with the rotation 8 lanes fall on 7 or 8 of the 8 bank groups (16^3x32,
+    // 8 -> 8 channels: WGTIME).
+    const int fs = ((tid & 31) + (tid >> 5)) & 31;
     // the thread's six planes (separate variables: arrays of them end up in
     // scratch memory in some instances)
     auto plane_base = [&](int r, const SpinorPtr &f, int nch) {
@@ -972,9 +977,12 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
       const unsigned ov = (unsigned)tg.jp * 6u * (unsigned)g.vh + (unsigned)tg.j;
       typedef void __attribute__((address_space(3))) *lds_t;
       const int wb = 2 * wave * 32;
-#define QCU_WG_LDS(R_)                                                                                   \
-  __builtin_amdgcn_global_load_lds((const void *)(gb##R_ + og), (lds_t)(sG + wb + 8 * (R_) * 32), 16, 0, 0); \
-  __builtin_amdgcn_global_load_lds((const void *)(vb##R_ + ov), (lds_t)(sV + wb + 8 * (R_) * 32), 16, 0, 0);
+      // planes of channels that do not exist are not read
+#define QCU_WG_LDS(R_)                                                                                         \
+  if (2 * wave + 8 * (R_) < 6 * a.cout)                                                                        \
+    __builtin_amdgcn_global_load_lds((const void *)(gb##R_ + og), (lds_t)(sG + wb + 8 * (R_) * 32), 16, 0, 0); \
+  if (2 * wave + 8 * (R_) < 6 * a.cin)                                                                         \
+    __builtin_amdgcn_global_load_lds((const void *)(vb##R_ + ov), (lds_t)(sV + wb + 8 * (R_) * 32), 16, 0, 0);
       QCU_WG_LDS(0) QCU_WG_LDS(1) QCU_WG_LDS(2) QCU_WG_LDS(3) QCU_WG_LDS(4) QCU_WG_LDS(5)
 #undef QCU_WG_LDS
       if (linker && tcon.hop) {
@@ -986,20 +994,22 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
       }
     };
     // the products of the wave's group h (0, 1) of the step
+    // float4 of site s in plane b
+    auto staged = [](const float4 *base, int b, int s) { return base[b * 32 + ((s - (b & 7)) & 31)]; };
     auto group = [&](int g0, int h) {
       const int s = 16 * h + 4 * wave + q;
       Ops x;
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         const int o = grow[mt] != 0.f ? 4 * mt + o_n : 0;
-        x.g[mt][0] = sG[(o * 6 + rslot) * 32 + s];
-        x.g[mt][1] = sG[(o * 6 + rslot + 1) * 32 + s];
+        x.g[mt][0] = staged(sG, o * 6 + rslot, s);
+        x.g[mt][1] = staged(sG, o * 6 + rslot + 1, s);
       }
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
         const int ch = gcol[nt] != 0.f ? 4 * nt + o_n : 0;
-        x.v[nt][0] = sV[(ch * 6 + rslot) * 32 + s];
-        x.v[nt][1] = sV[(ch * 6 + rslot + 1) * 32 + s];
+        x.v[nt][0] = staged(sV, ch * 6 + rslot, s);
+        x.v[nt][1] = staged(sV, ch * 6 + rslot + 1, s);
       }
       cf u[9];
       if (tcon.hop) {
