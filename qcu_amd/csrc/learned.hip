@@ -789,17 +789,11 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
   const float sg = SPLIT ? pow2_scale(__uint_as_float(*a.gmax), 14) : 1.f;
   const float sv = SPLIT ? pow2_scale(__uint_as_float(*a.amax), 14) : 1.f;
   // the lane's spin (3 colours) out of its two raw float4 slots
-  auto spin3 = [&](const float4 (&r)[2], float keep, cf (&v)[3]) {
+  auto spin3 = [&](const float4 (&r)[2], cf (&v)[3]) {
     const float4 x = r[0], y = r[1];
-    if (rodd) {
-      v[0] = mk(keep * x.z, keep * x.w);
-      v[1] = mk(keep * y.x, keep * y.y);
-      v[2] = mk(keep * y.z, keep * y.w);
-    } else {
-      v[0] = mk(keep * x.x, keep * x.y);
-      v[1] = mk(keep * x.z, keep * x.w);
-      v[2] = mk(keep * y.x, keep * y.y);
-    }
+    v[0] = rodd ? mk(x.z, x.w) : mk(x.x, x.y);
+    v[1] = rodd ? mk(y.x, y.y) : mk(x.z, x.w);
+    v[2] = rodd ? mk(y.z, y.w) : mk(y.x, y.y);
   };
   // one group of 4 sites: geometry and raw operands (loaded one group ahead)
   struct Geo {
@@ -810,14 +804,12 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
   struct Ops {
     float4 g[MT][2], v[NT][2], l[3];
   };
-  // lanes whose row or column channel does not exist read channel 0 and are
-  // scaled by zero, so every lane issues the same loads
+  // lanes whose row or column channel does not exist read channel 0, so every lane
+  // issues the same loads (the rows are scaled by zero; the columns are not kept)
   const int o_n = n >> 2;
-  float grow[MT], gcol[NT];
+  float grow[MT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt) grow[mt] = 4 * mt + o_n < a.cout ? sg : 0.f;
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) gcol[nt] = 4 * nt + o_n < a.cin ? sv : 0.f;
   const TermConst tcon = term_const(g, t);
   auto geo = [&](int grp) {
     Geo r;
@@ -843,7 +835,7 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
     }
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      const int ch = gcol[nt] != 0.f ? 4 * nt + o_n : 0;
+      const int ch = 4 * nt + o_n < a.cin ? 4 * nt + o_n : 0;
       const float4 *b = (const float4 *)chan_field(a.act, ch, ge.tg.jp, g.vh).p + ge.tg.j + (size_t)rslot * vh;
       x.v[nt][0] = b[0];
       x.v[nt][1] = b[vh];
@@ -852,20 +844,24 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
     for (int k = 0; k < 3; ++k)
       x.l[k] = ld_at<float4>(a.U.a, ((size_t)ge.tg.slab * 3 + k) * a.U.vh * 16, (unsigned)ge.tg.li * 16u);
   };
-  // the products of one group: rows x.g, columns x.v transported by u (a
-  // hop term; the site term leaves them as they are), sites weighted by keep
-  auto products = [&](const Ops &x, float keep, const cf (&u)[9]) {
+  // the products of one group: rows gv (the output gradient of channels 4 mt +
+  // n / 4, spin n % 4), columns vv (the inputs of channels 4 nt + n / 4, spin n % 4)
+  // transported by u, which carries their scale (the site term has the scale only);
+  // sites weighted by keep
+  auto products = [&](cf (&gv)[MT][3], cf (&vv)[NT][3], float keep, const cf (&u)[9]) {
     const bool hop = tcon.hop;  // uniform
-    // rows: output gradient of channels 4 mt + n / 4, spin n % 4
-    cf gv[MT][3];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) spin3(x.g[mt], keep * grow[mt], gv[mt]);
-    // columns: transported inputs of channels 4 nt + n / 4, spin n % 4
-    cf vv[NT][3];
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) gv[mt][c] = (keep * grow[mt]) * gv[mt][c];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
-      spin3(x.v[nt], gcol[nt], vv[nt]);
-      if (hop) transport1(u, vv[nt]);
+      if (hop) {
+        transport1(u, vv[nt]);
+      } else if (SPLIT) {
+#pragma unroll
+        for (int c = 0; c < 3; ++c) vv[nt][c] = sv * vv[nt][c];
+      }
     }
     if (SPLIT) {
       uint4 ah[MT], al[MT];
@@ -919,8 +915,13 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
   };
   auto compute = [&](const Ops &x, const Geo &ge) {
     cf u[9];
-    if (tcon.hop) term_matrix(x.l, 1, ge.tg.fwd, ge.tg.ph, u);
-    products(x, ge.keep, u);
+    if (tcon.hop) term_matrix(x.l, 1, ge.tg.fwd, ge.tg.ph * sv, u);
+    cf gv[MT][3], vv[NT][3];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) spin3(x.g[mt], gv[mt]);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) spin3(x.v[nt], vv[nt]);
+    products(gv, vv, ge.keep, u);
   };
   // shared memory: the staged operands of a step (LDS path), then the block
   // sum of the epilogue (after a barrier)
@@ -946,7 +947,8 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
     // sites rotated by b mod 8: a matrix-core operand is read at one site from 16
     // planes (4 channels x 4 spins) at once, which would all lie in the same banks,
     // and with the rotation 8 lanes fall on 7 or 8 of the 8 bank groups (16^3x32,
-    // 8 -> 8 channels: WGTIME).
+    // 8 -> 8 channels: 269 -> 238 us, and 219 us with the three complex
+    // numbers of a spin read as such instead of selected from two float4).
     const int fs = ((tid & 31) + (tid >> 5)) & 31;
     // the thread's six planes (separate variables: arrays of them end up in
     // scratch memory in some instances)
@@ -994,23 +996,23 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
       }
     };
     // the products of the wave's group h (0, 1) of the step
-    // float4 of site s in plane b
-    auto staged = [](const float4 *base, int b, int s) { return base[b * 32 + ((s - (b & 7)) & 31)]; };
+    // complex k of channel ch at site s
+    auto staged = [](const float4 *base, int ch, int k, int s) {
+      const int b = ch * 6 + (k >> 1);
+      const float2 v = ((const float2 *)(base + b * 32 + ((s - (b & 7)) & 31)))[k & 1];
+      return mk(v.x, v.y);
+    };
     auto group = [&](int g0, int h) {
       const int s = 16 * h + 4 * wave + q;
-      Ops x;
+      cf gv[MT][3], vv[NT][3];
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int o = grow[mt] != 0.f ? 4 * mt + o_n : 0;
-        x.g[mt][0] = staged(sG, o * 6 + rslot, s);
-        x.g[mt][1] = staged(sG, o * 6 + rslot + 1, s);
-      }
+      for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        const int ch = gcol[nt] != 0.f ? 4 * nt + o_n : 0;
-        x.v[nt][0] = staged(sV, ch * 6 + rslot, s);
-        x.v[nt][1] = staged(sV, ch * 6 + rslot + 1, s);
-      }
+        for (int c = 0; c < 3; ++c) gv[mt][c] = staged(sG, 4 * mt + o_n < a.cout ? 4 * mt + o_n : 0, 3 * rs + c, s);
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) vv[nt][c] = staged(sV, 4 * nt + o_n < a.cin ? 4 * nt + o_n : 0, 3 * rs + c, s);
       cf u[9];
       if (tcon.hop) {
 #pragma unroll
@@ -1019,7 +1021,7 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
           u[k] = mk(e.x, e.y);
         }
       }
-      products(x, (g0 + 4 * h + wave) * 4 + q < nsite ? 1.f : 0.f, u);
+      products(gv, vv, (g0 + 4 * h + wave) * 4 + q < nsite ? 1.f : 0.f, u);
     };
     int g0 = sb * 8;  // the block's first group; block-uniform, as every branch below
 #pragma unroll 1
@@ -1031,7 +1033,7 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
       __builtin_amdgcn_s_waitcnt(0);  // this wave's loads, those into LDS included, have landed
       if (linker && tcon.hop) {
         cf m[9];
-        term_matrix(raw, 1, tcon.fwd, ph, m);
+        term_matrix(raw, 1, tcon.fwd, ph * sv, m);
 #pragma unroll
         for (int k = 0; k < 9; ++k) sM[tid * 9 + k] = make_float2(m[k].re, m[k].im);
       }
