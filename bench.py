@@ -204,25 +204,23 @@ def main():
     assert all(r.converged and r.true_res <= TOL for r in lres), "learned solve did not reach 1e-10"
     log(f"learned+mixed: {t_learned * 1e3:.1f} ms {lres[-1]}")
 
-    # roofline of the dominant kernel of the timed solve: the network's second
-    # layer as the preconditioner runs it (k_net_second<8, true>): its even
-    # outputs from the one-channel input with combined matrices, its odd
-    # outputs from the first layer's even sites and the input, and in its
-    # epilogue the last layer's term fields for the third layer's odd sites;
-    # split FP16 on the matrix cores, timed with HIP events on the stream it
-    # runs on.  Its bound is memory: the compulsory bytes are the input's odd
-    # sites, the first layer's 8 channels at even sites, the FP32 links once,
-    # its 8 output channels (both parities) and the 9 term fields it writes;
-    # the measured traffic (profiles/) shows the neighbour channels re-read.
+    # roofline of the dominant kernel of the timed solve: the network's third and
+    # last layers as one composed step of the preconditioner (k_net_second<8, 2>):
+    # the last layer's 8 hop fields at even sites from the second layer's odd
+    # sites and the one-channel input; split FP16 on the matrix cores, timed with
+    # HIP events on the stream it runs on.  Its bound is memory: the compulsory
+    # bytes are the input's odd sites, the second layer's 8 channels at odd sites,
+    # the FP32 links once and the 8 fields it writes; the measured traffic
+    # (profiles/) shows the neighbour channels re-read.
     stages = [net.bench_precond_layer(k, iters=10) for k in range(4)]
-    ms_second = stages[1]
-    second_bytes = (96 + 8 * 96 + 8 * 48 + 2 * 8 * 96 + 9 * 96) * vh
-    second_GBps = second_bytes / (ms_second * 1e-3) / 1e9
-    second_traffic = traffic_of(SECOND_TRAFFIC)
-    # executed v_mfma_f32_32x32x16_f16 (32768 flops each) per 32 sites of
-    # both parities: even pass 4 K steps, odd pass 33, 6 products each per
-    # M tile pair x 3 colours (18 per K step), epilogue 72 + 36
-    second_mfma_flops = (4 * 18 + 33 * 18 + 72 + 36) * 32768 // 32 * vh
+    ms_tail = stages[2]
+    tail_bytes = (96 + 8 * 96 + 8 * 48 + 8 * 96) * vh
+    tail_GBps = tail_bytes / (ms_tail * 1e-3) / 1e9
+    tail_traffic = traffic_of(SECOND_TRAFFIC)
+    # executed v_mfma_f32_32x32x16_f16 (32768 flops each) per 32 even sites: 4 K
+    # steps of the input and 32 of the channels, 6 products each per M tile pair x
+    # 3 colours (18 per K step)
+    tail_mfma_flops = (4 * 18 + 32 * 18) * 32768 // 32 * vh
     # the plain 8 -> 8 layer (training's forward pass; every 8 -> 8 layer outside the preconditioner)
     ms_layer, fl_layer = net.bench_layer(1, iters=10)
     layer_bytes = 8 * 2 * vh * 96 * 2 + 8 * vh * 48
@@ -291,21 +289,21 @@ def main():
                      "pairs": "plain FP64 BiCGSTAB to 1e-8" if sol_pairs else None,
                      "epochs": args.train_epochs, "batch": args.train_batch,
                      "loss_first_epoch": float(losses[0]), "loss_last_epoch": float(losses[-1])},
-        "roofline": {"kernel": "network layer 2 as the preconditioner runs it (k_net_second<8, true>)",
+        "roofline": {"kernel": "network layers 3 and 4 as one step of the preconditioner (k_net_second<8, 2>)",
                      "bound": "hbm",
                      "compute": "v_mfma_f32_32x32x16_f16, FP32 operands split into FP16 hi + lo, three products "
                                 "accumulated in FP32 (FP32-accurate)",
-                     "bytes_count": "compulsory: the input's odd sites, layer 1's 8 channels at even sites, FP32 "
-                                    "links once, 8 output channels (both parities), the 9 term fields written",
-                     "achieved": round(second_GBps, 1), "peak": PEAK_GBS, "unit": "GB/s",
-                     "frac": round(second_GBps / PEAK_GBS, 3), "traffic": second_traffic,
-                     "traffic_GBps": None if second_traffic is None else
-                     round(second_traffic / (ms_second * 1e-3) / 1e9, 1),
-                     "ms_per_launch": round(ms_second, 4), "alg_bytes_per_launch": second_bytes,
-                     "fp16_mfma_TFLOPs": round(second_mfma_flops / (ms_second * 1e-3) / 1e12, 1),
-                     "fp16_mfma_frac": round(second_mfma_flops / (ms_second * 1e-3) / 1e12 / PEAK_FP16_TFLOPS, 3)},
-        "precond_layer_ms": {"layer1_first": round(stages[0], 4), "layer2_second": round(stages[1], 4),
-                             "layer3_fused_even_sites": round(stages[2], 4), "layer4_gather": round(stages[3], 4)},
+                     "bytes_count": "compulsory: the input's odd sites, layer 2's 8 channels at odd sites, FP32 "
+                                    "links once, the 8 term fields written",
+                     "achieved": round(tail_GBps, 1), "peak": PEAK_GBS, "unit": "GB/s",
+                     "frac": round(tail_GBps / PEAK_GBS, 3), "traffic": tail_traffic,
+                     "traffic_GBps": None if tail_traffic is None else
+                     round(tail_traffic / (ms_tail * 1e-3) / 1e9, 1),
+                     "ms_per_launch": round(ms_tail, 4), "alg_bytes_per_launch": tail_bytes,
+                     "fp16_mfma_TFLOPs": round(tail_mfma_flops / (ms_tail * 1e-3) / 1e12, 1),
+                     "fp16_mfma_frac": round(tail_mfma_flops / (ms_tail * 1e-3) / 1e12 / PEAK_FP16_TFLOPS, 3)},
+        "precond_layer_ms": {"layer1_first": round(stages[0], 4), "layer2_odd_sites": round(stages[1], 4),
+                             "layers3_4_composed": round(stages[2], 4), "layer4_gather": round(stages[3], 4)},
         "layer_8x8_plain": {"kernel": "network layer 8->8 channels (k_net_layer_split<32, 8, 2>)", "bound": "hbm",
                      "compute": "v_mfma_f32_32x32x16_f16, FP32 operands split into FP16 hi + lo, three products "
                                 "accumulated in FP32 (FP32-accurate)",

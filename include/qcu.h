@@ -103,7 +103,8 @@ int qcuDslash(QcuLatticeHandle h, void *out, const void *in, int parity, int clo
 /* qcuDslash without any allocation: no counterpart in the reference; for
  * callers that cannot allocate device memory (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  Same arguments and
- * result as qcuDslash.  The two staged half spinors live in a 32 MiB device
+ * result as qcuDslash.  The staged half spinors (FP64: a copy of an input that
+ * overlaps the output, and nothing else) live in a 32 MiB device
  * array of the library (one per GPU, held until the process ends), so the
  * lattice must satisfy 2 x Vh x (192 bytes FP64, 96 FP32, 52 FP16, each
  * rounded up to 256 bytes) <= 32 MiB (e.g. 16^3x32 in FP64); larger ones are
@@ -120,7 +121,8 @@ typedef struct QcuSolveParam_s {
   int max_iter;          /* BiCGSTAB iterations (sloppy iterations count) */
   int precision;         /* QCU_PREC_*: inner (sloppy) precision */
   double reliable_delta; /* reliable update when |r| < delta |r_last_update| */
-  int chunk;             /* iterations between host checks (graph length); 0: 8, or 4 with precond */
+  int chunk;             /* iterations between host checks (graph length); 0: at most 8, or 4 with precond,
+                            and fewer where the residual's pace brings the next check sooner */
   int use_graph;         /* capture the chunk as a hipGraph and replay it */
   void *precond;         /* QcuNetHandle or NULL */
   int legacy_stop;       /* 1: stop on Re<r,r> < tol absolute (reference rule) */
