@@ -36,6 +36,14 @@ struct QcuBatch_s {
 
 namespace qcu {
 
+int wait_null_stream() {
+  const hipError_t e = hipStreamQuery(nullptr);
+  if (e == hipSuccess) return 0;
+  (void)hipGetLastError();
+  if (e == hipErrorNotReady) QCU_HIP(hipStreamSynchronize(nullptr));
+  return 0;
+}
+
 int check_dev_ptr(const void *p, const char *what) {
   if (!p) {
     set_error(QCU_ERR_ARG, std::string(what) + " is null");
@@ -195,6 +203,7 @@ int legacy_dslash(void *out, void *in, void *gauge, QcuParam *param, int parity,
   QCU_TRY(check_dev_ptr(out, "fermion_out"));
   QCU_TRY(check_dev_ptr(in, "fermion_in"));
   QCU_TRY(check_dev_ptr(gauge, "gauge"));
+  QCU_TRY(wait_null_stream());
   std::lock_guard<std::mutex> lk(g_legacy_mu);
   int rc = 0;
   Legacy *L = legacy_ctx(param, clover, &rc);
@@ -231,6 +240,7 @@ int legacy_bicgstab(void *x, void *b, void *gauge, QcuParam *param) {
   QCU_TRY(check_dev_ptr(x, "fermion_out"));
   QCU_TRY(check_dev_ptr(b, "fermion_in"));
   QCU_TRY(check_dev_ptr(gauge, "gauge"));
+  QCU_TRY(wait_null_stream());
   std::lock_guard<std::mutex> lk(g_legacy_mu);
   int rc = 0;
   Legacy *L = legacy_ctx(param, 0, &rc);
@@ -317,6 +327,7 @@ int qcuLatticeLoadGauge(QcuLatticeHandle h, const void *gauge) {
   clear_error();
   QCU_CHECK(h, QCU_ERR_ARG, "null handle");
   QCU_TRY(check_dev_ptr(gauge, "gauge"));
+  QCU_TRY(wait_null_stream());
   return h->lat.load_gauge(gauge, 7);
 }
 
@@ -355,6 +366,7 @@ int qcuDslash(QcuLatticeHandle h, void *out, const void *in, int parity, int clo
   QCU_CHECK(!clover || lat.has_clover(), QCU_ERR_STATE, "lattice has no clover term (csw = 0)");
   QCU_TRY(check_dev_ptr(out, "out"));
   QCU_TRY(check_dev_ptr(in, "in"));
+  QCU_TRY(wait_null_stream());
   if (prec == P64) return direct_op(lat, out, in, half_bytes(lat), parity, 0, clover != 0, nullptr);
   for (Spinor &v : lat.stage) QCU_TRY(v.create(prec, lat.g.vh));
   return staged_op(lat, out, in, parity, prec, clover != 0, lat.stage[0].ptr(), lat.stage[1].ptr());
@@ -435,6 +447,7 @@ int qcuMatFull(QcuLatticeHandle h, void *out, const void *in) {
   QCU_CHECK(lat.gauge_loaded, QCU_ERR_STATE, "gauge field not loaded");
   QCU_TRY(check_dev_ptr(out, "out"));
   QCU_TRY(check_dev_ptr(in, "in"));
+  QCU_TRY(wait_null_stream());
   return direct_op(lat, out, in, 2 * half_bytes(lat), 0, 1, lat.has_clover(), nullptr);
 }
 
@@ -445,6 +458,7 @@ int qcuTrueResidual(QcuLatticeHandle h, const void *x, const void *b, double *re
   QCU_CHECK(lat.gauge_loaded, QCU_ERR_STATE, "gauge field not loaded");
   QCU_TRY(check_dev_ptr(x, "x"));
   QCU_TRY(check_dev_ptr(b, "b"));
+  QCU_TRY(wait_null_stream());
   Solver *S = nullptr;
   QCU_TRY(lattice_solver(lat, &S));
   const void *xs[1] = {x}, *bs[1] = {b};
@@ -459,6 +473,7 @@ int qcuSolve(QcuLatticeHandle h, void *x, const void *b, const QcuSolveParam *p,
   QCU_TRY(check_method(p));
   QCU_TRY(check_dev_ptr(x, "x"));
   QCU_TRY(check_dev_ptr(b, "b"));
+  QCU_TRY(wait_null_stream());
   Lattice &lat = h->lat;
   QCU_CHECK(lat.gauge_loaded, QCU_ERR_STATE, "gauge field not loaded");
   QCU_CHECK((lat.prec_mask >> p->precision) & 1, QCU_ERR_STATE, "links of the requested precision are not resident");
@@ -535,6 +550,7 @@ int qcuBatchSolve(QcuBatchHandle h, void *const *x, const void *const *b, const 
     QCU_TRY(check_dev_ptr(x[k], "x"));
     QCU_TRY(check_dev_ptr(b[k], "b"));
   }
+  QCU_TRY(wait_null_stream());
   std::vector<QcuSolveInfo> tmp(h->op.nsys);
   return full_solve(h->solver, x, b, *p, info ? info : tmp.data());
 }

@@ -2193,6 +2193,7 @@ int qcuNetForward(QcuNetHandle h, void *out, const void *in) {
   QCU_CHECK(h, QCU_ERR_ARG, "null handle");
   QCU_TRY(check_dev_ptr(out, "out"));
   QCU_TRY(check_dev_ptr(in, "in"));
+  QCU_TRY(wait_null_stream());
   Net &net = h->net;
   QCU_TRY(net_ready(net));
   hipStream_t s = net.lat->stream;
@@ -2218,6 +2219,7 @@ int qcuNetBackward(QcuNetHandle h, void *grad_in, const void *grad_out, const vo
   QCU_TRY(check_dev_ptr(grad_out, "grad_out"));
   QCU_TRY(check_dev_ptr(in, "in"));
   if (grad_in) QCU_TRY(check_dev_ptr(grad_in, "grad_in"));
+  QCU_TRY(wait_null_stream());
   Net &net = h->net;
   QCU_TRY(net_ready(net));
   hipStream_t s = net.lat->stream;
@@ -2257,6 +2259,7 @@ int qcuNetTrain(QcuNetHandle h, const void *const *srcs, int n, int epochs, int 
   clear_error();
   QCU_CHECK(h && srcs && n > 0 && epochs > 0 && batch > 0, QCU_ERR_ARG, "bad training arguments");
   for (int k = 0; k < n; ++k) QCU_TRY(check_dev_ptr(srcs[k], "srcs[k]"));
+  QCU_TRY(wait_null_stream());
   Net &net = h->net;
   QCU_TRY(net_ready(net));
   Lattice &lat = *net.lat;
@@ -2305,6 +2308,7 @@ int qcuNetApplyOdd(QcuNetHandle h, void *out, const void *in) {
   QCU_CHECK(h, QCU_ERR_ARG, "null handle");
   QCU_TRY(check_dev_ptr(out, "out"));
   QCU_TRY(check_dev_ptr(in, "in"));
+  QCU_TRY(wait_null_stream());
   Net &net = h->net;
   QCU_TRY(net_ready(net));
   hipStream_t s = net.lat->stream;
@@ -2327,6 +2331,7 @@ int qcuNetLossGrad(QcuNetHandle h, const void *src, double *loss) {
   clear_error();
   QCU_CHECK(h && loss, QCU_ERR_ARG, "null argument");
   QCU_TRY(check_dev_ptr(src, "src"));
+  QCU_TRY(wait_null_stream());
   Net &net = h->net;
   QCU_TRY(net_ready(net));
   hipStream_t s = net.lat->stream;
@@ -2567,6 +2572,7 @@ int qcuNetLoss(QcuNetHandle h, const void *const *srcs, int n, double *loss) {
   clear_error();
   QCU_CHECK(h && srcs && n > 0 && loss, QCU_ERR_ARG, "bad arguments");
   for (int k = 0; k < n; ++k) QCU_TRY(check_dev_ptr(srcs[k], "srcs[k]"));
+  QCU_TRY(wait_null_stream());
   Net &net = h->net;
   QCU_TRY(net_ready(net));
   hipStream_t s = net.lat->stream;

@@ -66,6 +66,9 @@ unsigned long long tune_generation();
 
 // 0 when p is a HIP device (or managed) pointer; else records the error
 int check_dev_ptr(const void *p, const char *what);
+// Waits for work queued on the null stream, the default stream of most callers: the
+// library's streams do not wait for it, and it may be writing a call's inputs.
+int wait_null_stream();
 
 // the preconditioner behind a QcuNetHandle; it must belong to lattice lat
 int net_precond(void *handle, const Lattice *lat, Precond **out);
