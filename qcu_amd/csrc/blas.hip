@@ -149,6 +149,11 @@ __global__ void __launch_bounds__(256) k_bicg_init(SpinorPtr r, SpinorPtr rt, Sp
   block_partial_rhs<1>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
+// The iterate, which nothing else in an iteration touches, and t and v at their last
+// use are non-temporal, so that they do not displace the vectors that the next
+// kernel reads (24^3x48 FP64 solve 16.7 -> 16.3 ms, 32^3x64 56.1 -> 55.4, 12 right-hand
+// sides of 24^3x48 FP32 90.4 -> 89.7; 16^3x32 unchanged).
+
 // p = r + beta (p - omega v)
 template <int P>
 __global__ void __launch_bounds__(256) k_p_update(SpinorPtr p, SpinorPtr r, SpinorPtr v, const SegDesc *segs, int nseg, const SysState *st) {
@@ -159,7 +164,7 @@ __global__ void __launch_bounds__(256) k_p_update(SpinorPtr p, SpinorPtr r, Spin
   cplx<T> pp[12], rr[12], vv[12];
   SpinorIO<P>::load(view<P>(p, c), c.t, pp);
   SpinorIO<P>::load(view<P>(r, c), c.t, rr);
-  SpinorIO<P>::load(view<P>(v, c), c.t, vv);
+  SpinorIO<P>::template load<true>(view<P>(v, c), c.t, vv);
 #pragma unroll
   for (int k = 0; k < 12; ++k) pp[k] = rr[k] + beta * (pp[k] - omega * vv[k]);
   SpinorIO<P>::store(view<P>(p, c), c.t, pp);
@@ -194,9 +199,9 @@ __global__ void __launch_bounds__(256) k_xr_update(SpinorPtr x, SpinorPtr r, Spi
     cplx<T> pp[12], ss[12], tt[12];
     SpinorIO<P>::load(view<P>(p, c), c.t, pp);
     SpinorIO<P>::load(view<P>(s, c), c.t, ss);
-    SpinorIO<P>::load(view<P>(t, c), c.t, tt);
+    SpinorIO<P>::template load<true>(view<P>(t, c), c.t, tt);
     cplx<TX> xx[12];
-    SpinorIO<Px>::load(view<Px>(x, c), c.t, xx);
+    SpinorIO<Px>::template load<true>(view<Px>(x, c), c.t, xx);
     const cplx<TX> al = cs<TX>(st[c.sys].alpha), omx = cs<TX>(st[c.sys].omega);
     if (PC) {
       cplx<T> sh[12];
@@ -213,7 +218,7 @@ __global__ void __launch_bounds__(256) k_xr_update(SpinorPtr x, SpinorPtr r, Spi
         xx[k] = xx[k] + al * pk + omx * sk;
       }
     }
-    SpinorIO<Px>::store(view<Px>(x, c), c.t, xx);
+    SpinorIO<Px>::template store<true>(view<Px>(x, c), c.t, xx);
     const cplx<T> om = cs<T>(st[c.sys].omega);
     cplx<T> rtt[12];
     SpinorIO<P>::load(view<P>(rt, c), c.t, rtt);

@@ -173,12 +173,14 @@ QCU_D V ld_at(const void *base, size_t comp_bytes, unsigned lane_off) {
   __builtin_memcpy(&v, &w, sizeof(V));
   return v;
 }
-template <class V>
+template <class V, bool NT = false>
 QCU_D void st_at(void *base, size_t comp_bytes, unsigned lane_off, const V &v) {
   typedef unsigned words __attribute__((ext_vector_type(sizeof(V) / 4)));
   words w;
   __builtin_memcpy(&w, &v, sizeof(V));
-  *(QCU_GLOBAL words *)((QCU_GLOBAL char *)base + comp_bytes + lane_off) = w;
+  QCU_GLOBAL words *p = (QCU_GLOBAL words *)((QCU_GLOBAL char *)base + comp_bytes + lane_off);
+  if (NT) __builtin_nontemporal_store(w, p);
+  else *p = w;
 }
 // the same as a non-temporal store: for fields written once and read by a
 // later kernel (the network's activations and term fields), which then need
@@ -223,38 +225,42 @@ struct SpinorIO;
 template <>
 struct SpinorIO<P64> {
   typedef double real;
+  template <bool NT = false>
   static QCU_D void load(const SpinorPtr &f, int i, cplx<double> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 12; ++k) {
-      double2 a = ld_at<double2>(f.p, (size_t)k * f.stride * 16, off);
+      double2 a = ld_at<double2, NT>(f.p, (size_t)k * f.stride * 16, off);
       v[k] = mk(a.x, a.y);
     }
   }
+  template <bool NT = false>
   static QCU_D void store(const SpinorPtr &f, int i, const cplx<double> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
-    for (int k = 0; k < 12; ++k) st_at<double2>(f.p, (size_t)k * f.stride * 16, off, make_double2(v[k].re, v[k].im));
+    for (int k = 0; k < 12; ++k) st_at<double2, NT>(f.p, (size_t)k * f.stride * 16, off, make_double2(v[k].re, v[k].im));
   }
 };
 
 template <>
 struct SpinorIO<P32> {
   typedef float real;
+  template <bool NT = false>
   static QCU_D void load(const SpinorPtr &f, int i, cplx<float> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      float4 a = ld_at<float4>(f.p, (size_t)k * f.stride * 16, off);
+      float4 a = ld_at<float4, NT>(f.p, (size_t)k * f.stride * 16, off);
       v[2 * k] = mk(a.x, a.y);
       v[2 * k + 1] = mk(a.z, a.w);
     }
   }
+  template <bool NT = false>
   static QCU_D void store(const SpinorPtr &f, int i, const cplx<float> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
 #pragma unroll
     for (int k = 0; k < 6; ++k)
-      st_at<float4>(f.p, (size_t)k * f.stride * 16, off,
+      st_at<float4, NT>(f.p, (size_t)k * f.stride * 16, off,
                     make_float4(v[2 * k].re, v[2 * k].im, v[2 * k + 1].re, v[2 * k + 1].im));
   }
 };
@@ -285,12 +291,13 @@ struct SpinorIO<P16> {
 #pragma unroll
     for (int k = 0; k < 12; ++k) v[k] = mk(m * h2f(f2h(v[k].re * inv)), m * h2f(f2h(v[k].im * inv)));
   }
+  template <bool NT = false>
   static QCU_D void load(const SpinorPtr &f, int i, cplx<float> (&v)[12]) {
     const unsigned off = (unsigned)i * 16u;
-    const float nrm = ld_at<float>(f.norm, 0, (unsigned)i * 4u);
+    const float nrm = ld_at<float, NT>(f.norm, 0, (unsigned)i * 4u);
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      uint4 a = ld_at<uint4>(f.p, (size_t)k * f.stride * 16, off);
+      uint4 a = ld_at<uint4, NT>(f.p, (size_t)k * f.stride * 16, off);
       unsigned w[4] = {a.x, a.y, a.z, a.w};
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
