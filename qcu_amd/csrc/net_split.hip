@@ -1236,62 +1236,55 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
 //   C[u][t][i] = W4_t W3_u          (u, t = 0..7; u = 8: zero)
 //   G[u][t][0] = (W4_t W3_8 + W4_8 W3_t) (W2_u W1_8 + W2_8 W1_u)   (u = 8: zero)
 //   S[8][0][i] = W4_8 W3_8          (other terms zero)
-// FP64 sums, rounded to FP32.  Block u forms the matrices of term u.
-__global__ void __launch_bounds__(256) k_net_compose_tail(const float2 *W1, const float2 *W2, const float2 *W3,
+// FP64 sums, rounded to FP32.  Block (u, t) forms the matrices of that pair of terms,
+// one entry of each sum per thread: 8 us.
+__global__ void __launch_bounds__(128) k_net_compose_tail(const float2 *W1, const float2 *W2, const float2 *W3,
                                                           const float2 *W4, float2 *C, float2 *G, float2 *S) {
-  __shared__ double2 M[8 * 8 * 16], E[8 * 16];
-  const int u = blockIdx.x, tid = threadIdx.x;
+  __shared__ double2 M[8 * 16], E[8 * 16];
+  const int u = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
+  const int i = tid >> 4, s = (tid >> 2) & 3, s2 = tid & 3;
   // sum_j sum_sp A[j][s][sp] B[j][sp][s2], j strides as and bs (in spin matrices)
-  auto mul = [](const float2 *A, int as, const float2 *B, int bs, int s, int s2, double2 &r) {
+  auto mul = [&](const float2 *A, int as, const float2 *B, int bs, double2 &r) {
+#pragma unroll
     for (int j = 0; j < 8; ++j)
+#pragma unroll
       for (int sp = 0; sp < 4; ++sp) {
         const float2 x = A[(size_t)j * as * 16 + s * 4 + sp], y = B[(size_t)j * bs * 16 + sp * 4 + s2];
         r.x += (double)x.x * y.x - (double)x.y * y.y;
         r.y += (double)x.x * y.y + (double)x.y * y.x;
       }
   };
-  auto w3 = [&](int t, int i) { return W3 + ((size_t)t * 64 + i) * 16; };  // outputs j: stride 8
-  auto w4 = [&](int t) { return W4 + (size_t)t * 8 * 16; };                // inputs j: stride 1
-  auto f32 = [](double2 v) { return make_float2((float)v.x, (float)v.y); };
-  for (int e = tid; e < 8 * 8 * 16; e += 256) {
-    const int t = e >> 7, i = (e >> 4) & 7, s = (e >> 2) & 3, s2 = e & 3;
-    double2 c = make_double2(0.0, 0.0), m = c;
-    if (u < 8) {
-      mul(w4(t), 1, w3(u, i), 8, s, s2, c);
-      mul(w4(t), 1, w3(8, i), 8, s, s2, m);
-      mul(w4(8), 1, w3(t, i), 8, s, s2, m);
-    }
-    M[e] = m;
-    C[(size_t)u * 1024 + e] = f32(c);
+  auto w3 = [&](int v) { return W3 + ((size_t)v * 64 + i) * 16; };  // outputs j: stride 8
+  auto w4 = [&](int v) { return W4 + (size_t)v * 8 * 16; };         // inputs j: stride 1
+  double2 c = make_double2(0.0, 0.0), m = c, v = c, w = c;
+  if (u < 8) {
+    mul(w4(t), 1, w3(u), 8, c);
+    mul(w4(t), 1, w3(8), 8, m);
+    mul(w4(8), 1, w3(t), 8, m);
+    mul(W2 + ((size_t)u * 64 + i * 8) * 16, 1, W1 + (size_t)8 * 8 * 16, 1, v);
+    mul(W2 + ((size_t)8 * 64 + i * 8) * 16, 1, W1 + (size_t)u * 8 * 16, 1, v);
+  } else if (t == 0) {
+    mul(w4(8), 1, w3(8), 8, w);
   }
-  if (tid < 8 * 16) {
-    const int i = tid >> 4, s = (tid >> 2) & 3, s2 = tid & 3;
-    double2 v = make_double2(0.0, 0.0), w = v;
-    if (u < 8) {
-      mul(W2 + ((size_t)u * 64 + i * 8) * 16, 1, W1 + (size_t)8 * 8 * 16, 1, s, s2, v);
-      mul(W2 + ((size_t)8 * 64 + i * 8) * 16, 1, W1 + (size_t)u * 8 * 16, 1, s, s2, v);
-    } else {
-      mul(w4(8), 1, w3(8, i), 8, s, s2, w);
-    }
-    E[tid] = v;
-    S[(size_t)u * 128 + tid] = f32(w);
-  }
+  C[((size_t)u * 8 + t) * 128 + tid] = make_float2((float)c.x, (float)c.y);
+  if (t == 0) S[(size_t)u * 128 + tid] = make_float2((float)w.x, (float)w.y);
+  M[tid] = m;
+  E[tid] = v;
   __syncthreads();
-  if (tid < 8 * 16) {
-    const int t = tid >> 4, s = (tid >> 2) & 3, s2 = tid & 3;
-    double2 v = make_double2(0.0, 0.0);
-    for (int i = 0; i < 8; ++i)
+  if (tid < 16) {
+    double2 g = make_double2(0.0, 0.0);
+    for (int k = 0; k < 8; ++k)
       for (int sp = 0; sp < 4; ++sp) {
-        const double2 x = M[(t * 8 + i) * 16 + s * 4 + sp], y = E[i * 16 + sp * 4 + s2];
-        v.x += x.x * y.x - x.y * y.y;
-        v.y += x.x * y.y + x.y * y.x;
+        const double2 x = M[k * 16 + s * 4 + sp], y = E[k * 16 + sp * 4 + s2];
+        g.x += x.x * y.x - x.y * y.y;
+        g.y += x.x * y.y + x.y * y.x;
       }
-    G[(size_t)u * 128 + tid] = f32(v);
+    G[((size_t)u * 8 + t) * 16 + tid] = make_float2((float)g.x, (float)g.y);
   }
 }
 
 int net_compose_tail(const float2 *const (&W)[4], float2 *C, float2 *G, float2 *S, hipStream_t s) {
-  hipLaunchKernelGGL(k_net_compose_tail, dim3(9), dim3(256), 0, s, W[0], W[1], W[2], W[3], C, G, S);
+  hipLaunchKernelGGL(k_net_compose_tail, dim3(9, 8), dim3(128), 0, s, W[0], W[1], W[2], W[3], C, G, S);
   QCU_HIP(hipGetLastError());
   return 0;
 }
