@@ -6,6 +6,7 @@
 // The reference converts in place through a temporary and cuBLAS copies
 // (src/lattice_cuda.cu:41-211); here the caller's buffers are only read (or
 // only written), and the internal copies stay resident.
+#include "qcu_hash.h"
 #include "qcu_internal.h"
 
 namespace qcu {
@@ -13,19 +14,10 @@ namespace qcu {
 // ---- content hash of an external gauge field -------------------------------
 // A 64-bit summary of every bit of the field, position-dependent, used by the
 // reference-named entry points to keep converted links and the clover term
-// while the caller's gauge is unchanged.  Each complex entry k with bit
-// patterns (a, b) is mixed with k and the mixed words are added modulo 2^64;
-// addition commutes, so the result does not depend on the block order, and a
-// load of the field forms it on the way.
-QCU_D unsigned long long hash_mix(unsigned long long a, unsigned long long b, unsigned long long k) {
-  unsigned long long x = a * 0x9E3779B97F4A7C15ull + b * 0xC2B2AE3D27D4EB4Full + k * 0x165667B19E3779F9ull;
-  x ^= x >> 29;
-  x *= 0xBF58476D1CE4E5B9ull;
-  x ^= x >> 32;
-  x *= 0x94D049BB133111EBull;
-  return x ^ (x >> 29);
-}
-
+// while the caller's gauge is unchanged.  Each complex entry k is mixed with k
+// (qcu_hash.h) and the mixed words are added modulo 2^64; addition commutes, so
+// the result does not depend on the block order, and a load of the field forms it
+// on the way.
 QCU_D unsigned long long hash_entry(double2 v, long k) {
   return hash_mix((unsigned long long)__double_as_longlong(v.x), (unsigned long long)__double_as_longlong(v.y),
                   (unsigned long long)k);
