@@ -497,6 +497,7 @@ int qcuBenchHop(QcuLatticeHandle h, int prec, int clover, int xpay, int iters, i
   Lattice &lat = h->lat;
   QCU_CHECK(lat.gauge_loaded, QCU_ERR_STATE, "gauge field not loaded");
   QCU_CHECK(!clover || lat.has_clover(), QCU_ERR_STATE, "lattice has no clover term");
+  QCU_CHECK(prec >= 0 && prec <= 2, QCU_ERR_ARG, "bad precision");
   LaunchCfg cfg = tuned_cfg(lat.self, prec);
   if (block > 0) cfg.block = block;
   if (remap >= 0) cfg.remap = remap;
@@ -558,6 +559,7 @@ int qcuBatchSolve(QcuBatchHandle h, void *const *x, const void *const *b, const 
 int qcuBatchBenchHop(QcuBatchHandle h, int prec, int xpay, int iters, double *ms) {
   clear_error();
   QCU_CHECK(h && ms, QCU_ERR_ARG, "null argument");
+  QCU_CHECK(prec >= 0 && prec <= 2, QCU_ERR_ARG, "bad precision");
   return bench_hop(h->op, h->stream, prec, h->op.has_clover, xpay, iters, tuned_cfg(h->op, prec), ms);
 }
 

@@ -102,6 +102,7 @@ static LaunchCfg find_cfg(const BatchOp &op, int prec) {
 }
 
 LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
+  if (prec < P64 || prec > P16) return LaunchCfg();  // no such shape: hop() refuses the precision
   const unsigned long long gen = tune_generation();
   if (op.cfg_gen[prec] != gen) {
     op.cfg[prec] = find_cfg(op, prec);
@@ -227,6 +228,7 @@ int qcuBatchTuneSet(QcuBatchHandle h, int prec, int block, int remap, int group)
 int qcuTuneGet(QcuLatticeHandle h, int prec, int *block, int *remap, int *group) {
   clear_error();
   QCU_CHECK(h && block && remap && group, QCU_ERR_ARG, "null argument");
+  QCU_CHECK(prec >= 0 && prec <= 2, QCU_ERR_ARG, "bad precision");
   LaunchCfg c = tuned_cfg(h->lat.self, prec);
   *block = c.block;
   *remap = c.remap;
