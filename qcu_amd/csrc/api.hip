@@ -130,6 +130,7 @@ size_t half_bytes(const Lattice &lat) { return (size_t)lat.g.vh * 12 * 16; }
 struct Legacy {
   Lattice lat;
   DevBuf hash_buf;                     // scratch of the gauge hash
+  DevBuf gate;                         // state that holds an operator back from a changed gauge
   unsigned long long *now = nullptr;   // hash of the caller's gauge (pinned host memory)
   const void *gauge = nullptr;         // caller's gauge of the resident links (null: none)
   unsigned long long hash = 0;         // its content hash
@@ -143,9 +144,10 @@ struct Legacy {
 // pointer with the same contents: a 64-bit hash of the field, one read of it,
 // decides; any change of pointer or contents reloads.  A load forms the hash on
 // the way; for a known pointer the hash runs ahead of the operator, which is
-// applied at once and repeated if the contents turn out to have changed.  16^3x32,
-// two gauges in turn and both parities: 336 us a round with the host waiting for
-// each hash and each step of a load, 262 us with one wait per call.
+// launched at once and writes nothing if the contents turn out to have changed (the
+// output stays as it is should the reload fail).  16^3x32, two gauges in turn and
+// both parities: 336 us a round with the host waiting for each hash and each step of
+// a load, 262 us with one wait per call.
 int legacy_reload(Legacy &L, const void *gauge) {
   L.gauge = nullptr;  // invalid until the reload succeeds
   QCU_TRY(L.lat.load_gauge(gauge, 1, (unsigned long long *)L.hash_buf.p, L.now));
@@ -167,7 +169,7 @@ int legacy_check(Legacy &L, bool *changed) {
 int legacy_load_gauge(Legacy &L, const void *gauge) {
   if (legacy_known(L, gauge)) {
     bool changed = false;
-    QCU_TRY(gauge_hash(gauge, L.lat.g, L.hash_buf.p, L.now, L.lat.stream));
+    QCU_TRY(gauge_hash(gauge, L.lat.g, L.hash_buf.p, L.now, L.hash, (SysState *)L.gate.p, L.lat.stream));
     QCU_TRY(legacy_check(L, &changed));
     if (!changed) return 0;
   }
@@ -187,6 +189,7 @@ Legacy *legacy_ctx(const QcuParam *param, int kind, int *rc) {
   std::unique_ptr<Legacy> l(new Legacy());
   *rc = kind == 0 ? l->lat.init(param->lattice_size, 0.125, 0.0, 1) : l->lat.init(param->lattice_size, 1.0, 1.0, 1);
   if (!*rc) *rc = l->hash_buf.alloc(gauge_hash_scratch_bytes(l->lat.g));
+  if (!*rc) *rc = l->gate.alloc(sizeof(SysState));
   if (!*rc && hipHostMalloc((void **)&l->now, sizeof(*l->now), hipHostMallocDefault) != hipSuccess) {
     set_error(QCU_ERR_ALLOC, "hipHostMalloc failed");
     *rc = QCU_ERR_ALLOC;
@@ -212,10 +215,11 @@ int legacy_dslash(void *out, void *in, void *gauge, QcuParam *param, int parity,
   const size_t half = half_bytes(lat), field = (size_t)lat.g.vh * 72 * 16;
   const bool apart = !overlap(out, half, in, half) && !overlap(out, half, gauge, field);
   if (legacy_known(*L, gauge) && apart) {
-    // the operator does not wait for the hash
+    // the host does not wait between the hash and the operator
     bool changed = false;
-    QCU_TRY(gauge_hash(gauge, lat.g, L->hash_buf.p, L->now, lat.stream));
-    QCU_TRY(hop_ext(lat.self, out, in, parity, 0, clover != 0, lat.stream));
+    SysState *gate = (SysState *)L->gate.p;
+    QCU_TRY(gauge_hash(gauge, lat.g, L->hash_buf.p, L->now, L->hash, gate, lat.stream));
+    QCU_TRY(hop_ext(lat.self, out, in, parity, 0, clover != 0, lat.stream, gate));
     QCU_TRY(legacy_check(*L, &changed));
     if (!changed) return 0;
     QCU_TRY(legacy_reload(*L, gauge));

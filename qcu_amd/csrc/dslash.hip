@@ -28,7 +28,7 @@ struct HopKArgs {
   int nseg;
   int parity;
   int remap;
-  SysState *st;  // per-system states, or null
+  const SysState *st;  // per-system states, or null
   double *partials;
 };
 
@@ -440,7 +440,8 @@ int hop_split_red(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, Spin
                      : dispatch<P32>(a, nb, op.has_clover, EPI_XPAY, red, true, false, cfg, s);
 }
 
-int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s) {
+int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s,
+            const SysState *gate) {
   QCU_CHECK(op.segs.size() == 1 && op.nsys == 1, QCU_ERR_ARG, "external fields: one lattice, one right-hand side");
   LaunchCfg cfg = tuned_cfg(op, P64);
   QCU_TRY(check_cfg(cfg));
@@ -451,6 +452,7 @@ int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, b
   a.nseg = 1;
   a.parity = parity;
   a.remap = cfg.remap;
+  a.st = gate;
   const int clover = use_clover && op.has_clover;
   const bool split = hop_is_split(op, cfg), nt = use_nt(op, P64, clover);
   const int nb = total_blocks(op.segs, split ? kSplitSites : cfg.block) * (mat ? 2 : 1);

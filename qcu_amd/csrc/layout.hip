@@ -45,25 +45,32 @@ __global__ void __launch_bounds__(256) k_gauge_hash(const double2 *ext, long n, 
   if (threadIdx.x == 0) part[blockIdx.x] = h;
 }
 
-__global__ void __launch_bounds__(256) k_hash_sum(const unsigned long long *part, int n, unsigned long long *out) {
+// gate: a state whose done says whether the hash is another one than known
+__global__ void __launch_bounds__(256) k_hash_sum(const unsigned long long *part, int n, unsigned long long *out,
+                                                  unsigned long long known, SysState *gate) {
   unsigned long long h = 0;
   for (int k = threadIdx.x; k < n; k += blockDim.x) h += part[k];
   h = block_hash(h);
-  if (threadIdx.x == 0) *out = h;
+  if (threadIdx.x == 0) {
+    *out = h;
+    if (gate) gate->done = h != known;
+  }
 }
 
-static int hash_sum(const void *part, long n, unsigned long long *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_hash_sum, dim3(1), dim3(256), 0, s, (const unsigned long long *)part, (int)n, out);
+static int hash_sum(const void *part, long n, unsigned long long *out, unsigned long long known, SysState *gate,
+                    hipStream_t s) {
+  hipLaunchKernelGGL(k_hash_sum, dim3(1), dim3(256), 0, s, (const unsigned long long *)part, (int)n, out, known, gate);
   QCU_HIP(hipGetLastError());
   return 0;
 }
 
-int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, hipStream_t s) {
+int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, unsigned long long known,
+               SysState *gate, hipStream_t s) {
   const long n = 36L * 2 * g.vh;  // complex entries: [4][2][Vh][3][3]
   hipLaunchKernelGGL(k_gauge_hash, dim3(kHashBlocks), dim3(256), 0, s, (const double2 *)ext, n,
                      (unsigned long long *)scratch);
   QCU_HIP(hipGetLastError());
-  return hash_sum(scratch, kHashBlocks, out, s);
+  return hash_sum(scratch, kHashBlocks, out, known, gate, s);
 }
 
 static long gauge_blocks(const Geom &g) { return (8L * g.vh + 255) / 256; }
@@ -138,7 +145,7 @@ int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeO
     QCU_CHECK(mask == 1, QCU_ERR_ARG, "bad precision mask");
     hipLaunchKernelGGL((k_gauge_in<1, true>), nb, bs, 0, s, e, g, o);
     QCU_HIP(hipGetLastError());
-    return hash_sum(o.hash, nb.x, o.hash_out, s);
+    return hash_sum(o.hash, nb.x, o.hash_out, 0, nullptr, s);
   }
   switch (mask) {
     case 1: hipLaunchKernelGGL((k_gauge_in<1, false>), nb, bs, 0, s, e, g, o); break;

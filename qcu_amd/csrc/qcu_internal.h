@@ -136,8 +136,10 @@ struct GaugeOut {
 // mask bit k: links of precision k are written (bit 0, FP64, always set)
 int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeOut &out, hipStream_t s);
 // 64-bit content hash of an external gauge field into *out (memory the device can
-// write); scratch: gauge_hash_scratch_bytes() of device memory
-int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, hipStream_t s);
+// write); scratch: gauge_hash_scratch_bytes() of device memory; gate->done becomes 1
+// where the hash is another one than known, else 0
+int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, unsigned long long known,
+               SysState *gate, hipStream_t s);
 size_t gauge_hash_scratch_bytes(const Geom &g);
 // external one-parity field <-> system (seg, rhs) of a batch vector
 int spinor_ext_to_batch(const void *ext, const BatchOp &op, int seg, int rhs, SpinorPtr dst, int prec,
@@ -165,8 +167,9 @@ int hop_split_red(const BatchOp &op, int prec, SpinorPtr out, SpinorPtr in, Spin
                   SysState *st, double *partials, hipStream_t s);
 // the FP64 hop on the caller's fields of a single lattice, which must not overlap:
 // out = [A_p^-1] D_{p,1-p} in on one-parity fields, or (mat) out = A in - kappa D in
-// on full ones
-int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s);
+// on full ones; with a gate (device memory) whose done is set out is left as it is
+int hop_ext(const BatchOp &op, void *out, const void *in, int parity, int mat, bool use_clover, hipStream_t s,
+            const SysState *gate = nullptr);
 
 // clover.hip
 // packed A and A^-1 of one parity; FP32 and FP16 copies of A^-1 where asked for
