@@ -98,7 +98,7 @@ __global__ void __launch_bounds__(8 * kSplitSites) k_it_even(ItArgs a) {
   const int k = n / sd.nrhs, rhs = n - k * sd.nrhs;
   const bool valid = n < sd.nthr;
   int i;
-  const Site s = ordered_site(g, sd.zslab, valid ? k : 0, 0, i);
+  const Site s = ordered_site(g, sd.zslab, k, 0, i);
   const int t = i * sd.nrhs + rhs;
   const SpinorPtr rv = seg_view(a.r, P, sd.voff, sd.nthr), vv = seg_view(a.v, P, sd.voff, sd.nthr),
                   pv = seg_view(a.p, P, sd.voff, sd.nthr);

@@ -116,7 +116,7 @@ struct Site {
   int xh, y, z, t, xodd;  // xodd: full x coordinate is odd
 };
 
-QCU_D Site decode(const Geom &g, int i, int parity) {
+QCU_HD Site decode(const Geom &g, int i, int parity) {
   Site s;
   int r = i / g.lxh;
   s.xh = i - r * g.lxh;
@@ -131,7 +131,10 @@ QCU_D Site decode(const Geom &g, int i, int parity) {
 // Site number k of the order in which the hop kernels visit the sites: with
 // zslab = 0 the storage order, else slabs of zslab z planes one after the other,
 // t by t within a slab (the last slab may be thinner).  i: the half-site index.
-QCU_D Site ordered_site(const Geom &g, int zslab, int k, int parity, int &i) {
+// Past the last site (lanes that fill up a wave) there is no slab to divide by: k
+// there stands for the last site.
+QCU_HD Site ordered_site(const Geom &g, int zslab, int k, int parity, int &i) {
+  k = k < g.vh ? k : g.vh - 1;
   if (zslab == 0) {
     i = k;
     return decode(g, k, parity);
