@@ -14,6 +14,7 @@
 #include "../../include/qcu.h"
 #include "qcu_lattice.h"
 #include "qcu_solver.h"
+#include "qcu_tune.h"
 
 namespace qcu {
 
@@ -36,7 +37,7 @@ static void set_tuned(const std::string &key, LaunchCfg c) {
   ++g_tune_gen;
 }
 
-// back to the shape that the rule of dslash.hip picks
+// back to the shape that the rule picks
 static void set_automatic(const std::string &key) {
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -90,15 +91,7 @@ static LaunchCfg find_cfg(const BatchOp &op, int prec) {
     auto it = g_tuned.find(tune_key(op, prec));
     if (it != g_tuned.end()) return it->second;
   }
-  // no shape tuned or pinned: single-wave blocks refill a SIMD as soon as a wave
-  // ends (24^3x48 FP64 142 against 149 us in blocks of 256); large batches take
-  // longer blocks, which run as fast there and write fewer block partials.  The
-  // low precisions fence their directions in pairs (24^3x48 FP32 65 against 73 us
-  // unfenced), FP64 needs every load in flight (32^3x64 plain 282 against 288 us).
-  LaunchCfg c;
-  c.block = op.nvsites <= (1 << 20) ? 64 : 256;
-  c.group = prec == P64 ? 0 : 2;
-  return c;
+  return rule_cfg(op.nvsites, prec);
 }
 
 LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
@@ -149,26 +142,12 @@ int bench_hop(const BatchOp &op, hipStream_t s, int prec, int clover, int xpay, 
 
 static int tune_op(const BatchOp &op, hipStream_t s, int prec, double *best_ms, LaunchCfg *out) {
   const int clover = op.has_clover ? 1 : 0;
-  const int blocks[] = {64, 128, 256};
-  // the shape that the rule picks, then each one-thread-per-site shape
+  const LaunchCfg rule = rule_cfg(op.nvsites, prec);
   LaunchCfg best;
-  double bms = 1e30;
-  QCU_TRY(bench_hop(op, s, prec, clover, 1, 20, best, &bms));
-  for (int grp = 0; grp < 3; ++grp)
-    for (int b : blocks)
-      for (int r = 0; r < 2; ++r) {
-        LaunchCfg c;
-        c.block = b;
-        c.remap = r;
-        c.group = grp;
-        c.automatic = false;
-        double ms = 0;
-        QCU_TRY(bench_hop(op, s, prec, clover, 1, 20, c, &ms));
-        if (ms < bms) {
-          bms = ms;
-          best = c;
-        }
-      }
+  double bms = 0;
+  QCU_TRY(fastest_shape(
+      rule, hop_is_split(op, rule),
+      [&](const LaunchCfg &c, double *ms) { return bench_hop(op, s, prec, clover, 1, 20, c, ms); }, &best, &bms));
   if (best.automatic)
     set_automatic(tune_key(op, prec));
   else
