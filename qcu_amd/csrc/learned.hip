@@ -731,28 +731,13 @@ __global__ void __launch_bounds__(256) k_net_wgrad(NetWgradArgs a) {
 // through LDS and the block sums are added in a fixed order by
 // k_net_wgrad_fin.
 //
-// The grid is one row of 9 x kWgBlocks blocks.  The 9 blocks (one per term)
+// The grid is one row of 9 x wgrad_blocks() blocks.  The 9 blocks (one per term)
 // of a site block sb are 8 block indices apart inside a window of 72: blocks
 // go to the XCDs in turn, so all 9 run at about the same time on one XCD and
 // read the output gradient and the input field of their sites from its L2,
 // instead of from HBM once per term.  XCD k takes the site blocks
 // k nsb / 8 .. (k + 1) nsb / 8 - 1, so at each step of the waves' sweep it
 // works on one contiguous stretch of sites (their y neighbours included).
-constexpr int kWgBlocks = 1024;  // most blocks per term (a multiple of 8)
-
-// Blocks per term, a multiple of 8.  Each leaves an 8 KiB sum that
-// k_net_wgrad_fin reads again, so a block takes at least 16 steps of 32 sites;
-// smaller lattices take up to 88 blocks, which with 9 terms and 3 blocks per CU
-// fill the chip once (16^3x32, 8 -> 8: 1024 blocks 282 + 80 us for the sum, 256
-// blocks 270 + 6 us).
-static int wgrad_blocks(int vh) {
-  const int steps = (2 * vh + 31) / 32;
-  int n = steps / 16;
-  if (n < 88) n = steps < 88 ? steps : 88;
-  n = (n + 7) & ~7;
-  return n < kWgBlocks ? n : kWgBlocks;
-}
-
 template <int MT, int NT, bool SPLIT, bool LDS>
 __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *part) {
   const Geom g = a.g;
@@ -1930,7 +1915,7 @@ int Net::backward(SpinorPtr gout, hipStream_t s, bool want_grad_in, SpinorPtr gr
     if (use_mfma) {
       const int mt = (cout + 3) / 4, nt = (cin + 3) / 4;
       static_assert(kWgBlocks % 8 == 0, "term blocks of a site block share an XCD");
-      const int nwb = wgrad_blocks(lat->g.vh);
+      const int nwb = wgrad_blocks(lat->g.vh, wg_lds);
       const dim3 grid(9 * nwb);
       float *pp = (float *)wpart.p;
       float2 *dst = (float2 *)gW.p + woff[k];

@@ -251,6 +251,19 @@ int net_pack_second(const float2 *W1, const float2 *W2, void *Apk, float *winv, 
 int net_compose_tail(const float2 *const (&W)[4], float2 *C, float2 *G, float2 *S, hipStream_t s);
 int net_layer_second(const NetSecondArgs &a, int part, hipStream_t s);
 
+// Blocks per term of the weight gradient's products (a multiple of 8).  A block's FP32
+// sums end in k_net_wgrad_fin's FP64 ones, so more blocks are shorter FP32 sums: as
+// many as there are steps of 32 sites (without LDS of 16: a wave then takes its groups
+// of 4 one at a time), up to 1024, beyond which each block takes several.
+// Fewer blocks write and read fewer of the 8 KiB block sums, at the price of longer
+// FP32 sums (16^3x32, 8 -> 8: 256 blocks of 16 steps 226 us and 6 us for the FP64 sums,
+// 1024 blocks of 4 steps 238 and 16 us); no size takes longer ones than 1024 blocks give.
+constexpr int kWgBlocks = 1024;
+inline int wgrad_blocks(int vh, bool lds) {
+  const long long per = lds ? 32 : 16, steps = (2LL * vh + per - 1) / per;
+  return (int)(steps < kWgBlocks ? (steps + 7) & ~7LL : kWgBlocks);
+}
+
 typedef _Float16 h8v __attribute__((ext_vector_type(8)));
 
 // exact power of two that brings a largest magnitude mx below 2^top (1 for a
