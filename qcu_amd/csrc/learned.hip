@@ -1751,7 +1751,7 @@ int Net::pack_apply(hipStream_t s) {
   if (tail_split()) {
     const float2 *w = (const float2 *)W.p;
     float2 *C = (float2 *)wcomp.p, *G = C + 9 * 8 * 8 * 16, *S = G + 9 * 8 * 16;
-    QCU_TRY(net_compose_tail({w + woff[0], w + woff[1], w + woff[2], w + woff[3]}, C, G, S, s));
+    QCU_TRY(net_compose_tail({w + woff[0], w + woff[1], w + woff[2], w + woff[3]}, p2winv(), C, G, S, s));
     QCU_TRY(net_pack_split(C, 8, 8, tail_c(), tail_winv(), 32, s));
     QCU_TRY(net_pack_first(G, tail_g(), tail_winv() + 1, s));
     QCU_TRY(net_pack_fuse(S, tail_s(), tail_winv() + 2, s));
@@ -1860,6 +1860,7 @@ int Net::forward(const SysState *st, hipStream_t s, bool odd_only_last, int zero
         q.winv = tail_winv() + 1;
         q.Ah = (const uint4 *)tail_c();
         q.winvh = tail_winv();
+        q.winve = p2winv();
         q.out_max = nullptr;
       }
       QCU_TRY(net_layer_second(q, k == 2 ? 2 : tail ? 1 : 0, s));

@@ -965,6 +965,9 @@ __global__ void __launch_bounds__(256) k_net_pack_second(const float2 *W1, const
 // it (transports and splits, half of the time); loads two steps ahead, or all
 // terms of two channels before the next two, measured no faster.
 enum { SECOND_BOTH, SECOND_ODD, SECOND_TAIL };
+// the power of two above E's largest entry (winve: its inverse packing scale), by
+// which G is divided
+QCU_D double tail_unit(const float *winve) { return 16384.0 * winve[0]; }
 template <int WAVES, int MODE>
 __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
   typedef SplitShape<32> SH;
@@ -980,11 +983,15 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
   const Geom g = a.g;
   // operand scales: s0 the input's, s1 the first layer's even sites'
   const float s0 = pow2_scale(__uint_as_float(*a.in_max), 14);
-  const float s1 = pow2_scale(__uint_as_float(*a.l1_max), 14);
+  float s1 = pow2_scale(__uint_as_float(*a.l1_max), 14);
   const float oe = a.winv[0] / s0;    // even sites: E against the input
+  // the input's part (site term S, or G) -> the hop terms' scale; where the hop terms
+  // are 2^60 times smaller, their scale gives way instead of overflowing the sum
+  const double win = MODE == SECOND_TAIL ? a.winv[0] * tail_unit(a.winve) : (double)a.winv[1];
+  const double ratio = win * s1 / ((double)a.winvh[0] * s0);
+  const float rs = (float)fmin(ratio, 0x1p60);
+  if (ratio > 0x1p60) s1 = (float)(s1 * (0x1p60 / ratio));
   const float oo = a.winvh[0] / s1;   // the hop terms against L1
-  // the input's part (site term S, or G) -> the hop terms' scale
-  const float rs = (a.winv[MODE == SECOND_TAIL ? 0 : 1] * s1) / (a.winvh[0] * s0);
   const int lane = threadIdx.x & 63, gq = lane >> 5, n = lane & 31;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const size_t field = (size_t)g.vh * 96, plane = (size_t)g.vh * 16;
@@ -1234,12 +1241,16 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
 // The composed matrices of a 1-8-8-8-1 preconditioner (see k_net_second), as
 // weights in the layout of an 8 -> 8, a 1 -> 8 and an 8 -> 1 layer:
 //   C[u][t][i] = W4_t W3_u          (u, t = 0..7; u = 8: zero)
-//   G[u][t][0] = (W4_t W3_8 + W4_8 W3_t) (W2_u W1_8 + W2_8 W1_u)   (u = 8: zero)
+//   G[u][t][0] = (W4_t W3_8 + W4_8 W3_t) E_u / tail_unit,
+//                E_u = W2_u W1_8 + W2_8 W1_u   (u = 8: zero)
 //   S[8][0][i] = W4_8 W3_8          (other terms zero)
-// FP64 sums, rounded to FP32.  Block (u, t) forms the matrices of that pair of terms,
-// one entry of each sum per thread: 8 us.
+// FP64 sums, rounded to FP32.  Without the unit G, a product of four layers' weights,
+// would leave FP32's range for weights of 2^32 or 2^-38, where every layer's output
+// can be of order one.  Block (u, t) forms the matrices of that pair of terms, one
+// entry of each sum per thread: 8 us.
 __global__ void __launch_bounds__(128) k_net_compose_tail(const float2 *W1, const float2 *W2, const float2 *W3,
-                                                          const float2 *W4, float2 *C, float2 *G, float2 *S) {
+                                                          const float2 *W4, const float *winve, float2 *C, float2 *G,
+                                                          float2 *S) {
   __shared__ double2 M[8 * 16], E[8 * 16];
   const int u = blockIdx.x, t = blockIdx.y, tid = threadIdx.x;
   const int i = tid >> 4, s = (tid >> 2) & 3, s2 = tid & 3;
@@ -1279,12 +1290,13 @@ __global__ void __launch_bounds__(128) k_net_compose_tail(const float2 *W1, cons
         g.x += x.x * y.x - x.y * y.y;
         g.y += x.x * y.y + x.y * y.x;
       }
-    G[((size_t)u * 8 + t) * 16 + tid] = make_float2((float)g.x, (float)g.y);
+    const double unit = tail_unit(winve);
+    G[((size_t)u * 8 + t) * 16 + tid] = make_float2((float)(g.x / unit), (float)(g.y / unit));
   }
 }
 
-int net_compose_tail(const float2 *const (&W)[4], float2 *C, float2 *G, float2 *S, hipStream_t s) {
-  hipLaunchKernelGGL(k_net_compose_tail, dim3(9, 8), dim3(128), 0, s, W[0], W[1], W[2], W[3], C, G, S);
+int net_compose_tail(const float2 *const (&W)[4], const float *winve, float2 *C, float2 *G, float2 *S, hipStream_t s) {
+  hipLaunchKernelGGL(k_net_compose_tail, dim3(9, 8), dim3(128), 0, s, W[0], W[1], W[2], W[3], winve, C, G, S);
   QCU_HIP(hipGetLastError());
   return 0;
 }

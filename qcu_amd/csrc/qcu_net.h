@@ -244,11 +244,13 @@ struct NetSecondArgs {
   const uint4 *A2 = nullptr;
   const float *winv2 = nullptr;
   char *mix = nullptr;
+  const float *winve = nullptr;  // part 2: E's inverse scale (net_pack_second), G's unit
 };
 int net_pack_second(const float2 *W1, const float2 *W2, void *Apk, float *winv, hipStream_t s);
 // matrices of net_layer_second's parts 1 and 2, composed of the weights W of a
-// 1-8-8-8-1 network: C an 8 -> 8, G a 1 -> 8 and S an 8 -> 1 layer's weights
-int net_compose_tail(const float2 *const (&W)[4], float2 *C, float2 *G, float2 *S, hipStream_t s);
+// 1-8-8-8-1 network: C an 8 -> 8, G a 1 -> 8 (in units of E's scale; winve: what
+// net_pack_second left for E) and S an 8 -> 1 layer's weights
+int net_compose_tail(const float2 *const (&W)[4], const float *winve, float2 *C, float2 *G, float2 *S, hipStream_t s);
 int net_layer_second(const NetSecondArgs &a, int part, hipStream_t s);
 
 // Blocks per term of the weight gradient's products (a multiple of 8).  A block's FP32
