@@ -61,22 +61,30 @@ QCU_HD cplx<T> mul_mi(cplx<T> a) { return mk(a.im, -a.re); }
 QCU_HD double fma_(double a, double b, double c) { return __builtin_fma(a, b, c); }
 QCU_HD float fma_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 template <class T>
-QCU_HD void cmad(cplx<T> &a, cplx<T> b, cplx<T> c) {
+QCU_HD cplx<T> prod_(cplx<T> b, cplx<T> c) {
 #pragma clang fp contract(off)
-  a.re = a.re + fma_(b.re, c.re, -(b.im * c.im));
-  a.im = a.im + fma_(b.re, c.im, b.im * c.re);
+  return mk(fma_(b.re, c.re, -(b.im * c.im)), fma_(b.re, c.im, b.im * c.re));
+}
+template <class T>
+QCU_HD cplx<T> prodj_(cplx<T> b, cplx<T> c) {
+#pragma clang fp contract(off)
+  return mk(fma_(b.re, c.re, b.im * c.im), fma_(b.re, c.im, -(b.im * c.re)));
+}
+template <class T>
+QCU_HD void cmad(cplx<T> &a, cplx<T> b, cplx<T> c) {
+  a = a + prod_(b, c);
 }
 template <class T>
 QCU_HD void cmadj(cplx<T> &a, cplx<T> b, cplx<T> c) {
-#pragma clang fp contract(off)
-  a.re = a.re + fma_(b.re, c.re, b.im * c.im);
-  a.im = a.im + fma_(b.re, c.im, -(b.im * c.re));
+  a = a + prodj_(b, c);
 }
 // cmad / cmadj, or with CHAIN the products as chained FMAs: 2 instructions per
-// component instead of 3, at one more rounding.  For the FP16 fields, whose hop
-// is near its vector rate (24^3x48 with 12 right-hand sides 356 against 310 us)
-// and whose halves the FMAs take unconverted; the FP32 hop is slower with it
-// (380 against 395 us: longer dependent chains).
+// component instead of 3, with two roundings of the running sum instead of one of it
+// and two of the product.  For the FP16 fields, whose hop is near its vector rate
+// (24^3x48 with 12 right-hand sides 356 against 310 us) and whose halves the FMAs
+// take unconverted; its error is that of the stored halves either way (clover hop at
+// 16^3x32 against FP64: 3.4366e-4 unchained, 3.4365e-4).  The FP32 hop is slower with
+// it (380 against 395 us: longer dependent chains).
 template <bool CHAIN, class T>
 QCU_HD void cmad_(cplx<T> &a, cplx<T> b, cplx<T> c) {
   if (CHAIN) {
@@ -473,27 +481,46 @@ struct CloverIO<P16> {
 
 // s a, never fused into what follows
 template <class T>
-QCU_D cplx<T> scale_(T s, cplx<T> a) {
+QCU_HD cplx<T> scale_(T s, cplx<T> a) {
 #pragma clang fp contract(off)
   return mk(s * a.re, s * a.im);
 }
 
+// Row of a clover block times a spinor, begun: the diagonal's product and the first
+// off-diagonal one p (unless CHAIN, where that follows as chained FMAs) rounded once.
+// A rounding of its own for the diagonal, the largest term, shows: clover hop in FP64
+// 2.35e-16 off instead of 2.30e-16, full operator 1.40e-16 instead of 1.33e-16, FP32
+// hop 1.094e-7 instead of 1.064e-7.
+template <class T>
+QCU_HD cplx<T> diag_plus(T d, cplx<T> x, cplx<T> p) {
+  return mk(fma_(d, x.re, p.re), fma_(d, x.im, p.im));
+}
+
 // out_b = C_b * v_b for chiral block b (spins {2b, 2b+1}) from its 36 packed reals
 template <bool CHAIN = false, class T>
-QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
+QCU_HD void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
   cplx<T> o[6];
   const cplx<T> *x = v + 6 * b;
 #pragma unroll
   for (int r = 0; r < 6; ++r) {
     cplx<T> acc = scale_(cb[r], x[r]);
+    const int first = CHAIN ? 6 : (r == 0 ? 1 : 0);
 #pragma unroll
     for (int col = 0; col < 6; ++col) {
       if (col < r) {
-        int k = 6 + 2 * (r * (r - 1) / 2 + col);
-        cmad_<CHAIN>(acc, mk(cb[k], cb[k + 1]), x[col]);
+        const int k = 6 + 2 * (r * (r - 1) / 2 + col);
+        const cplx<T> c = mk(cb[k], cb[k + 1]);
+        if (col == first)
+          acc = diag_plus(cb[r], x[r], prod_(c, x[col]));
+        else
+          cmad_<CHAIN>(acc, c, x[col]);
       } else if (col > r) {
-        int k = 6 + 2 * (col * (col - 1) / 2 + r);
-        cmadj_<CHAIN>(acc, mk(cb[k], cb[k + 1]), x[col]);
+        const int k = 6 + 2 * (col * (col - 1) / 2 + r);
+        const cplx<T> c = mk(cb[k], cb[k + 1]);
+        if (col == first)
+          acc = diag_plus(cb[r], x[r], prodj_(c, x[col]));
+        else
+          cmadj_<CHAIN>(acc, c, x[col]);
       }
     }
     o[r] = acc;
@@ -504,7 +531,7 @@ QCU_D void clover_apply_block(const T *cb, cplx<T> (&v)[12], int b) {
 
 // out = C * v for one site (both chiral blocks)
 template <bool CHAIN, class T>
-QCU_D void clover_apply_site(const T (&c)[72], cplx<T> (&v)[12]) {
+QCU_HD void clover_apply_site(const T (&c)[72], cplx<T> (&v)[12]) {
   clover_apply_block<CHAIN>(c, v, 0);
   clover_apply_block<CHAIN>(c + 36, v, 1);
 }

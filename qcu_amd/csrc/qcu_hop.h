@@ -310,7 +310,10 @@ struct CloverRows {
 #pragma unroll
     for (int k = 0; k < 5; ++k) {
       const cplx<T> c = CloverWord<P>::value(e[q][k]);
-      if (k < r)
+      if (k == 0 && P != P16) {
+        const bool low = q == 1 || j > 0;  // column 0; row 0 begins with the adjoint of column 1
+        acc = diag_plus(diag, v, prod_(mk(c.re, low ? c.im : -c.im), x[low ? 0 : 1][lane]));
+      } else if (k < r)
         cmad_<P == P16>(acc, c, x[k][lane]);
       else
         cmadj_<P == P16>(acc, c, x[k + 1][lane]);
