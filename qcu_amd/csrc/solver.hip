@@ -172,8 +172,10 @@ static int prepare_split(Solver &S, VecSet &V) {
   return V.split_buf.alloc(2 * part + S.nsys * sizeof(SysState));
 }
 
-static int enqueue_chunk(Solver &S, VecSet &V, Precond *K, int n) {
-  if (!split_chunk(S, V, K, n)) {
+// split: as split_chunk() said when prepare_split() made room for it.  Asked again, it
+// may say something else: another thread's tuning changes the shapes at any time.
+static int enqueue_chunk(Solver &S, VecSet &V, Precond *K, int n, bool split) {
+  if (!split) {
     for (int k = 0; k < n; ++k) QCU_TRY(enqueue_iteration(S, V, K));
     return 0;
   }
@@ -197,8 +199,9 @@ static int enqueue_chunk(Solver &S, VecSet &V, Precond *K, int n) {
 }
 
 static int run_chunk(Solver &S, VecSet &V, Precond *K, int chunk, bool use_graph) {
-  if (split_chunk(S, V, K, chunk)) QCU_TRY(prepare_split(S, V));
-  if (!use_graph) return enqueue_chunk(S, V, K, chunk);
+  const bool split = split_chunk(S, V, K, chunk);
+  if (split) QCU_TRY(prepare_split(S, V));
+  if (!use_graph) return enqueue_chunk(S, V, K, chunk, split);
   if (V.graph_tune != tune_generation()) {
     // the graphs hold the launch shapes of their capture: a newly tuned (or
     // set) shape needs new graphs
@@ -223,7 +226,7 @@ static int run_chunk(Solver &S, VecSet &V, Precond *K, int chunk, bool use_graph
   if (it == V.graphs.end()) {
     hipGraph_t graph;
     QCU_HIP(hipStreamBeginCapture(S.stream, hipStreamCaptureModeThreadLocal));
-    const int rc = enqueue_chunk(S, V, K, chunk);
+    const int rc = enqueue_chunk(S, V, K, chunk, split);
     hipError_t e = hipStreamEndCapture(S.stream, &graph);
     if (rc) return rc;
     QCU_HIP(e);
