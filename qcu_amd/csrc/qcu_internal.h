@@ -3,6 +3,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <string>
 #include <vector>
 
@@ -99,6 +100,32 @@ struct LaunchCfg {
   bool automatic = true;  // no shape was tuned or pinned: dslash.hip may take its split kernel
 };
 
+// The launch shape of each precision as last looked up, with the tune generation it
+// was looked up in.  A lattice's is read by the threads of its own handle and of its
+// networks' handles, so shape and generation are one word.
+struct ShapeMemo {
+  bool get(int prec, unsigned long long gen, LaunchCfg *c) const {
+    const unsigned long long w = word[prec].load(std::memory_order_relaxed);
+    if (w >> 16 != gen) return false;
+    c->block = (int)(w & 511);
+    c->remap = (int)(w >> 9 & 1);
+    c->group = (int)(w >> 10 & 3);
+    c->automatic = w >> 12 & 1;
+    return true;
+  }
+  void put(int prec, unsigned long long gen, const LaunchCfg &c) {
+    word[prec].store(gen << 16 | (unsigned)c.automatic << 12 | (unsigned)c.group << 10 | (unsigned)c.remap << 9 |
+                         (unsigned)c.block,
+                     std::memory_order_relaxed);
+  }
+  void clear() {
+    for (auto &w : word) w.store(0, std::memory_order_relaxed);
+  }
+
+ private:
+  std::atomic<unsigned long long> word[3] = {};  // generations begin at 1
+};
+
 // --------------------------------------------------------------------------
 // batches: the segment table (qcu_batch.h) on the host and the device
 // --------------------------------------------------------------------------
@@ -115,9 +142,7 @@ struct BatchOp {
   bool has_clover = false;
   std::string tune_base;  // see tune_key()
   std::vector<char> uploaded;  // contents of the device table
-  // the launch shapes last looked up, valid for tune generation cfg_gen
-  mutable LaunchCfg cfg[3];
-  mutable unsigned long long cfg_gen[3] = {0, 0, 0};
+  mutable ShapeMemo shapes;  // the launch shapes last looked up
   // one segment per lattice with nrhs[k] right-hand sides
   int build(const std::vector<const Lattice *> &lats, const std::vector<int> &nrhs, hipStream_t s);
   int max_blocks(int bsz) const;

@@ -93,7 +93,7 @@ int BatchOp::build(const std::vector<const Lattice *> &ls, const std::vector<int
   const int pcap = max_blocks(64) + 1;
   for (SegDesc &d : segs) d.pcap = pcap;
   tune_base = qcu::tune_base(*this);
-  for (unsigned long long &gen : cfg_gen) gen = 0;
+  shapes.clear();
   std::vector<int> first;  // see find_seg()
   for (int k = 0; k < kSegBlockSizes; ++k) {
     const int bsz = seg_block_size(k);

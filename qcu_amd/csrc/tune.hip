@@ -97,11 +97,12 @@ static LaunchCfg find_cfg(const BatchOp &op, int prec) {
 LaunchCfg tuned_cfg(const BatchOp &op, int prec) {
   if (prec < P64 || prec > P16) return LaunchCfg();  // no such shape: hop() refuses the precision
   const unsigned long long gen = tune_generation();
-  if (op.cfg_gen[prec] != gen) {
-    op.cfg[prec] = find_cfg(op, prec);
-    op.cfg_gen[prec] = gen;
+  LaunchCfg c;
+  if (!op.shapes.get(prec, gen, &c)) {
+    c = find_cfg(op, prec);
+    op.shapes.put(prec, gen, c);
   }
-  return op.cfg[prec];
+  return c;
 }
 
 // average milliseconds per launch of the hop kernel on resident fields

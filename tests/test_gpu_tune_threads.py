@@ -64,3 +64,35 @@ def test_solves_beside_tuning(orc, csw):
     _beside(work, other)
     lat.close()
     same.close()
+
+
+def test_network_and_lattice_threads_beside_tuning(orc):
+    """a network's handle in one thread, its lattice's in another, shapes changing"""
+    import numpy as np
+    from qcu_amd.lattice import FP32, FP64, LearnedPreconditioner
+    L, csw = (4, 6, 4, 10), 1.0
+    U = orc.gauge_random(L, 0.3, 1810)
+    lat, same = _lattice(L, U, csw), _lattice(L, U, csw)
+    net = LearnedPreconditioner(lat, (1, 4, 1), seed=1811)
+    src = dev(orc.gauss((orc.vol(L) // 2, 4, 3), 1812))
+    psi = orc.gauss((orc.vol(L) // 2, 4, 3), 1813)
+    pd, ref = dev(psi), orc.clover_dslash(psi, U, L, 0, KAPPA * csw, -1)
+    want = net.loss_grad(src)
+
+    def other():
+        for prec in (FP64, FP32):
+            for shape in ((64, 1, 0), (256, 0, 2), (128, 1, 1)):
+                same.set_launch_shape(prec, *shape)
+        loss, grad = net.loss_grad(src)
+        assert abs(loss - want[0]) <= 1e-6 * abs(want[0])
+        assert np.linalg.norm(grad - want[1]) <= 1e-4 * np.linalg.norm(want[1])
+
+    def work():
+        for k in range(200):
+            out = host(lat.dslash(pd, 0, clover=True, prec=k % 2))
+            assert np.linalg.norm(out - ref) <= (2e-6 if k % 2 else 1e-12) * np.linalg.norm(ref), k
+
+    _beside(work, other)
+    net.close()
+    lat.close()
+    same.close()
