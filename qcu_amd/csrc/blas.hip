@@ -257,21 +257,25 @@ __global__ void __launch_bounds__(256) k_dot2(SpinorPtr a_, SpinorPtr b_, const 
   block_partial_rhs<3>(acc, partials, blockIdx.x, c.t0, c.nrhs, c.pcap);
 }
 
-// y = a x + b y (all systems)
-template <int Px, int Py>
-__global__ void __launch_bounds__(256) k_axpby(double a, SpinorPtr x, double b, SpinorPtr y, const SegDesc *segs, int nseg) {
+// y = x (FP64) in precision P, and x = 0 (all systems)
+template <int P>
+__global__ void __launch_bounds__(256) k_convert(SpinorPtr y, SpinorPtr x, const SegDesc *segs, int nseg) {
   const TCtx c = tctx(segs, nseg, nullptr);
   if (!c.valid) return;
-  typedef RT<Py> T;
-  cplx<RT<Px>> xx[12];
-  cplx<T> yy[12];
-  if (a != 0.0) SpinorIO<Px>::load(view<Px>(x, c), c.t, xx);
-  else zero12<Px>(xx);
-  if (b != 0.0) SpinorIO<Py>::load(view<Py>(y, c), c.t, yy);
-  else zero12<Py>(yy);
-#pragma unroll
-  for (int k = 0; k < 12; ++k) yy[k] = mk<T>((T)(a * xx[k].re + b * yy[k].re), (T)(a * xx[k].im + b * yy[k].im));
-  SpinorIO<Py>::store(view<Py>(y, c), c.t, yy);
+  cplx<double> xx[12];
+  cplx<RT<P>> yy[12];
+  SpinorIO<P64>::load(view<P64>(x, c), c.t, xx);
+  cvt<P, P64>(xx, yy);
+  SpinorIO<P>::store(view<P>(y, c), c.t, yy);
+}
+
+template <int P>
+__global__ void __launch_bounds__(256) k_zero(SpinorPtr x, const SegDesc *segs, int nseg) {
+  const TCtx c = tctx(segs, nseg, nullptr);
+  if (!c.valid) return;
+  cplx<RT<P>> xx[12];
+  zero12<P>(xx);
+  SpinorIO<P>::store(view<P>(x, c), c.t, xx);
 }
 
 // y += x (FP64), x = 0: a reliable update takes the correction into the solution
@@ -715,33 +719,27 @@ int reliable_residual(const BatchOp &op, SpinorPtr r, SpinorPtr rt, SpinorPtr r6
   return finish(op, partials, bs, 3, FK_RELIABLE, st, nullptr, s);
 }
 
-int axpby(const BatchOp &op, double a, SpinorPtr x, int px, double b, SpinorPtr y, int py, hipStream_t s) {
+int spinor_convert(const BatchOp &op, SpinorPtr dst, int pdst, SpinorPtr src, hipStream_t s) {
   const int bs = 256, nb = batch_blocks(op, bs);
-#define QCU_AXPBY(A, B)                                                                         \
-  if (px == A && py == B) {                                                                   \
-    hipLaunchKernelGGL((k_axpby<A, B>), dim3(nb), dim3(bs), 0, s, a, x, b, y, QCU_SEGS);      \
-    QCU_HIP(hipGetLastError());                                                               \
-    return 0;                                                                                 \
+  switch (pdst) {
+    case P64: hipLaunchKernelGGL(k_convert<P64>, dim3(nb), dim3(bs), 0, s, dst, src, QCU_SEGS); break;
+    case P32: hipLaunchKernelGGL(k_convert<P32>, dim3(nb), dim3(bs), 0, s, dst, src, QCU_SEGS); break;
+    default: hipLaunchKernelGGL(k_convert<P16>, dim3(nb), dim3(bs), 0, s, dst, src, QCU_SEGS); break;
   }
-  QCU_AXPBY(P64, P64)
-  QCU_AXPBY(P32, P64)
-  QCU_AXPBY(P16, P64)
-  QCU_AXPBY(P64, P32)
-  QCU_AXPBY(P32, P32)
-  QCU_AXPBY(P16, P32)
-  QCU_AXPBY(P64, P16)
-  QCU_AXPBY(P32, P16)
-  QCU_AXPBY(P16, P16)
-#undef QCU_AXPBY
-  set_error(QCU_ERR_ARG, "axpby: bad precision");
-  return QCU_ERR_ARG;
+  QCU_HIP(hipGetLastError());
+  return 0;
 }
 
-int spinor_convert(const BatchOp &op, SpinorPtr dst, int pdst, SpinorPtr src, int psrc, hipStream_t s) {
-  return axpby(op, 1.0, src, psrc, 0.0, dst, pdst, s);
+int zero_spinor(const BatchOp &op, SpinorPtr x, int px, hipStream_t s) {
+  const int bs = 256, nb = batch_blocks(op, bs);
+  switch (px) {
+    case P64: hipLaunchKernelGGL(k_zero<P64>, dim3(nb), dim3(bs), 0, s, x, QCU_SEGS); break;
+    case P32: hipLaunchKernelGGL(k_zero<P32>, dim3(nb), dim3(bs), 0, s, x, QCU_SEGS); break;
+    default: hipLaunchKernelGGL(k_zero<P16>, dim3(nb), dim3(bs), 0, s, x, QCU_SEGS); break;
+  }
+  QCU_HIP(hipGetLastError());
+  return 0;
 }
-
-int zero_spinor(const BatchOp &op, SpinorPtr x, int px, hipStream_t s) { return axpby(op, 0.0, x, px, 0.0, x, px, s); }
 
 int xmy_norm(const BatchOp &op, SpinorPtr b, SpinorPtr r, SysState *st, double *partials, int store,
              hipStream_t s) {

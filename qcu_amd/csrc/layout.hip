@@ -158,7 +158,8 @@ int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeO
   return 0;
 }
 
-// external one-parity field [Vh][4][3] <-> system (segment seg, rhs r) of a batch vector
+// external one-parity field [Vh][4][3] <-> system (segment seg, rhs r) of a batch vector,
+// FP32 or FP16
 template <int P>
 __global__ void k_spinor_in(const double2 *ext, int vh, int nrhs, int rhs, SpinorPtr dst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -195,7 +196,6 @@ int spinor_ext_to_batch(const void *ext, const BatchOp &op, int seg, int rhs, Sp
   const int vh = d.g.vh, bs = 256, nb = (vh + bs - 1) / bs;
   const double2 *e = (const double2 *)ext;
   switch (prec) {
-    case P64: hipLaunchKernelGGL(k_spinor_in<P64>, dim3(nb), dim3(bs), 0, s, e, vh, d.nrhs, rhs, v); break;
     case P32: hipLaunchKernelGGL(k_spinor_in<P32>, dim3(nb), dim3(bs), 0, s, e, vh, d.nrhs, rhs, v); break;
     case P16: hipLaunchKernelGGL(k_spinor_in<P16>, dim3(nb), dim3(bs), 0, s, e, vh, d.nrhs, rhs, v); break;
     default: set_error(QCU_ERR_ARG, "bad precision"); return QCU_ERR_ARG;
@@ -212,7 +212,6 @@ int spinor_batch_to_ext(SpinorPtr src, const BatchOp &op, int seg, int rhs, void
   const int vh = d.g.vh, bs = 256, nb = (vh + bs - 1) / bs;
   double2 *e = (double2 *)ext;
   switch (prec) {
-    case P64: hipLaunchKernelGGL(k_spinor_out<P64>, dim3(nb), dim3(bs), 0, s, v, vh, d.nrhs, rhs, e); break;
     case P32: hipLaunchKernelGGL(k_spinor_out<P32>, dim3(nb), dim3(bs), 0, s, v, vh, d.nrhs, rhs, e); break;
     case P16: hipLaunchKernelGGL(k_spinor_out<P16>, dim3(nb), dim3(bs), 0, s, v, vh, d.nrhs, rhs, e); break;
     default: set_error(QCU_ERR_ARG, "bad precision"); return QCU_ERR_ARG;

@@ -95,7 +95,7 @@ QCU_D void term_link_matrix(const LinkPtr &U, const TermGeo &tg, cf (&m)[9]) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
       const size_t cb = ((size_t)tg.slab * 3 + k) * U.vh * 16;
-      raw[k] = NT ? ld_nt(U.a, cb, (unsigned)tg.li * 16u) : ld_at<float4>(U.a, cb, (unsigned)tg.li * 16u);
+      raw[k] = NT ? ld_at<float4, true>(U.a, cb, (unsigned)tg.li * 16u) : ld_at<float4>(U.a, cb, (unsigned)tg.li * 16u);
     }
   }
   term_matrix(raw, tg.hop, tg.fwd, tg.ph, m);
@@ -593,7 +593,7 @@ __global__ void __launch_bounds__(256) k_net_gather(NetGatherArgs a) {
   auto load = [&](const SpinorPtr &f, int j, cf(&v)[12]) {
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
-      const float4 q = ld_nt(f.p, (size_t)k * f.stride * 16, (unsigned)j * 16u);
+      const float4 q = ld_at<float4, true>(f.p, (size_t)k * f.stride * 16, (unsigned)j * 16u);
       v[2 * k] = mk(q.x, q.y);
       v[2 * k + 1] = mk(q.z, q.w);
     }

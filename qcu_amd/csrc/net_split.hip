@@ -282,7 +282,7 @@ QCU_D void fused_epilogue(const MixOut &mo, const f16v (&acc)[3][2], float oscal
         v.y = dy[l0 % 3][e0 + 1] * yscale;
         v.z = dy[l1 % 3][e1] * yscale;
         v.w = dy[l1 % 3][e1 + 1] * yscale;
-        st_nt(ob, (size_t)(3 * g + q) * plane, off, v);
+        st_at<float4, true>(ob, (size_t)(3 * g + q) * plane, off, v);
       }
     }
   }
@@ -476,7 +476,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_layer_split(NetSplitArgs a) 
             f.z = acc[l1 % 3][mt][e1] * oscale;
             f.w = acc[l1 % 3][mt][e1 + 1] * oscale;
             omax = fmaxf(omax, fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))));
-            st_nt(ob, (size_t)(3 * (sb / 2) + q) * plane, off, f);
+            st_at<float4, true>(ob, (size_t)(3 * (sb / 2) + q) * plane, off, f);
           }
         }
     }
@@ -746,7 +746,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_first(NetFirstArgs a) {
           f.z = acc[l1 % 3][mt][e1] * oscale;
           f.w = acc[l1 % 3][mt][e1 + 1] * oscale;
           omax = fmaxf(omax, fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))));
-          st_nt(ob, (size_t)(3 * gq + q) * plane, off, f);
+          st_at<float4, true>(ob, (size_t)(3 * gq + q) * plane, off, f);
         }
       }
   };
@@ -757,7 +757,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_first(NetFirstArgs a) {
   // each link is read once (by the even sites' hops)
   auto load_link = [&](const TermGeo &tg, float4 (&l)[3]) {
 #pragma unroll
-    for (int k = 0; k < 3; ++k) l[k] = ld_nt(a.U.a, ((size_t)tg.slab * 3 + k) * plane, (unsigned)tg.li * 16u);
+    for (int k = 0; k < 3; ++k) l[k] = ld_at<float4, true>(a.U.a, ((size_t)tg.slab * 3 + k) * plane, (unsigned)tg.li * 16u);
   };
   int i = 0;
   bool ok = false;
@@ -1054,7 +1054,7 @@ __global__ void __launch_bounds__(64 * WAVES) k_net_second(NetSecondArgs a) {
           f.z = acc[l1 % 3][mt][e1] * os;
           f.w = acc[l1 % 3][mt][e1 + 1] * os;
           omax = fmaxf(omax, fmaxf(fmaxf(fabsf(f.x), fabsf(f.y)), fmaxf(fabsf(f.z), fabsf(f.w))));
-          st_nt(ob, (size_t)(3 * gq + q) * plane, off, f);
+          st_at<float4, true>(ob, (size_t)(3 * gq + q) * plane, off, f);
         }
       }
   };

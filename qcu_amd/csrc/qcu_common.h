@@ -170,10 +170,12 @@ QCU_HD Site ordered_site(const Geom &g, int zslab, int k, int parity, int &i) {
 // kept in scalar registers) plus a 32-bit per-lane byte offset, so that the
 // compiler can use the scalar-base / 32-bit-offset form of global memory
 // instructions instead of a 64-bit address per load and per component.
-// NT: non-temporal, for data a kernel reads once.  The global address space is
-// stated: the compiler cannot know it of a base that was itself read from memory
-// (a segment's links and clover blocks), and would use flat loads, which return
-// out of order and make every wait a full one.
+// NT: non-temporal, for data a kernel reads once, or writes for a later kernel to read
+// (the network's activations and term fields): they need not displace the lines that
+// the kernel reads again.  The global address space is stated: the compiler cannot
+// know it of a base that was itself read from memory (a segment's links and clover
+// blocks), and would use flat loads, which return out of order and make every wait a
+// full one.
 #define QCU_GLOBAL __attribute__((address_space(1)))
 template <class V, bool NT = false>
 QCU_D V ld_at(const void *base, size_t comp_bytes, unsigned lane_off) {
@@ -192,21 +194,6 @@ QCU_D void st_at(void *base, size_t comp_bytes, unsigned lane_off, const V &v) {
   QCU_GLOBAL words *p = (QCU_GLOBAL words *)((QCU_GLOBAL char *)base + comp_bytes + lane_off);
   if (NT) __builtin_nontemporal_store(w, p);
   else *p = w;
-}
-// the same as a non-temporal store: for fields written once and read by a
-// later kernel (the network's activations and term fields), which then need
-// not displace the lines that the writing kernel still reads
-QCU_D void st_nt(void *base, size_t comp_bytes, unsigned lane_off, const float4 &v) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  const f4 w = {v.x, v.y, v.z, v.w};
-  __builtin_nontemporal_store(w, (f4 *)((char *)base + comp_bytes + lane_off));
-}
-// a non-temporal load: for data the kernel reads once, which then need not
-// displace the lines it reads again
-QCU_D float4 ld_nt(const void *base, size_t comp_bytes, unsigned lane_off) {
-  typedef float f4 __attribute__((ext_vector_type(4)));
-  const f4 w = __builtin_nontemporal_load((const f4 *)((const char *)base + comp_bytes + lane_off));
-  return make_float4(w.x, w.y, w.z, w.w);
 }
 
 // ---------------------------------------------------------------------------

@@ -166,7 +166,7 @@ int gauge_ext_to_internal(const void *ext, const Geom &g, int mask, const GaugeO
 int gauge_hash(const void *ext, const Geom &g, void *scratch, unsigned long long *out, unsigned long long known,
                SysState *gate, hipStream_t s);
 size_t gauge_hash_scratch_bytes(const Geom &g);
-// external one-parity field <-> system (seg, rhs) of a batch vector
+// external one-parity field <-> system (seg, rhs) of a batch vector in FP32 or FP16
 int spinor_ext_to_batch(const void *ext, const BatchOp &op, int seg, int rhs, SpinorPtr dst, int prec,
                         hipStream_t s);
 int spinor_batch_to_ext(SpinorPtr src, const BatchOp &op, int seg, int rhs, void *ext, int prec, hipStream_t s);
@@ -227,9 +227,8 @@ int fold(const BatchOp &op, SpinorPtr x, int px, SpinorPtr y, hipStream_t s);
 // r = r64 in the solver's precision, then rho, beta, rr and rr_ref of every system
 int reliable_residual(const BatchOp &op, SpinorPtr r, SpinorPtr rt, SpinorPtr r64, int prec, SysState *st,
                       double *partials, hipStream_t s);
-// y = a*x + b*y  (real a, b; mixed precisions allowed)
-int axpby(const BatchOp &op, double a, SpinorPtr x, int px, double b, SpinorPtr y, int py, hipStream_t s);
-int spinor_convert(const BatchOp &op, SpinorPtr dst, int pdst, SpinorPtr src, int psrc, hipStream_t s);
+// dst = src (FP64) in precision pdst
+int spinor_convert(const BatchOp &op, SpinorPtr dst, int pdst, SpinorPtr src, hipStream_t s);
 int zero_spinor(const BatchOp &op, SpinorPtr x, int px, hipStream_t s);
 // r = b - r (FP64); store: |r|^2 of system k into st[k].tmp[0]
 int xmy_norm(const BatchOp &op, SpinorPtr b, SpinorPtr r, SysState *st, double *partials, int store, hipStream_t s);

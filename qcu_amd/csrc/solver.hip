@@ -393,7 +393,7 @@ static int schur_solve(Solver &S, int prec, const std::vector<double> &target2, 
     }
     if (restart) {
       // a breakdown restarts the Krylov spaces of the batch from the current residuals
-      QCU_TRY(spinor_convert(op, V->rt.ptr(), prec, S.r64.ptr(), P64, S.stream));
+      QCU_TRY(spinor_convert(op, V->rt.ptr(), prec, S.r64.ptr(), S.stream));
       QCU_TRY(zero_spinor(op, V->p.ptr(), prec, S.stream));
       QCU_TRY(zero_spinor(op, V->v.ptr(), prec, S.stream));
       for (int k = 0; k < nsys; ++k) {

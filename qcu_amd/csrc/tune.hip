@@ -118,8 +118,8 @@ int bench_hop(const BatchOp &op, hipStream_t s, int prec, int clover, int xpay, 
   QCU_TRY(c.create(prec, n));
   QCU_TRY(g64.create(P64, n));
   QCU_TRY(gen_gauss(g64.data.p, (long)n * 12, 77, s));
-  QCU_TRY(spinor_convert(op, a.ptr(), prec, g64.ptr(), P64, s));
-  QCU_TRY(spinor_convert(op, c.ptr(), prec, g64.ptr(), P64, s));
+  QCU_TRY(spinor_convert(op, a.ptr(), prec, g64.ptr(), s));
+  QCU_TRY(spinor_convert(op, c.ptr(), prec, g64.ptr(), s));
   SpinorPtr none{};
   auto launch = [&](int k) {
     return hop(op, prec, (k & 1) ? a.ptr() : b.ptr(), (k & 1) ? b.ptr() : a.ptr(), k & 1, xpay ? EPI_XPAY : EPI_PLAIN,
