@@ -17,7 +17,8 @@
  *   - the converted links and the clover term stay resident while the same
  *     gauge pointer holds the same contents (a 64-bit hash of the field,
  *     computed on the device at every call, decides; the reference rebuilds
- *     them at every call).
+ *     them at every call).  Where changed contents cannot be loaded (a singular
+ *     clover block) the output is left as it was.
  * Errors never abort the process and never throw: the void entry points record
  * the failure, readable with qcuGetLastError()/qcuGetLastErrorString().
  *
@@ -178,6 +179,7 @@ int qcuBatchTune(QcuBatchHandle h, int prec, double *best_ms);
  * tuning a rule on the size and precision picks the shape, and small lattices run
  * a kernel of their own; qcuTune keeps that choice where it is the fastest */
 int qcuTune(QcuLatticeHandle h, int prec, double *best_ms);
+/* the shape in use, tuned, pinned or the rule's (QCU_ERR_ARG for an unknown precision) */
 int qcuTuneGet(QcuLatticeHandle h, int prec, int *block, int *remap, int *group);
 /* pins the launch shape of the hop kernel for this lattice (or batch) and
  * precision instead of tuning it: block 64, 128 or 256 threads; remap 0/1

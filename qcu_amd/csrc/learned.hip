@@ -932,8 +932,8 @@ __global__ void __launch_bounds__(256) k_net_wgrad_mfma(NetWgradArgs a, float *p
     // sites rotated by b mod 8: a matrix-core operand is read at one site from 16
     // planes (4 channels x 4 spins) at once, which would all lie in the same banks,
     // and with the rotation 8 lanes fall on 7 or 8 of the 8 bank groups (16^3x32,
-    // 8 -> 8 channels: 269 -> 238 us, and 219 us with the three complex
-    // numbers of a spin read as such instead of selected from two float4).
+    // 8 -> 8 channels, 256 blocks per term: 269 -> 238 us, and 219 us with the three
+    // complex numbers of a spin read as such instead of selected from two float4).
     const int fs = ((tid & 31) + (tid >> 5)) & 31;
     // the thread's six planes (separate variables: arrays of them end up in
     // scratch memory in some instances)
@@ -1609,8 +1609,8 @@ int Net::layer(SpinorPtr in, SpinorPtr out, const float2 *Wl, int cin, int cout,
     b.npar = nparity;
     b.ns = split_ns;
     // z slabs per XCD where the lattice splits into them, for one parity and for
-    // both (both, one 8 -> 8 layer: 16^3x32 138 -> 135 us, 24^3x48 769 -> 712,
-    // 32^3x64 2141 -> 2138 against chunks interleaved over the grid)
+    // both (both, one 8 -> 8 layer against chunks interleaved over the grid: 16^3x32
+    // 138 -> 135 us, 24^3x48 769 -> 712, 32^3x64 no gain, 2141 and 2123 to 2146)
     b.order = split_order >= 0 ? split_order : 2;
     b.st = st;
     b.A2 = (const uint4 *)io->A2;
@@ -1744,7 +1744,7 @@ int Net::pack_split(int dir, hipStream_t s) {
 
 // Packs what only a pass that keeps no activations uses (the preconditioner's).  A
 // training step, whose weights are new each time, does not pay for it (a step of 4
-// sources: 8^3x16 1.88 -> 1.77 ms, 16^3x32 6.43 -> 5.87 ms).
+// sources takes 0.1 ms less at 8^3x16, where it is 1.8 ms, and 0.6 of 6.4 at 16^3x32).
 int Net::pack_apply(hipStream_t s) {
   if (second_split())
     QCU_TRY(net_pack_second((const float2 *)W.p + woff[0], (const float2 *)W.p + woff[1], p2pk.p, p2winv(), s));
