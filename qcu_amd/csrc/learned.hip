@@ -87,15 +87,23 @@ struct NetLayerArgs {
 };
 
 // the colour matrix of term tg at this site (FP32 links)
-// NT: non-temporal loads (links the kernel reads once)
+// NT: non-temporal loads (links the kernel reads once).  Through a pointer to float4:
+// with ld_at() the compiler keeps fewer loads of the next terms in flight (k_net_gather
+// 113 instead of 119 registers, 90.5 instead of 84.9 us at 24^3x48).
 template <bool NT = false>
 QCU_D void term_link_matrix(const LinkPtr &U, const TermGeo &tg, cf (&m)[9]) {
+  typedef float f4 __attribute__((ext_vector_type(4)));
   float4 raw[3];
   if (tg.hop) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const size_t cb = ((size_t)tg.slab * 3 + k) * U.vh * 16;
-      raw[k] = NT ? ld_at<float4, true>(U.a, cb, (unsigned)tg.li * 16u) : ld_at<float4>(U.a, cb, (unsigned)tg.li * 16u);
+      const char *src = (const char *)U.a + ((size_t)tg.slab * 3 + k) * U.vh * 16 + (unsigned)tg.li * 16u;
+      if (NT) {
+        const f4 w = __builtin_nontemporal_load((const f4 *)src);
+        raw[k] = make_float4(w.x, w.y, w.z, w.w);
+      } else {
+        raw[k] = *(const float4 *)src;
+      }
     }
   }
   term_matrix(raw, tg.hop, tg.fwd, tg.ph, m);
