@@ -259,7 +259,9 @@ int net_layer_second(const NetSecondArgs &a, int part, hipStream_t s);
 // of 4 one at a time), up to 1024, beyond which each block takes several.
 // Fewer blocks write and read fewer of the 8 KiB block sums, at the price of longer
 // FP32 sums (16^3x32, 8 -> 8: 256 blocks of 16 steps 226 us and 6 us for the FP64 sums,
-// 1024 blocks of 4 steps 238 and 16 us); no size takes longer ones than 1024 blocks give.
+// 1024 blocks of 4 steps 238 and 16 us).  But their length is most of the gradient's
+// error: 16^4, 1-8-8-8-1, 128 blocks of 16 steps 7.2e-7 off 64 bits, 1024 blocks of 2
+// 5.0e-7 (1-4-1: 5.4e-7 and 2.7e-7).  No size takes longer sums than 1024 blocks give.
 constexpr int kWgBlocks = 1024;
 inline int wgrad_blocks(int vh, bool lds) {
   const long long per = lds ? 32 : 16, steps = (2LL * vh + per - 1) / per;
